@@ -28,6 +28,7 @@ SOURCES = [
     "elementwise.hip",
     "fold.hip",
     "stencil2d.hip",
+    "gol.hip",
     "stencil3d.hip",
     "batch.hip",
     "serve.hip",

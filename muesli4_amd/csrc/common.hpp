@@ -5,6 +5,7 @@
 
 #include <cstddef>
 #include <cstdint>
+#include <functional>
 #include <string>
 
 #include "msl_hip.h"
@@ -55,6 +56,12 @@ int noalloc_setup(int device);
 // first call is cached per name, dflt included: callers whose default
 // varies pass a fixed sentinel (0) and apply their default themselves.
 int tune_int(const char *name, int dflt);
+
+// Iteration loops captured once into a HIP graph and replayed: runs the
+// graph cached under `key`, capturing body()'s launches first when there is
+// none (runtime.hip).
+std::string graph_key(const char *kind, const void *a, const void *b, long p0, long p1, long p2, long p3, long p4);
+int run_cached_graph(const std::string &key, const std::function<int()> &body);
 
 // Number of workgroups that fills the device for a streaming kernel.
 inline int streaming_blocks(size_t work_items, int threads, int per_cu) {

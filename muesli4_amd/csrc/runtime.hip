@@ -7,6 +7,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <functional>
 #include <map>
 #include <mutex>
 #include <vector>
@@ -91,6 +92,51 @@ int workspace(size_t bytes, void **ptr) {
     g_ws_bytes = want;
     *ptr = g_ws;
     return MSL_OK;
+}
+
+// ---- graph cache for iteration loops ---------------------------------------
+struct GraphCache {
+    std::mutex mu;
+    std::map<std::string, hipGraphExec_t> graphs;
+};
+static GraphCache g_cache;
+
+int run_cached_graph(const std::string &key, const std::function<int()> &body) {
+    hipGraphExec_t exec = nullptr;
+    {
+        std::lock_guard<std::mutex> lock(g_cache.mu);
+        auto it = g_cache.graphs.find(key);
+        if (it != g_cache.graphs.end()) exec = it->second;
+    }
+    if (!exec) {
+        int rc = msl_graph_begin();
+        if (rc) return rc;
+        int brc = body();
+        void *g = nullptr;
+        int erc = msl_graph_end(&g);
+        if (brc) {
+            if (g) msl_graph_destroy(g);
+            return brc;
+        }
+        if (erc) return erc;
+        exec = (hipGraphExec_t)g;
+        std::lock_guard<std::mutex> lock(g_cache.mu);
+        if (g_cache.graphs.size() > 64) {
+            // a cached graph may still be running: drain the stream first
+            MSL_HIP_TRY(hipStreamSynchronize(ctx().stream));
+            for (auto &kv : g_cache.graphs) (void)hipGraphExecDestroy(kv.second);
+            g_cache.graphs.clear();
+        }
+        g_cache.graphs[key] = exec;
+    }
+    MSL_HIP_TRY(hipGraphLaunch(exec, ctx().stream));
+    return MSL_OK;
+}
+
+std::string graph_key(const char *kind, const void *a, const void *b, long p0, long p1, long p2, long p3, long p4) {
+    char buf[256];
+    snprintf(buf, sizeof buf, "%s|%p|%p|%ld|%ld|%ld|%ld|%ld", kind, a, b, p0, p1, p2, p3, p4);
+    return std::string(buf);
 }
 
 }  // namespace mslhip

@@ -255,16 +255,6 @@ int gol_step(int32_t *out, const int32_t *in, int rows, int cols) {
     return launch_strip(out, in, rows, cols, (int32_t)0, pol, 0, "msl_gol_i32");
 }
 
-// ---- Game of Life, several generations per launch ---------------------------
-// A block owns a 64-column x (4 * RPW)-row window of the grid (cells outside
-// the grid read 0): lane l holds column l, wave w rows [w*RPW, (w+1)*RPW)
-// in registers.  Each generation exchanges the waves' first and last rows
-// through LDS, forms vertical 3-sums in registers and the horizontal ones by
-// DPP lane shifts, and applies B3/S23; cells outside the grid stay 0, as in
-// the one-step kernel.  The window edges lack neighbours, so after s
-// generations only cells at least s from every window edge are exact; the
-// block stores the central (64 - 2K) x (4*RPW - 2K) tile, exact after up to
-// K generations.  Integer rule: bit-identical to s single steps.
 // Whole-wave lane shifts with the vacated lane reading 0 (bound_ctrl): no
 // 'old' operand to materialise, so the compiler folds the shift into the
 // add that consumes it (v_add_f32_dpp / v_add_u32_dpp).
@@ -275,66 +265,12 @@ __device__ __forceinline__ int32_t lane_from_right(int32_t v) {  // lane l gets 
     return __builtin_amdgcn_update_dpp(0, v, 0x130, 0xF, 0xF, true);
 }
 
-template <int K, int RPW>
-__global__ __launch_bounds__(256) void gol_multi_kernel(int32_t *__restrict__ out, const int32_t *__restrict__ in,
-                                                        int rows, int cols, int steps, int tiles_x) {
-    constexpr int H = 4 * RPW, TW = 64 - 2 * K, TH = H - 2 * K;
-    __shared__ int32_t edge[4][2][64];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int tx = blockIdx.x % tiles_x, ty = blockIdx.x / tiles_x;
-    const int gx = tx * TW - K + lane;
-    const int gy0 = ty * TH - K + wave * RPW;
-    const bool colok = (unsigned)gx < (unsigned)cols;
-    int32_t c[RPW + 2];  // rows gy0-1 .. gy0+RPW
-#pragma unroll
-    for (int i = 0; i < RPW; i++) {
-        const int gy = gy0 + i;
-        c[i + 1] = (colok && (unsigned)gy < (unsigned)rows) ? in[(size_t)gy * cols + gx] : 0;
-    }
-    for (int s = 0; s < steps; s++) {
-        edge[wave][0][lane] = c[1];
-        edge[wave][1][lane] = c[RPW];
-        __syncthreads();
-        c[0] = wave > 0 ? edge[wave - 1][1][lane] : 0;
-        c[RPW + 1] = wave < 3 ? edge[wave + 1][0][lane] : 0;
-        __syncthreads();
-        int32_t nw[RPW];
-#pragma unroll
-        for (int i = 0; i < RPW; i++) {
-            const int32_t vs = c[i] + c[i + 1] + c[i + 2];
-            const int32_t live = c[i + 1];
-            const int32_t sum = lane_from_left(vs) + vs + lane_from_right(vs) - live;
-            // B3/S23 as in examples/gameoflife.cpp:18-43
-            int32_t next = 0;
-            if (live == 1 && (sum == 2 || sum == 3)) next = 1;
-            if (live == 0 && sum == 3) next = 1;
-            const int gy = gy0 + i;
-            nw[i] = (colok && (unsigned)gy < (unsigned)rows) ? next : 0;
-        }
-#pragma unroll
-        for (int i = 0; i < RPW; i++) c[i + 1] = nw[i];
-    }
-    if (lane >= K && lane < 64 - K && colok) {
-#pragma unroll
-        for (int i = 0; i < RPW; i++) {
-            const int wy = wave * RPW + i, gy = gy0 + i;
-            if (wy >= K && wy < H - K && gy < rows) out[(size_t)gy * cols + gx] = c[i + 1];
-        }
-    }
-}
-
-constexpr int kGolSteps = 4;  // generations per launch
-constexpr int kGolRows = 8;   // rows per wave: 64 x 32 windows, 56 x 24 tiles
-// Grids of at most kGolSmallCells cells are launch-bound: there, 8
-// generations per launch on 64 x 64 windows (48 x 48 tiles) run faster
-// despite the wider overlap (1024^2: 2.16 -> 2.01 us per generation); from
-// 2048^2 on the 4-generation windows are 7-9 % faster.
-constexpr int kGolSmallSteps = 8;
-constexpr int kGolSmallRows = 16;
-constexpr long kGolSmallCells = 1L << 20;
-
-// Mean blur of radius 1, several generations per launch, laid out like the
-// Game of Life kernel above: lane = column, wave = RPW rows, row sums
+// Mean blur of radius 1, several generations per launch.  A block owns a
+// 64-column x (4 * RPW)-row window of the grid: lane l holds column l, wave w
+// rows [w*RPW, (w+1)*RPW) in registers.  The window edges lack neighbours, so
+// after s generations only cells at least s from every window edge are exact;
+// the block stores the central (64 - 2K) x (4*RPW - 2K) tile, exact after up
+// to K generations.  Row sums
 // ((0 + left) + centre) + right with the side cells by DPP, column sums
 // ((0 + above) + row) + below with the wave edge rows through LDS, then the
 // exact division by 9 -- the operation order of the one-step kernel (the
@@ -443,17 +379,6 @@ static int mean3_multi_step(float *out, const float *in, int rows, int cols, flo
     return check_launch("msl_stencil2d_mean_iterate_f32");
 }
 
-template <int K, int RPW>
-static int gol_multi_step(int32_t *out, const int32_t *in, int rows, int cols, int steps) {
-    constexpr int TW = 64 - 2 * K, TH = 4 * RPW - 2 * K;
-    const int tiles_x = (cols + TW - 1) / TW;
-    const long blocks = (long)tiles_x * ((rows + TH - 1) / TH);
-    MSL_REQUIRE(blocks <= INT32_MAX, "msl_gol_iterate_i32: grid too large");
-    MSL_REQUIRE(steps >= 1 && steps <= K, "msl_gol_iterate_i32: generations per launch out of range");
-    gol_multi_kernel<K, RPW><<<(int)blocks, 256, 0, ctx().stream>>>(out, in, rows, cols, steps, tiles_x);
-    return check_launch("msl_gol_iterate_i32");
-}
-
 // Generations per launch of msl_stencil2d_mean_iterate_f32, in launch order
 // (1 = the one-step kernel; otherwise the six-generation register-window
 // kernel at r = 1 or the two-generation march at r = 2 .. kMaxMean2R on rows
@@ -510,52 +435,6 @@ __global__ __launch_bounds__(256) void div_check_kernel(float d, float rcp, unsi
         __syncthreads();
     }
     if (threadIdx.x == 0 && part[0]) atomicAdd(count, (unsigned long long)part[0]);
-}
-
-// ---- graph cache for iteration loops ---------------------------------------
-struct GraphCache {
-    std::mutex mu;
-    std::map<std::string, hipGraphExec_t> graphs;
-};
-static GraphCache g_cache;
-
-template <typename Body>
-int run_cached_graph(const std::string &key, Body body) {
-    hipGraphExec_t exec = nullptr;
-    {
-        std::lock_guard<std::mutex> lock(g_cache.mu);
-        auto it = g_cache.graphs.find(key);
-        if (it != g_cache.graphs.end()) exec = it->second;
-    }
-    if (!exec) {
-        int rc = msl_graph_begin();
-        if (rc) return rc;
-        int brc = body();
-        void *g = nullptr;
-        int erc = msl_graph_end(&g);
-        if (brc) {
-            if (g) msl_graph_destroy(g);
-            return brc;
-        }
-        if (erc) return erc;
-        exec = (hipGraphExec_t)g;
-        std::lock_guard<std::mutex> lock(g_cache.mu);
-        if (g_cache.graphs.size() > 64) {
-            // a cached graph may still be running: drain the stream first
-            MSL_HIP_TRY(hipStreamSynchronize(ctx().stream));
-            for (auto &kv : g_cache.graphs) (void)hipGraphExecDestroy(kv.second);
-            g_cache.graphs.clear();
-        }
-        g_cache.graphs[key] = exec;
-    }
-    MSL_HIP_TRY(hipGraphLaunch(exec, ctx().stream));
-    return MSL_OK;
-}
-
-std::string graph_key(const char *kind, const void *a, const void *b, long p0, long p1, long p2, long p3, long p4) {
-    char buf[256];
-    snprintf(buf, sizeof buf, "%s|%p|%p|%ld|%ld|%ld|%ld|%ld", kind, a, b, p0, p1, p2, p3, p4);
-    return std::string(buf);
 }
 
 }  // namespace mslhip
@@ -656,29 +535,5 @@ int msl_selftest_div_six(uint64_t *h_mismatches) {
 }
 
 int msl_gol_i32(int32_t *d_out, const int32_t *d_in, int rows, int cols) { return gol_step(d_out, d_in, rows, cols); }
-
-int msl_gol_iterate_i32(int32_t *d_a, int32_t *d_b, int rows, int cols, int iters, int *h_result_in_b) {
-    int rc = ensure_ready();
-    if (rc) return rc;
-    MSL_REQUIRE(iters >= 0, "msl_gol_iterate_i32: negative iteration count");
-    MSL_REQUIRE(rows >= 0 && cols >= 0, "msl_gol_iterate_i32: negative shape");
-    if (h_result_in_b) *h_result_in_b = iters & 1;
-    if (iters == 0 || rows == 0 || cols == 0) return MSL_OK;
-    MSL_REQUIRE((int64_t)rows * cols <= INT32_MAX, "msl_gol_iterate_i32: grid too large");
-    MSL_REQUIRE(d_a && d_b && d_a != d_b, "msl_gol_iterate_i32: null or aliased buffers");
-    const bool small = (long)rows * cols <= kGolSmallCells;
-    const std::vector<int> plan = generation_plan(iters, small ? kGolSmallSteps : kGolSteps);
-    std::string key = graph_key("gol", d_a, d_b, rows, cols, iters, 0, 0);
-    return run_cached_graph(key, [&]() {
-        for (size_t k = 0; k < plan.size(); k++) {
-            int32_t *src = (k & 1) ? d_b : d_a;
-            int32_t *dst = (k & 1) ? d_a : d_b;
-            int brc = small ? gol_multi_step<kGolSmallSteps, kGolSmallRows>(dst, src, rows, cols, plan[k])
-                            : gol_multi_step<kGolSteps, kGolRows>(dst, src, rows, cols, plan[k]);
-            if (brc) return brc;
-        }
-        return MSL_OK;
-    });
-}
 
 }  // extern "C"
