@@ -6,7 +6,8 @@
 // two launches and no host copy: the array is streamed once with 16-byte
 // loads (each lane accumulates, then a wave64 shuffle tree and a 4-wave LDS
 // combine produce one partial per block) and one block combines the partials
-// in a fixed order.  Results stay in device memory.
+// in a fixed order; short arrays do both in one block.  The result goes to
+// device memory, or straight to the pinned host slot for the _host forms.
 //
 // Compensated sum: every lane keeps (s, c) and adds each element with Knuth's
 // TwoSum (s' = s + x exactly split into s' and the rounding error, which is
@@ -98,16 +99,14 @@ __device__ __forceinline__ typename P::Part block_reduce(typename P::Part v) {
     return r;  // identical in every thread
 }
 
-// Stage 1: every block streams its grid-stride share with four 16-byte loads
-// in flight per lane and reduces it to one partial.  The order of every
-// combination is fixed, so results are deterministic for a given grid size.
-template <typename P, bool kF64Final>
-__global__ __launch_bounds__(kFoldThreads) void fold_kernel(const typename P::In *__restrict__ in, size_t n,
-                                                            typename P::Part *__restrict__ partials, int vec_ok) {
+// One thread's share of an array folded by threads `stride` apart (first
+// index i): 16-byte loads, U of them in flight, then the scalar rest.
+template <typename P>
+__device__ __forceinline__ typename P::Part fold_share(const typename P::In *__restrict__ in, size_t n, size_t i,
+                                                       size_t stride, int vec_ok) {
     using V = typename P::V;
     typename P::Part acc = P::init();
-    const size_t stride = (size_t)gridDim.x * kFoldThreads;
-    size_t i = (size_t)blockIdx.x * kFoldThreads + threadIdx.x;
+    const size_t first = i;
     if (vec_ok) {
         const size_t n4 = n / 4;
         const V *in4 = reinterpret_cast<const V *>(in);
@@ -131,11 +130,21 @@ __global__ __launch_bounds__(kFoldThreads) void fold_kernel(const typename P::In
             V v = in4[i];
             P::push(acc, v.x); P::push(acc, v.y); P::push(acc, v.z); P::push(acc, v.w);
         }
-        i = n4 * 4 + (size_t)blockIdx.x * kFoldThreads + threadIdx.x;
+        i = n4 * 4 + first;
     }
     for (; i < n; i += stride) P::push(acc, in[i]);
-    const typename P::Part r = block_reduce<P>(acc);
+    return acc;
+}
 
+// Stage 1: every block streams its grid-stride share and reduces it to one
+// partial.  The order of every combination is fixed, so results are
+// deterministic for a given grid size.
+template <typename P>
+__global__ __launch_bounds__(kFoldThreads) void fold_kernel(const typename P::In *__restrict__ in, size_t n,
+                                                            typename P::Part *__restrict__ partials, int vec_ok) {
+    const typename P::Part acc = fold_share<P>(in, n, (size_t)blockIdx.x * kFoldThreads + threadIdx.x,
+                                               (size_t)gridDim.x * kFoldThreads, vec_ok);
+    const typename P::Part r = block_reduce<P>(acc);
     if (threadIdx.x == 0) partials[blockIdx.x] = r;
 }
 
@@ -173,6 +182,51 @@ __global__ __launch_bounds__(kFoldThreads) void fold_final_kernel(const typename
     }
 }
 
+// Both stages in one launch for arrays of at most kSmallParts partials: one
+// block of four groups of 256 threads takes the shares of the nparts blocks
+// that fold_kernel would have had, group g those of blocks g, g + 4, ..., and
+// combines them in the order of fold_kernel and fold_final_kernel, so the
+// result is bit-identical to theirs.  Bound by launch and load latency: the
+// whole call (result on the host) takes 13.9 us at 10007 floats and 15.9 at
+// 40960, two launches 16.3 at any size up to 2^20 (the compensated sum; the
+// line lies where it meets them, the integer sum and max would gain to 16
+// partials).  With a third launch that copied the scalar it was 18.1.
+constexpr int kSmallParts = 10;
+constexpr int kSmallThreads = 4 * kFoldThreads;
+
+template <typename P, bool kF64Final>
+__global__ __launch_bounds__(kSmallThreads) void fold_small_kernel(const typename P::In *__restrict__ in, size_t n,
+                                                                   int nparts, void *__restrict__ result,
+                                                                   int vec_ok) {
+    using Part = typename P::Part;
+    __shared__ Part lds[kSmallParts][kFoldWaves];
+    const int t = threadIdx.x & (kFoldThreads - 1), group = threadIdx.x / kFoldThreads;
+    for (int vb = group; vb < nparts; vb += 4) {
+        const Part r = wave_reduce<P>(
+            fold_share<P>(in, n, (size_t)vb * kFoldThreads + t, (size_t)nparts * kFoldThreads, vec_ok));
+        if ((t & 63) == 0) lds[vb][t >> 6] = r;
+    }
+    __syncthreads();
+    if (threadIdx.x >= 64) return;
+    Part p = P::init();
+    if ((int)threadIdx.x < nparts) {
+        p = lds[threadIdx.x][0];
+#pragma unroll
+        for (int w = 1; w < kFoldWaves; w++) p = P::combine(p, lds[threadIdx.x][w]);
+    }
+    if constexpr (kF64Final) {
+        double d = 0.0;
+        d += (double)p.s;
+        d += (double)p.c;
+#pragma unroll
+        for (int m = 32; m >= 1; m >>= 1) d += __shfl_xor(d, m);
+        if (threadIdx.x == 0) *reinterpret_cast<double *>(result) = d;
+    } else {
+        p = wave_reduce<P>(P::combine(P::init(), p));
+        if (threadIdx.x == 0) *reinterpret_cast<Part *>(result) = p;
+    }
+}
+
 // Two blocks per CU: the read-only stream needs more loads in flight than
 // one block's four 16-byte loads per lane (8192^2 floats with the input
 // evicted from the Infinity Cache: 4.7 TB/s with one block per CU, 5.7 with
@@ -185,9 +239,22 @@ inline int fold_blocks(size_t n) {
     return (int)want;
 }
 
-// Workspace layout: [0, 256) result scalars, partials from byte 512.
-constexpr size_t kResultBytes = 256;
-constexpr size_t kPartialsOffset = 512;
+// Enqueues a fold of n elements into *result; `partials` (one per block of
+// fold_blocks(n)) is only used when the array takes two launches.
+template <typename P, bool kF64Final>
+int launch_fold(const typename P::In *in, size_t n, int blocks, typename P::Part *partials, void *result,
+                const char *name) {
+    const int vec_ok = (((uintptr_t)in) & 15u) == 0;
+    if (blocks <= kSmallParts) {
+        fold_small_kernel<P, kF64Final><<<1, kSmallThreads, 0, ctx().stream>>>(in, n, blocks, result, vec_ok);
+        return check_launch(name);
+    }
+    fold_kernel<P><<<blocks, kFoldThreads, 0, ctx().stream>>>(in, n, partials, vec_ok);
+    int rc = check_launch(name);
+    if (rc) return rc;
+    fold_final_kernel<P, kF64Final><<<1, kFoldThreads, 0, ctx().stream>>>(partials, blocks, result);
+    return check_launch(name);
+}
 
 template <typename P, bool kF64Final>
 int run_fold(const typename P::In *in, size_t n, void *d_result, const char *name) {
@@ -196,19 +263,26 @@ int run_fold(const typename P::In *in, size_t n, void *d_result, const char *nam
     MSL_REQUIRE(in != nullptr || n == 0, std::string(name) + ": null input");
     const int blocks = fold_blocks(n);
     void *ws = nullptr;
-    rc = workspace(kPartialsOffset + (size_t)blocks * sizeof(typename P::Part), &ws);
-    if (rc) return rc;
-    auto *partials = reinterpret_cast<typename P::Part *>((char *)ws + kPartialsOffset);
-    if (!d_result) d_result = ws;
-    const int vec_ok = (((uintptr_t)in) & 15u) == 0;
-    fold_kernel<P, kF64Final><<<blocks, kFoldThreads, 0, ctx().stream>>>(in, n, partials, vec_ok);
-    rc = check_launch(name);
-    if (rc) return rc;
-    fold_final_kernel<P, kF64Final><<<1, kFoldThreads, 0, ctx().stream>>>(partials, blocks, d_result);
-    return check_launch(name);
+    if (blocks > kSmallParts) {
+        rc = workspace((size_t)blocks * sizeof(typename P::Part), &ws);
+        if (rc) return rc;
+    }
+    return launch_fold<P, kF64Final>(in, n, blocks, static_cast<typename P::Part *>(ws), d_result, name);
 }
 
-int scratch_result(void **p) { return workspace(kResultBytes, p); }
+// Folds into the pinned result slot and waits: the last kernel stores the
+// scalar to host memory itself, with no copy launch behind it.
+template <typename P, bool kF64Final, typename R>
+int run_fold_host(const typename P::In *in, size_t n, R *h_result, const char *name) {
+    void *slot = nullptr;
+    int rc = msl_result_slot(&slot, nullptr);
+    if (rc) return rc;
+    rc = run_fold<P, kF64Final>(in, n, slot, name);
+    if (rc) return rc;
+    MSL_HIP_TRY(hipStreamSynchronize(ctx().stream));
+    *h_result = *static_cast<const R *>(slot);
+    return MSL_OK;
+}
 
 // ---- allocation-free compensated fold ---------------------------------------
 // msl_fold_sum_f32_noalloc keeps its block partials in this file-scope device
@@ -259,22 +333,12 @@ int msl_fold_sum_f32_noalloc(const float *d_in, size_t n, double *d_result) {
                                        "(lower MSL_FOLD_BLOCKS_PER_CU)");
     Pair *partials = reinterpret_cast<Pair *>(g_scratch_ptr[ctx().device]);
     MSL_REQUIRE(partials != nullptr, "msl_fold_sum_f32_noalloc: scratch not set up on this device");
-    const int vec_ok = (((uintptr_t)d_in) & 15u) == 0;
-    fold_kernel<CompSumPolicy, true><<<blocks, kFoldThreads, 0, ctx().stream>>>(d_in, n, partials, vec_ok);
-    rc = check_launch("msl_fold_sum_f32_noalloc");
-    if (rc) return rc;
-    fold_final_kernel<CompSumPolicy, true><<<1, kFoldThreads, 0, ctx().stream>>>(partials, blocks, d_result);
-    return check_launch("msl_fold_sum_f32_noalloc");
+    return launch_fold<CompSumPolicy, true>(d_in, n, blocks, partials, d_result, "msl_fold_sum_f32_noalloc");
 }
 
 int msl_fold_sum_f32_host(const float *d_in, size_t n, double *h_sum64, float *h_sum32) {
-    int rc = run_fold<CompSumPolicy, true>(d_in, n, nullptr, "msl_fold_sum_f32_host");
-    if (rc) return rc;
-    void *ws = nullptr;
-    rc = scratch_result(&ws);
-    if (rc) return rc;
     double r = 0.0;
-    rc = msl_memcpy_d2h(&r, ws, sizeof(double));
+    int rc = run_fold_host<CompSumPolicy, true>(d_in, n, &r, "msl_fold_sum_f32_host");
     if (rc) return rc;
     if (h_sum64) *h_sum64 = r;
     if (h_sum32) *h_sum32 = (float)r;
@@ -283,37 +347,18 @@ int msl_fold_sum_f32_host(const float *d_in, size_t n, double *h_sum64, float *h
 
 int msl_fold_sum_u32_host(const uint32_t *d_in, size_t n, uint32_t *h_sum) {
     MSL_REQUIRE(h_sum != nullptr, "msl_fold_sum_u32_host: null result pointer");
-    int rc = run_fold<SumU32Policy, false>(d_in, n, nullptr, "msl_fold_sum_u32_host");
-    if (rc) return rc;
-    void *ws = nullptr;
-    rc = scratch_result(&ws);
-    if (rc) return rc;
-    return msl_memcpy_d2h(h_sum, ws, sizeof(uint32_t));
+    return run_fold_host<SumU32Policy, false>(d_in, n, h_sum, "msl_fold_sum_u32_host");
 }
 
 int msl_fold_sum_i32_host(const int32_t *d_in, size_t n, int64_t *h_sum) {
     MSL_REQUIRE(h_sum != nullptr, "msl_fold_sum_i32_host: null result pointer");
-    int rc = run_fold<SumI32Policy, false>(d_in, n, nullptr, "msl_fold_sum_i32_host");
-    if (rc) return rc;
-    void *ws = nullptr;
-    rc = scratch_result(&ws);
-    if (rc) return rc;
-    long long r = 0;
-    rc = msl_memcpy_d2h(&r, ws, sizeof(long long));
-    if (rc) return rc;
-    *h_sum = (int64_t)r;
-    return MSL_OK;
+    return run_fold_host<SumI32Policy, false>(d_in, n, h_sum, "msl_fold_sum_i32_host");
 }
 
 int msl_fold_max_f32_host(const float *d_in, size_t n, float *h_max) {
     MSL_REQUIRE(h_max != nullptr, "msl_fold_max_f32_host: null result pointer");
     MSL_REQUIRE(n > 0, "msl_fold_max_f32_host: empty input");
-    int rc = run_fold<MaxF32Policy, false>(d_in, n, nullptr, "msl_fold_max_f32_host");
-    if (rc) return rc;
-    void *ws = nullptr;
-    rc = scratch_result(&ws);
-    if (rc) return rc;
-    return msl_memcpy_d2h(h_max, ws, sizeof(float));
+    return run_fold_host<MaxF32Policy, false>(d_in, n, h_max, "msl_fold_max_f32_host");
 }
 
 }  // extern "C"
