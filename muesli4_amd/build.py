@@ -29,6 +29,7 @@ SOURCES = [
     "fold.hip",
     "stencil2d.hip",
     "gol.hip",
+    "blur_tile.hip",
     "stencil3d.hip",
     "batch.hip",
     "serve.hip",

@@ -16,6 +16,7 @@
 #include <string>
 #include <vector>
 
+#include "blur_tile.hpp"
 #include "strip.hpp"
 
 namespace mslhip {
@@ -102,6 +103,14 @@ inline int row_mode(const T *in, const T *out, int cols) {
     return kScalar;
 }
 
+// Single steps of radius kTile1MinR and above on grids of at most
+// kTile1MaxCells run the tile kernel (blur_tile.hip): us per step, strip
+// march / tile: 500 x 517 r = 4 5.7 / 4.8, 5 6.5 / 5.0, 10 11.1 / 5.3;
+// 1024^2 r = 4 5.9 / 6.4, 5 6.8 / 6.3, 10 11.7 / 7.1; 2048^2 r = 4 9.3 / 10.7,
+// 6 12.9 / 11.2, 10 17.7 / 13.2; 3000^2 r = 6 17.6 / 19.3, 10 22.1 / 24.4.
+constexpr int kTile1MinR = 5;
+constexpr long kTile1MaxCells = 9L << 19;  // 4.7 million
+
 struct StripShape {
     int seg, strips_x, segs, nitems, c;
 };
@@ -119,8 +128,7 @@ inline StripShape strip_shape(int rows, int cols, int r, int seg, bool streamed)
     StripShape s;
     const long cus = ctx().num_cus;
     const long strips4 = (cols + kStripW - 1) / kStripW;
-    s.c = tune_int("MSL_STRIP_C", 0);
-    if (s.c != 1 && s.c != 4) s.c = strips4 * ((rows + 7) / 8) < 8 * cus ? 1 : 4;
+    s.c = r < kTile1MinR && strips4 * ((rows + 7) / 8) < 8 * cus ? 1 : 4;
     const int sw = 64 * s.c;
     s.strips_x = (cols + sw - 1) / sw;
     if (seg <= 0) seg = tune_int("MSL_STRIP_SEG", 0);
@@ -150,13 +158,14 @@ int launch_strip(typename Pol::T *out, const typename Pol::T *in, int rows, int 
     StripShape s = strip_shape(rows, cols, Pol::R, seg, nt);
     const int blocks = (s.nitems + 3) / 4;
     const int mode = row_mode(in, out, cols);
-    if (s.c == 1 && nt)
-        strip_stencil_kernel<Pol, kAligned, true, 1><<<blocks, 256, 0, ctx().stream>>>(out, in, rows, cols, nv, s.seg,
-                                                                                         s.strips_x, s.nitems, pol);
-    else if (s.c == 1)
-        strip_stencil_kernel<Pol, kAligned, false, 1><<<blocks, 256, 0, ctx().stream>>>(out, in, rows, cols, nv, s.seg,
-                                                                                          s.strips_x, s.nitems, pol);
-    else if (mode == kAligned && nt)
+    if constexpr (Pol::R < kTile1MinR) {
+        if (s.c == 1) {
+            strip_stencil_kernel<Pol, kAligned, false, 1><<<blocks, 256, 0, ctx().stream>>>(
+                out, in, rows, cols, nv, s.seg, s.strips_x, s.nitems, pol);
+            return check_launch(name);
+        }
+    }
+    if (mode == kAligned && nt)
         strip_stencil_kernel<Pol, kAligned, true><<<blocks, 256, 0, ctx().stream>>>(out, in, rows, cols, nv, s.seg,
                                                                                       s.strips_x, s.nitems, pol);
     else if (mode == kAligned)
@@ -240,6 +249,12 @@ int mean_step(float *out, const float *in, int rows, int cols, int r, float nv, 
     MSL_REQUIRE((int64_t)rows * cols <= INT32_MAX && cols < (1 << 30), "msl_stencil2d_mean_f32: grid too large");
     if (rows == 0 || cols == 0) return MSL_OK;
     MSL_REQUIRE(out && in && out != in, "msl_stencil2d_mean_f32: null or aliased buffers");
+    if (r >= kTile1MinR && (long)rows * cols <= kTile1MaxCells && seg <= 0) {
+        // 64-row tiles once they give two workgroups per CU, else 32-row ones
+        const int tile_w = (64 - 2 * r) / 4 * 4;
+        const long tiles = (long)((cols + tile_w - 1) / tile_w) * ((rows + 63) / 64);
+        return blur_tile_step(out, in, rows, cols, r, nv, 1, TileShape{64, 2, tiles < 2L * ctx().num_cus ? 32 : 64, 0.0});
+    }
     return kMeanLaunchers[r](out, in, rows, cols, nv, seg);
 }
 
@@ -379,24 +394,70 @@ static int mean3_multi_step(float *out, const float *in, int rows, int cols, flo
     return check_launch("msl_stencil2d_mean_iterate_f32");
 }
 
-// Generations per launch of msl_stencil2d_mean_iterate_f32, in launch order
-// (1 = the one-step kernel; otherwise the six-generation register-window
-// kernel at r = 1 or the two-generation march at r = 2 .. kMaxMean2R on rows
-// of 4 or more cells).  MSL_MEAN_GENS = 1 or 2 forces one or two generations
-// per launch for r >= 2 (read on every call, so a process can compare both).
-static std::vector<int> mean_iterate_plan(const float *d_a, const float *d_b, int rows, int cols, int r, int iters) {
-    if (r == 1) return generation_plan(iters, kMean3Steps);
-    const char *ge = getenv("MSL_MEAN_GENS");
-    const int gens_env = ge ? atoi(ge) : 0;
-    const bool pairs = r <= kMaxMean2R && row_mode(d_a, d_b, cols) != kScalar &&
-                       (gens_env == 2 || (gens_env != 1 && mean2_default(r, rows, cols)));
-    return pairs ? generation_plan(iters, 2) : std::vector<int>(iters, 1);
+// Grids whose iterations run in tiles (several generations per launch in
+// LDS): radius 2 and above up to these many cells, unless the two-generation
+// march takes them (mean2_default).  us per generation of the best tile and
+// of the march: 4096^2 r = 5 20.4 / 26.4, 6 21.6 / 26.0, 8 28.0 / 28.3;
+// 3000^2 r = 8 16.9 / 20.3, 9 20.6 / 22.5, 10 23.8 / 22.2; 2048^2 r = 10
+// 13.0 / 17.7; 500 x 517 r = 3 2.1 / 4.9.
+static bool tile_default(int r, int rows, int cols) {
+    const long cells = (long)rows * cols;
+    return r >= 2 && !mean2_default(r, rows, cols) && cells <= (r <= 8 ? 1L << 24 : 9L << 19);
 }
 
-static std::string plan_signature(const std::vector<int> &plan) {
-    std::string sig = "|";
-    for (int g : plan) sig += (char)('0' + g);
-    return sig;
+enum LaunchKind { kLaunchStep, kLaunchMulti3, kLaunchPair, kLaunchTile };
+
+struct MeanLaunch {
+    int gens;
+    LaunchKind kind;
+    TileShape tile;
+};
+
+// The launches of msl_stencil2d_mean_iterate_f32, in order: the
+// six-generation register-window kernel at r = 1, the two-generation march at
+// r = 2 .. kMaxMean2R on large grids with rows of 4 or more cells, tiles with
+// the number of generations that the model prices lowest on smaller ones,
+// else the one-step kernel.  MSL_MEAN_GENS = 1 or 2 forces one or two
+// generations per launch for r >= 2 (read on every call, so a process can
+// compare both).
+static int mean_gens_env() {
+    const char *ge = getenv("MSL_MEAN_GENS");
+    return ge ? atoi(ge) : 0;
+}
+
+static std::vector<MeanLaunch> mean_iterate_plan(const float *d_a, const float *d_b, int rows, int cols, int r,
+                                                 int iters) {
+    auto launches = [](const std::vector<int> &gens, LaunchKind kind) {
+        std::vector<MeanLaunch> plan;
+        for (int g : gens) plan.push_back(MeanLaunch{g, g == 1 ? kLaunchStep : kind, TileShape{}});
+        return plan;
+    };
+    if (r == 1) return launches(generation_plan(iters, kMean3Steps), kLaunchMulti3);
+    const int gens_env = mean_gens_env();
+    const bool pairs = r <= kMaxMean2R && row_mode(d_a, d_b, cols) != kScalar &&
+                       (gens_env == 2 || (gens_env != 1 && mean2_default(r, rows, cols)));
+    if (pairs) return launches(generation_plan(iters, 2), kLaunchPair);
+    if (gens_env == 0 && iters > 1 && tile_default(r, rows, cols)) {
+        TileShape shape[kMean3Steps + 1];
+        std::vector<int> best;
+        double best_us = 1e30;
+        for (int k = 1; k <= kMean3Steps; k++) {
+            shape[k] = tile_shape(rows, cols, r, k);
+            if (shape[k].w == 0) break;
+            const std::vector<int> gens = generation_plan(iters, k);
+            double us = 0.0;
+            for (int g : gens) us += shape[g].us;
+            if (us < best_us) {
+                best_us = us;
+                best = gens;
+            }
+        }
+        std::vector<MeanLaunch> plan = launches(best, kLaunchTile);
+        for (MeanLaunch &l : plan)
+            if (l.kind == kLaunchTile) l.tile = shape[l.gens];
+        return plan;
+    }
+    return launches(std::vector<int>(iters, 1), kLaunchStep);
 }
 
 // ---- exhaustive check of div_odd_square against IEEE division -------------
@@ -463,16 +524,21 @@ int msl_stencil2d_mean_iterate_f32(float *d_a, float *d_b, int rows, int cols, i
     nvb.f = nv;
     MSL_REQUIRE((int64_t)rows * cols <= INT32_MAX && cols < (1 << 30), "msl_stencil2d_mean_iterate_f32: grid too large");
     MSL_REQUIRE(d_a && d_b && d_a != d_b, "msl_stencil2d_mean_iterate_f32: null or aliased buffers");
-    const std::vector<int> plan = mean_iterate_plan(d_a, d_b, rows, cols, r, iters);
     std::string key = graph_key("mean2d", d_a, d_b, rows, cols, r, nvb.i, iters);
-    key += plan_signature(plan);
+    key += "|" + std::to_string(mean_gens_env());
     return run_cached_graph(key, [&]() {
+        const std::vector<MeanLaunch> plan = mean_iterate_plan(d_a, d_b, rows, cols, r, iters);
         for (size_t k = 0; k < plan.size(); k++) {
+            const MeanLaunch &l = plan[k];
             float *src = (k & 1) ? d_b : d_a;
             float *dst = (k & 1) ? d_a : d_b;
-            int brc = plan[k] == 1   ? mean_step(dst, src, rows, cols, r, nv, 0)
-                      : r == 1       ? mean3_multi_step(dst, src, rows, cols, nv, plan[k])
-                                     : kMean2Launchers[r](dst, src, rows, cols, nv, 0);
+            int brc = MSL_OK;
+            switch (l.kind) {
+                case kLaunchStep: brc = mean_step(dst, src, rows, cols, r, nv, 0); break;
+                case kLaunchMulti3: brc = mean3_multi_step(dst, src, rows, cols, nv, l.gens); break;
+                case kLaunchPair: brc = kMean2Launchers[r](dst, src, rows, cols, nv, 0); break;
+                case kLaunchTile: brc = blur_tile_step(dst, src, rows, cols, r, nv, l.gens, l.tile); break;
+            }
             if (brc) return brc;
         }
         return MSL_OK;
@@ -484,11 +550,13 @@ int msl_stencil2d_mean_iterate_plan(const float *d_a, const float *d_b, int rows
     MSL_REQUIRE(iters >= 0 && rows >= 0 && cols >= 0, "msl_stencil2d_mean_iterate_plan: negative argument");
     MSL_REQUIRE(r >= 1 && r <= kMaxMeanR, "msl_stencil2d_mean_iterate_plan: radius must be in [1, 16]");
     MSL_REQUIRE(h_launches != nullptr && capacity >= 0, "msl_stencil2d_mean_iterate_plan: bad output arguments");
-    std::vector<int> plan;
+    int rc = ensure_ready();  // the tile model counts the device's CUs
+    if (rc) return rc;
+    std::vector<MeanLaunch> plan;
     if (iters > 0 && rows > 0 && cols > 0) plan = mean_iterate_plan(d_a, d_b, rows, cols, r, iters);
     *h_launches = (int)plan.size();
     MSL_REQUIRE(h_gens != nullptr || plan.empty() || capacity == 0, "msl_stencil2d_mean_iterate_plan: null output");
-    for (size_t k = 0; k < plan.size() && (int)k < capacity; k++) h_gens[k] = plan[k];
+    for (size_t k = 0; k < plan.size() && (int)k < capacity; k++) h_gens[k] = plan[k].gens;
     return MSL_OK;
 }
 
