@@ -144,7 +144,8 @@ __device__ __forceinline__ void heat7_march(float *__restrict__ out, const float
 // Generation-1 cells outside the cube are nv, as the second step reads them.
 // Every cell is computed in the one-step order, so the result is
 // bit-identical to two single steps.  kResidual: max |generation 2 -
-// generation 1| into *dmax.
+// generation 1| into *dmax.  kSingle: generation 1 only, of the same tile
+// (the odd step of a job whose items are laid out for two).
 constexpr int kT2X = kTX - 4;  // output columns of a two-generation wave tile
 // Output rows of a two-generation wave tile: 5 rows (90 VGPRs, five waves
 // per SIMD) beat 8 (124, four) although the y halo grows from 4/8 to 4/5
@@ -152,7 +153,7 @@ constexpr int kT2X = kTX - 4;  // output columns of a two-generation wave tile
 // 320^3: 8 rows 7.13 ms, 5 6.90).
 constexpr int kT2Y = 5;
 
-template <bool kResidual, bool NT = true>
+template <bool kResidual, bool NT = true, bool kSingle = false>
 __device__ __forceinline__ void heat7x2_march(float *__restrict__ out, const float *__restrict__ in, int nx, int ny,
                                               int nz, float nv, int x0, int y0, int z0, int z1, float *dmax) {
     constexpr int NI = kT2Y + 4;  // input rows y0-2 .. y0+kT2Y+1
@@ -232,7 +233,8 @@ __device__ __forceinline__ void heat7x2_march(float *__restrict__ out, const flo
             char *op = reinterpret_cast<char *>(out + (size_t)min(max(zo, 0), nz - 1) * plane);
 #pragma unroll
             for (int j = 0; j < kT2Y; j++) {
-                const float v = cell(g1[j], g1[j + 1], g1[j + 2], g1[j + 1], g1[j + 1], tb, tc, ta);
+                const float v =
+                    kSingle ? g1[j + 1][tc] : cell(g1[j], g1[j + 1], g1[j + 2], g1[j + 1], g1[j + 1], tb, tc, ta);
                 // output row y0+j is input row j+2: stored when in the cube
                 if (zo >= z0 && zo < z1 && lane >= 2 && lane <= 61 && ((iok >> (j + 2)) & 1u)) {
                     float *o = reinterpret_cast<float *>(op + ioff[j + 2]);

@@ -14,14 +14,14 @@
 //     in the engine's arena, a single device allocation carved by a
 //     first-fit allocator with coalescing (no per-job hipMalloc, no
 //     fragmentation growth beyond the free list);
-//   * every round advances each active stencil job by one step: one
-//     persistent launch covers all active blur jobs' (strip, segment) items,
-//     one covers all heat jobs' (tile, z-segment) items, one covers the
-//     chunks of the map+fold jobs admitted this round; a job's state stays
-//     resident in the arena across rounds.  When the active jobs' items
-//     cannot fill the GPU (light load), a round advances each job by up to
-//     kMaxSub steps instead, one launch per step, so that the per-round
-//     host work and launches are spread over several steps;
+//   * every round advances each active stencil job by several steps in one
+//     or more launches: one persistent launch covers all active blur jobs'
+//     tiles and advances each by the generations its radius allows in LDS
+//     (blur_tile.hpp), one covers all heat jobs' (tile, z-segment) items, two
+//     generations each, one covers the chunks of the map+fold jobs admitted
+//     this round; a job's state stays resident in the arena across rounds.
+//     The number of launches (at most kMaxSub) aims at kRoundUs of work, so
+//     that the per-round host work and small launches stay a modest share;
 //   * after a job's last step its final state is folded (compensated FP32
 //     pairs per fixed 64K-element chunk, combined in FP64 in chunk order;
 //     wrapping u32 for map+fold) and the round's results are copied to
@@ -34,8 +34,8 @@
 // Every stencil cell is computed in the operation order of the single-grid
 // kernels whatever the tiling, and the fold partition depends only on the
 // job's size, so every result is bit-identical whether the job runs alone
-// or in a mix.  The tiling itself follows the load: at light load the blur
-// segments are shortened until a job alone spreads over the device.
+// or in a mix.  The tiling itself follows the load: at light load smaller
+// tiles and shorter z-segments spread a job alone over the device.
 #include <algorithm>
 #include <chrono>
 #include <cstring>
@@ -47,6 +47,7 @@
 #include <vector>
 
 #include "blur_item.hpp"
+#include "blur_tile.hpp"
 #include "heat.hpp"
 
 namespace mslhip {
@@ -55,31 +56,33 @@ int mean_step(float *out, const float *in, int rows, int cols, int r, float nv, 
 int heat_step(float *out, const float *in, int nx, int ny, int nz, float nv, float *maxdiff);
 
 constexpr int kRing = 3;             // rounds in flight
-constexpr int kMaxSub = 8;           // steps per round while the active items cannot fill the GPU
+constexpr int kMaxSub = 8;           // most launches per round and stencil kind
+constexpr double kRoundUs = 250.0;   // GPU time that a round's launches aim at
 constexpr int kMapChunk = 1 << 16;   // elements per map+fold work item
-constexpr int kHeatZseg = 16;        // z-planes per heat work item
+constexpr int kSumChunk = 1 << 13;   // elements per work item of a final state's fold
 constexpr size_t kAlign = 256;
 const float kScale255 = 255.0f / 16777216.0f;
 const float kScaleUnit = 1.0f / 16777216.0f;
 
 // ---- per-round descriptors (device) ------------------------------------------
-// A stencil job's step k of the round (k < nsub) reads state a when
+// Launch k of the round advances a stencil job by `gens` generations, or by
+// what is left of its `steps` in the round; it reads state a when
 // parity0 + k is even (b otherwise) and writes the other one.
 struct SBlur {
     float *a;
     float *b;
-    int rows, cols, r, kind;
+    int rows, cols, r;
     float nv;
-    int strips_x, seg, item0, nitems, parity0, nsub;
+    int tiles_x, tile_w, tile_h, item0, nitems, parity0, gens, steps;
 };
 struct SHeat {
     float *a;
     float *b;
     int nx, ny, nz;
     float nv;
-    int xtiles, ytiles, zseg, item0, nitems, parity0, nsub;
+    int xtiles, ytiles, zseg, item0, nitems, parity0, steps;
 };
-// The final state of a finishing stencil job, folded in kMapChunk chunks.
+// The final state of a finishing stencil job, folded in kSumChunk chunks.
 struct SSum {
     const float *data;
     long long n;
@@ -96,8 +99,8 @@ struct SFinal {
 };
 
 // item_desc[i] = largest j with starts[j] <= i (starts ascending, starts[0] = 0);
-// also clears the round's nctr work-queue counters of this kind, one per step
-// of the round (the work kernels run after this one on the same stream).
+// also clears the round's nctr work-queue counters of this kind, one per launch
+// (the work kernels run after this one on the same stream).
 __global__ void serve_expand_kernel(const int *__restrict__ starts, int ndesc, int nitems, int *__restrict__ item_desc,
                                     unsigned *__restrict__ ctr, int nctr) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -121,44 +124,70 @@ __device__ __forceinline__ int serve_next_item(unsigned *ctr, int stride) {
     return stride + __builtin_amdgcn_readfirstlane((int)nx);
 }
 
-// Step k of the round over every item of every active blur job (items of
-// jobs with fewer steps in this round are skipped).
-__global__ __launch_bounds__(256) void serve_blur_kernel(const SBlur *__restrict__ descs,
-                                                         const int *__restrict__ item_desc, int nitems,
-                                                         unsigned *__restrict__ ctr, int k_step) {
-    __shared__ __attribute__((aligned(16))) float lds[4][2 * kBatchLdsw];
-    const int wave = threadIdx.x >> 6;
-    const int nw = gridDim.x * 4;
-    for (int i = __builtin_amdgcn_readfirstlane((int)xcd_tile(blockIdx.x, gridDim.x) * 4 + wave); i < nitems;
-         i = serve_next_item(ctr, nw)) {
-        const int j = __builtin_amdgcn_readfirstlane(item_desc[i]);
-        const SBlur g = descs[j];
-        if (k_step >= g.nsub) continue;
-        const bool odd = (g.parity0 + k_step) & 1;
-        const float *src = odd ? g.b : g.a;
-        float *dst = odd ? g.a : g.b;
-        const int k = i - g.item0;
-        const int sw = g.kind == kKindNarrow1 ? 64 : 256;
-        const int xs = (k % g.strips_x) * sw;
-        const int sy = k / g.strips_x;
-        const int y0 = sy * g.seg;
-        const int y1 = min(y0 + g.seg, g.rows);
-        LaneSum ls;
-        blur_item_r<false>(g.r, src, dst, g.rows, g.cols, g.nv, g.kind, xs, y0, y1, lds[wave], &ls, sy & 1);
+// Most generations of a blur job per launch: as many as the LDS tile still
+// leaves at least half of its columns and rows (W = 128: the fewest row
+// overlaps per output; W = 64, at light load, where launches count).
+// us per generation of 2048^2 at 1 / 2 / 3 / 4 generations and W = 128, M = 4:
+// r = 3 10.6 / 7.3 / 6.8 / 6.1, r = 5 11.1 / 9.1 / 8.4 / 8.5, r = 7 12.0 /
+// 10.4 / 11.0, r = 10 13.6 / 13.4 / 19.6.
+constexpr int kHeavyGens[kBatchMaxR + 1] = {0, 6, 4, 4, 3, 3, 2, 2, 2, 2, 2};
+constexpr int kLightGens[kBatchMaxR + 1] = {0, 6, 6, 6, 4, 4, 3, 3, 2, 2, 2};
+constexpr int kHeavyW = 128, kHeavyM = 4;
+constexpr int kLightW = 64, kLightM = 1;
+
+template <int W, int M, int R = 1>
+__device__ __forceinline__ void serve_blur_tile(const SBlur &g, const float *src, float *dst, int gens, int tx, int ty,
+                                                float *lds) {
+    if constexpr (R < kBatchMaxR) {
+        if (g.r != R) return serve_blur_tile<W, M, R + 1>(g, src, dst, gens, tx, ty, lds);
+    }
+    blur_tile<R, W, M>(dst, src, g.rows, g.cols, g.nv, gens, g.tile_w, g.tile_h, tx, ty, lds);
+}
+
+// LDS of the largest tile of either kind: 64 output rows of the first
+// generation at the largest radius.
+constexpr size_t serve_tile_lds(int w) { return blur_tile_lds(kBatchMaxR, w, kTileRows, 1); }
+
+// Launch k of the round over every tile of every active blur job (tiles of
+// jobs that are done in this round are skipped); one workgroup per tile, the
+// next tile from the launch's counter.  Bound by VALU issue at load and by
+// the latency of a tile's barriers and loads otherwise.  128 jobs at once:
+// 42 ms of one-step strip items (486 launches of 86 us) before.
+template <int W, int M>
+__global__ __launch_bounds__(16 * W / M) void serve_blur_kernel(const SBlur *__restrict__ descs,
+                                                                const int *__restrict__ item_desc, int nitems,
+                                                                unsigned *__restrict__ ctr, int k_launch) {
+    extern __shared__ __attribute__((aligned(16))) float lds[];
+    __shared__ int next;
+    for (int i = (int)xcd_tile(blockIdx.x, gridDim.x); i < nitems;) {
+        const SBlur g = descs[__builtin_amdgcn_readfirstlane(item_desc[i])];
+        const int gens = min(g.gens, g.steps - k_launch * g.gens);
+        if (gens > 0) {
+            const bool odd = (g.parity0 + k_launch) & 1;
+            const int k = i - g.item0;
+            serve_blur_tile<W, M>(g, odd ? g.b : g.a, odd ? g.a : g.b, gens, k % g.tiles_x, k / g.tiles_x, lds);
+        }
+        if (threadIdx.x == 0) next = (int)(gridDim.x + atomicAdd(ctr, 1u));
+        __syncthreads();  // also: the tile's last reads of lds are done
+        i = __builtin_amdgcn_readfirstlane(next);
+        __syncthreads();
     }
 }
 
+// Launch k of the round over every item of every active heat job: two
+// generations, or the last one of an odd count.
 __global__ __launch_bounds__(256) void serve_heat_kernel(const SHeat *__restrict__ descs,
                                                          const int *__restrict__ item_desc, int nitems,
-                                                         unsigned *__restrict__ ctr, int k_step) {
+                                                         unsigned *__restrict__ ctr, int k_launch) {
     const int wave = threadIdx.x >> 6;
     const int nw = gridDim.x * 4;
     for (int i = __builtin_amdgcn_readfirstlane((int)xcd_tile(blockIdx.x, gridDim.x) * 4 + wave); i < nitems;
          i = serve_next_item(ctr, nw)) {
         const int j = __builtin_amdgcn_readfirstlane(item_desc[i]);
         const SHeat g = descs[j];
-        if (k_step >= g.nsub) continue;
-        const bool odd = (g.parity0 + k_step) & 1;
+        const int gens = g.steps - 2 * k_launch;
+        if (gens <= 0) continue;
+        const bool odd = (g.parity0 + k_launch) & 1;
         const float *src = odd ? g.b : g.a;
         float *dst = odd ? g.a : g.b;
         const int k = i - g.item0;
@@ -167,8 +196,10 @@ __global__ __launch_bounds__(256) void serve_heat_kernel(const SHeat *__restrict
         const int yt = rest % g.ytiles;
         const int z0 = (rest / g.ytiles) * g.zseg;
         const int z1 = min(z0 + g.zseg, g.nz);
-        float dmax = 0.0f;
-        heat7_march<false, false>(dst, src, g.nx, g.ny, g.nz, g.nv, xt * kTX, yt * kTY, z0, z1, &dmax, nullptr);
+        if (gens >= 2)
+            heat7x2_march<false, true>(dst, src, g.nx, g.ny, g.nz, g.nv, xt * kT2X, yt * kT2Y, z0, z1, nullptr);
+        else
+            heat7x2_march<false, true, true>(dst, src, g.nx, g.ny, g.nz, g.nv, xt * kT2X, yt * kT2Y, z0, z1, nullptr);
     }
 }
 
@@ -206,9 +237,11 @@ __global__ __launch_bounds__(256) void serve_map_kernel(const SMap *__restrict__
     }
 }
 
-// Compensated sum of one kMapChunk chunk of a finished stencil job's final
-// state: each lane pushes its elements (16-byte loads, lane-strided) into a
-// TwoSum pair, the wave combines the lanes in a fixed butterfly.
+// Compensated sum of one kSumChunk chunk of a finished stencil job's final
+// state: each lane pushes its elements (16-byte loads, lane-strided, four in
+// flight) into a TwoSum pair, the wave combines the lanes in a fixed
+// butterfly.  Short chunks: a job's few chunks run at once, each a chain of
+// loads (64 Ki elements per chunk, one load in flight: 126 us a launch).
 __global__ __launch_bounds__(256) void serve_sum_kernel(const SSum *__restrict__ descs,
                                                         const int *__restrict__ item_desc, int nitems,
                                                         float2 *__restrict__ partials) {
@@ -218,15 +251,28 @@ __global__ __launch_bounds__(256) void serve_sum_kernel(const SSum *__restrict__
          i += nw) {
         const int j = __builtin_amdgcn_readfirstlane(item_desc[i]);
         const SSum g = descs[j];
-        const long long e0 = (long long)(i - g.item0) * kMapChunk;
-        const long long e1 = min(e0 + (long long)kMapChunk, g.n);
+        const long long e0 = (long long)(i - g.item0) * kSumChunk;
+        const long long e1 = min(e0 + (long long)kSumChunk, g.n);
         LaneSum ls;
         long long e = e0;
         if ((((uintptr_t)(g.data + e0)) & 15u) == 0) {
             typedef float v4f_t __attribute__((ext_vector_type(4)));
             const long long nq = (e1 - e0) / 4;
             const v4f_t *q = reinterpret_cast<const v4f_t *>(g.data + e0);
-            for (long long t = lane; t < nq; t += 64) {
+            long long t = lane;
+            for (; t + 192 < nq; t += 256) {
+                v4f_t v[4];
+#pragma unroll
+                for (int u = 0; u < 4; u++) v[u] = q[t + 64 * u];
+#pragma unroll
+                for (int u = 0; u < 4; u++) {
+                    ls.push(v[u].x);
+                    ls.push(v[u].y);
+                    ls.push(v[u].z);
+                    ls.push(v[u].w);
+                }
+            }
+            for (; t < nq; t += 64) {
                 const v4f_t v = q[t];
                 ls.push(v.x);
                 ls.push(v.y);
@@ -338,9 +384,10 @@ struct SJob {
     float *a = nullptr, *b = nullptr;
     uint32_t *u = nullptr;
     int steps_done = 0;
-    int nsub = 0;  // steps in the round being planned
-    // tiling
-    int kind = 0, strips_x = 0, seg = 0, xtiles = 0, ytiles = 0, nitems = 0;
+    int in_b = 0;     // 1: the state after steps_done steps is in b
+    // the round being planned: steps, generations per launch, tiling
+    int steps = 0, gens = 0;
+    int tile_w = 0, tile_h = 0, tiles_x = 0, xtiles = 0, ytiles = 0, zseg = 0, nitems = 0;
     double sum = 0.0;
     uint32_t sum_u32 = 0;
 };
@@ -410,45 +457,29 @@ static int validate_job(const msl_job &j, size_t budget) {
     return MSL_OK;
 }
 
-// A job's strip layout and (for the fold) chunk count, fixed at admission.
-// Blur segments of a round: 64 rows (32 for one column per lane) under
-// load; at light load (fine) short enough that a job alone spreads over the
-// device, about 4 waves per CU (a large grid served alone otherwise ran on an
-// eighth of the GPU), but at least 4 / 8 / 16 rows for r <= 2, <= 6 and
-// above so that the 2r halo rows stay a modest share.  The results do not
-// depend on the segments.
-static void tile_blur(SJob &J, bool fine) {
+// A blur job's tiles of a round.  Under load W = 128 tiles of up to 48 rows;
+// at light load W = 64 tiles, as low as 8 rows, that spread the job over about
+// one workgroup per CU.  The results do not depend on the tiles.
+static void tile_blur(SJob &J, bool light) {
     const msl_job &s = J.spec;
-    const int rows = s.d0;
-    const int seg_max = J.kind == kKindNarrow1 ? 32 : 64;
-    J.seg = seg_max;
-    if (fine) {
-        const long target = (long)ctx().num_cus * 4;
-        const long segs = (target + J.strips_x - 1) / J.strips_x;
-        const int seg_min = s.r <= 2 ? 4 : (s.r <= 6 ? 8 : 16);
-        J.seg = std::min(seg_max, std::max(seg_min, (int)((rows + segs - 1) / segs)));
-    }
-    J.nitems = J.strips_x * ((rows + J.seg - 1) / J.seg);
+    const int w = light ? kLightW : kHeavyW;
+    J.gens = std::min(light ? kLightGens[s.r] : kHeavyGens[s.r], s.steps);
+    J.tile_w = (w - 2 * s.r * J.gens) / 4 * 4;
+    J.tiles_x = (s.d1 + J.tile_w - 1) / J.tile_w;
+    J.tile_h = std::min((kTileRows - 2 * s.r * (J.gens - 1)) / 8 * 8, 48);
+    if (light)
+        while (J.tile_h > 8 && (long)J.tiles_x * ((s.d0 + J.tile_h - 1) / J.tile_h) < ctx().num_cus / 2) J.tile_h -= 8;
+    J.nitems = J.tiles_x * ((s.d0 + J.tile_h - 1) / J.tile_h);
 }
 
-static void plan_job(SJob &J) {
+// A heat job's items of a round: the march handles whole blocks of kP planes
+// of its zseg + 1, so zseg is one less than a multiple.
+static void tile_heat(SJob &J, int zseg) {
     const msl_job &s = J.spec;
-    if (s.kind == MSL_JOB_BLUR2D) {
-        const int cols = s.d1;
-        const bool narrow = cols < 192 || s.r > kBatchMaxR4 || cols < 4;
-        const uintptr_t al = (uintptr_t)J.a | (uintptr_t)J.b;
-        J.kind = narrow ? kKindNarrow1 : (((cols & 3) == 0 && (al & 15u) == 0) ? kKindAligned4 : kKindUnaligned4);
-        const int sw = narrow ? 64 : 256;
-        J.strips_x = (cols + sw - 1) / sw;
-        tile_blur(J, false);
-    } else if (s.kind == MSL_JOB_HEAT3D) {
-        J.xtiles = (s.d0 + kTX - 1) / kTX;
-        J.ytiles = (s.d1 + kTY - 1) / kTY;
-        J.seg = kHeatZseg;
-        J.nitems = J.xtiles * J.ytiles * ((s.d2 + kHeatZseg - 1) / kHeatZseg);
-    } else {
-        J.nitems = (int)((s.n + kMapChunk - 1) / kMapChunk);
-    }
+    J.xtiles = (s.d0 + kT2X - 1) / kT2X;
+    J.ytiles = (s.d1 + kT2Y - 1) / kT2Y;
+    J.zseg = zseg;
+    J.nitems = J.xtiles * J.ytiles * ((s.d2 + zseg - 1) / zseg);
 }
 
 static int slot_alloc(RoundSlot &R, int max_active) {
@@ -611,7 +642,7 @@ static int run_round(Server &S, int *did_work) {
                 J->a = reinterpret_cast<float *>(p);
                 J->b = reinterpret_cast<float *>(p + J->bytes / 2);
             }
-            plan_job(*J);
+            if (s.kind == MSL_JOB_MAPFOLD_U32) J->nitems = (int)((s.n + kMapChunk - 1) / kMapChunk);
             int frc = MSL_OK;
             if (s.kind == MSL_JOB_BLUR2D) {
                 frc = msl_fill_uniform_f32(J->a, (size_t)s.d0 * s.d1, s.seed, kScale255);
@@ -631,8 +662,7 @@ static int run_round(Server &S, int *did_work) {
 
     // ---- descriptors of this round
     std::stable_sort(S.blur.begin(), S.blur.end(), [](const SJob *x, const SJob *y) {
-        if (x->spec.r != y->spec.r) return x->spec.r < y->spec.r;
-        return x->kind < y->kind;
+        return x->spec.r < y->spec.r;
     });
     std::vector<SBlur> db;
     std::vector<SHeat> dh;
@@ -642,24 +672,38 @@ static int run_round(Server &S, int *did_work) {
     std::vector<int> sb, sh, sm, ss;
     std::vector<std::pair<SJob *, int>> finishing;
     int items[4] = {0, 0, 0, 0};
-    // Light load: the active stencil jobs' items at the default tiling
-    // cannot fill one persistent launch (3 workgroups of 4 waves per CU).
-    // Then the blur segments are shortened and each job advances up to
-    // kMaxSub steps this round (per-round host work and launch latency would
-    // otherwise dominate); under load one step with the default tiling.
-    long stencil_items = 0;
+    // Light load: fewer W = 128 tiles than two per CU.
+    long blur_items = 0, heat_items = 0;
+    double blur_us = 0.0, heat_us = 0.0;
     for (SJob *J : S.blur) {
+        const msl_job &s = J->spec;
         tile_blur(*J, false);
-        stencil_items += J->nitems;
+        blur_items += J->nitems;
+        // VALU issue of a launch: 4 cycles per 64 lane operations on 4 SIMDs
+        // per CU at 2.4 GHz, with a third for the tiles' overlaps
+        blur_us += (double)s.d0 * s.d1 * J->gens * (4 * s.r + 10) * 1.33 / (ctx().num_cus * 64 * 2400.0);
     }
-    for (SJob *J : S.heat) stencil_items += J->nitems;
-    const bool light = stencil_items < (long)ctx().num_cus * 12;
-    const int ksteps = light ? kMaxSub : 1;
+    const bool light = blur_items < 2L * ctx().num_cus;
     if (light)
         for (SJob *J : S.blur) tile_blur(*J, true);
-    // the fold of a finishing stencil job: its final state in kMapChunk chunks
+    // z-segments of 31 planes (32 steps of the march); shorter ones while the
+    // items are fewer than 8 waves per CU
+    for (int zseg = 31;; zseg = (zseg - 1) / 2) {
+        heat_items = 0;
+        for (SJob *J : S.heat) {
+            tile_heat(*J, zseg);
+            heat_items += J->nitems;
+        }
+        if (zseg <= 7 || heat_items >= 8L * ctx().num_cus) break;
+    }
+    for (SJob *J : S.heat)  // 8 bytes per cell and launch at 3.5 TB/s
+        heat_us += (double)J->spec.d0 * J->spec.d1 * J->spec.d2 * 8.0 / 3.5e6;
+    // at least 8 us per launch of either kind
+    const double sub_us = (S.blur.empty() ? 0.0 : std::max(8.0, blur_us)) + (S.heat.empty() ? 0.0 : std::max(8.0, heat_us));
+    const int nsub = std::max(1, std::min(kMaxSub, (int)(kRoundUs / sub_us)));
+    // the fold of a finishing stencil job: its final state in kSumChunk chunks
     auto add_sum = [&](SJob *J, const float *data, long long n, int slot) {
-        const int nchunks = (int)((n + kMapChunk - 1) / kMapChunk);
+        const int nchunks = (int)((n + kSumChunk - 1) / kSumChunk);
         ds.push_back(SSum{data, n, items[3], nchunks});
         ss.push_back(items[3]);
         fin.push_back(SFinal{J->spec.kind, items[3], nchunks, slot});
@@ -667,26 +711,33 @@ static int run_round(Server &S, int *did_work) {
         items[3] += nchunks;
     };
     int nsub_max[2] = {0, 0};
+    // the job's steps of this round, and the buffer that holds its state after
+    auto plan_steps = [&](SJob *J, int gens, int *most) {
+        J->steps = std::min(gens * nsub, J->spec.steps - J->steps_done);
+        const int launches = (J->steps + gens - 1) / gens;
+        *most = std::max(*most, launches);
+        return (J->in_b + launches) & 1;
+    };
     for (SJob *J : S.blur) {
         const msl_job &s = J->spec;
-        J->nsub = std::min(ksteps, s.steps - J->steps_done);
-        nsub_max[0] = std::max(nsub_max[0], J->nsub);
-        db.push_back(SBlur{J->a, J->b, s.d0, s.d1, s.r, J->kind, s.nv, J->strips_x, J->seg, items[0], J->nitems,
-                           J->steps_done & 1, J->nsub});
+        const int to_b = plan_steps(J, J->gens, &nsub_max[0]);
+        db.push_back(SBlur{J->a, J->b, s.d0, s.d1, s.r, s.nv, J->tiles_x, J->tile_w, J->tile_h, items[0], J->nitems,
+                           J->in_b, J->gens, J->steps});
         sb.push_back(items[0]);
-        if (J->steps_done + J->nsub == s.steps)
-            add_sum(J, (s.steps & 1) ? J->b : J->a, (long long)s.d0 * s.d1, (int)fin.size());
+        J->in_b = to_b;
+        if (J->steps_done + J->steps == s.steps)
+            add_sum(J, to_b ? J->b : J->a, (long long)s.d0 * s.d1, (int)fin.size());
         items[0] += J->nitems;
     }
     for (SJob *J : S.heat) {
         const msl_job &s = J->spec;
-        J->nsub = std::min(ksteps, s.steps - J->steps_done);
-        nsub_max[1] = std::max(nsub_max[1], J->nsub);
-        dh.push_back(SHeat{J->a, J->b, s.d0, s.d1, s.d2, s.nv, J->xtiles, J->ytiles, J->seg, items[1], J->nitems,
-                           J->steps_done & 1, J->nsub});
+        const int to_b = plan_steps(J, 2, &nsub_max[1]);
+        dh.push_back(SHeat{J->a, J->b, s.d0, s.d1, s.d2, s.nv, J->xtiles, J->ytiles, J->zseg, items[1], J->nitems,
+                           J->in_b, J->steps});
         sh.push_back(items[1]);
-        if (J->steps_done + J->nsub == s.steps)
-            add_sum(J, (s.steps & 1) ? J->b : J->a, (long long)s.d0 * s.d1 * s.d2, (int)fin.size());
+        J->in_b = to_b;
+        if (J->steps_done + J->steps == s.steps)
+            add_sum(J, to_b ? J->b : J->a, (long long)s.d0 * s.d1 * s.d2, (int)fin.size());
         items[1] += J->nitems;
     }
     for (SJob *J : maps) {
@@ -745,9 +796,14 @@ static int run_round(Server &S, int *did_work) {
         serve_expand_kernel<<<(items[1] + 255) / 256, 256, 0, st>>>(gsh, (int)dh.size(), items[1], R.d_item_desc[1],
                                                                     R.d_ctr + kMaxSub, nsub_max[1]);
     for (int k = 0; k < std::max(nsub_max[0], nsub_max[1]); k++) {
-        if (k < nsub_max[0])
-            serve_blur_kernel<<<persistent(items[0], 3), 256, 0, st>>>(gb, R.d_item_desc[0], items[0], R.d_ctr + k,
-                                                                       k);
+        if (k < nsub_max[0] && light)
+            serve_blur_kernel<kLightW, kLightM>
+                <<<std::min(items[0], cus), 16 * kLightW / kLightM, serve_tile_lds(kLightW), st>>>(
+                    gb, R.d_item_desc[0], items[0], R.d_ctr + k, k);
+        else if (k < nsub_max[0])
+            serve_blur_kernel<kHeavyW, kHeavyM>
+                <<<std::min(items[0], cus * 3), 16 * kHeavyW / kHeavyM, serve_tile_lds(kHeavyW), st>>>(
+                    gb, R.d_item_desc[0], items[0], R.d_ctr + k, k);
         if (k < nsub_max[1])
             serve_heat_kernel<<<persistent(items[1], 3), 256, 0, st>>>(gh, R.d_item_desc[1], items[1],
                                                                        R.d_ctr + kMaxSub + k, k);
@@ -774,7 +830,7 @@ static int run_round(Server &S, int *did_work) {
     auto advance = [](std::vector<SJob *> &v) {
         size_t w = 0;
         for (SJob *J : v) {
-            J->steps_done += J->nsub;
+            J->steps_done += J->steps;
             if (J->steps_done < J->spec.steps) v[w++] = J;
         }
         v.resize(w);
@@ -940,7 +996,7 @@ int msl_server_poll(void *server, int64_t id, msl_job_result *h_result, void *h_
             src = J->u;
         } else {
             nbytes = (s.kind == MSL_JOB_BLUR2D ? (size_t)s.d0 * s.d1 : (size_t)s.d0 * s.d1 * s.d2) * 4;
-            src = (s.steps & 1) ? J->b : J->a;
+            src = J->in_b ? J->b : J->a;
         }
         MSL_REQUIRE(final_bytes >= nbytes, "msl_server_poll: final buffer too small");
         MSL_HIP_TRY(hipMemcpyAsync(h_final, src, nbytes, hipMemcpyDeviceToHost, ctx().stream));
