@@ -31,6 +31,8 @@ SOURCES = [
     "gol.hip",
     "blur_tile.hip",
     "stencil3d.hip",
+    "heat_tile.hip",
+    "heat_pair.hip",
     "batch.hip",
     "serve.hip",
 ]

@@ -12,6 +12,8 @@
 // is computed in exactly that order (examples/heatdiffusion.cpp:55-65).
 #pragma once
 
+#include <type_traits>
+
 #include "strip.hpp"
 
 namespace mslhip {
@@ -143,9 +145,8 @@ __device__ __forceinline__ void heat7_march(float *__restrict__ out, const float
 // then generation 2 of plane z-1 from the ring of generation-1 planes.
 // Generation-1 cells outside the cube are nv, as the second step reads them.
 // Every cell is computed in the one-step order, so the result is
-// bit-identical to two single steps.  kResidual: max |generation 2 -
-// generation 1| into *dmax.  kSingle: generation 1 only, of the same tile
-// (the odd step of a job whose items are laid out for two).
+// bit-identical to two single steps.  kSingle: generation 1 only, of the same
+// tile (the odd step of a job whose items are laid out for two).
 constexpr int kT2X = kTX - 4;  // output columns of a two-generation wave tile
 // Output rows of a two-generation wave tile: 5 rows (90 VGPRs, five waves
 // per SIMD) beat 8 (124, four) although the y halo grows from 4/8 to 4/5
@@ -153,9 +154,9 @@ constexpr int kT2X = kTX - 4;  // output columns of a two-generation wave tile
 // 320^3: 8 rows 7.13 ms, 5 6.90).
 constexpr int kT2Y = 5;
 
-template <bool kResidual, bool NT = true, bool kSingle = false>
+template <bool kSingle>
 __device__ __forceinline__ void heat7x2_march(float *__restrict__ out, const float *__restrict__ in, int nx, int ny,
-                                              int nz, float nv, int x0, int y0, int z0, int z1, float *dmax) {
+                                              int nz, float nv, int x0, int y0, int z0, int z1) {
     constexpr int NI = kT2Y + 4;  // input rows y0-2 .. y0+kT2Y+1
     constexpr int N1 = kT2Y + 2;  // generation-1 rows y0-1 .. y0+kT2Y
     const int lane = threadIdx.x & 63;
@@ -184,9 +185,10 @@ __device__ __forceinline__ void heat7x2_march(float *__restrict__ out, const flo
 #pragma unroll
         for (int j = 0; j < NI; j++) inp[j][slot] = (zok && ((iok >> j) & 1u)) ? inp[j][slot] : nv;
     };
-    // one step of the 7-point rule on a lane's column: rows r-1, r, r+1 of
-    // plane slots (below, centre, above), x neighbours from the adjacent lanes
-    auto cell = [&](float(&a)[kP], float(&m)[kP], float(&b)[kP], float(&zl)[kP], float(&zh)[kP], int sb, int sc,
+    // one step of the 7-point rule on a lane's column before the division:
+    // rows r-1, r, r+1 of plane slots (below, centre, above), x neighbours from
+    // the adjacent lanes
+    auto sum7 = [&](float(&a)[kP], float(&m)[kP], float(&b)[kP], float(&zl)[kP], float(&zh)[kP], int sb, int sc,
                     int sa) -> float {
         (void)sb;
         (void)sa;
@@ -196,17 +198,36 @@ __device__ __forceinline__ void heat7x2_march(float *__restrict__ out, const flo
         v = __fadd_rn(v, a[sc]);             // y-1
         v = __fadd_rn(v, b[sc]);             // y+1
         v = __fadd_rn(v, zl[sb]);            // z-1
-        v = __fadd_rn(v, zh[sa]);            // z+1
-        return div6_plus0(v);
+        return __fadd_rn(v, zh[sa]);         // z+1
+    };
+    // The divisions of a plane's rows take the three-operation form; when one
+    // of the wave's results asks for it, all are redone by the full form (the
+    // sums are still in registers).
+    auto divide = [&](auto &v, auto n) {
+        constexpr int N = decltype(n)::value;
+        float q[N];
+        bool suspect = false;
+#pragma unroll
+        for (int j = 0; j < N; j++) {
+            q[j] = div6_fast(v[j]);
+            suspect |= div6_suspect(q[j]);
+        }
+        if (__any(suspect)) {
+#pragma unroll
+            for (int j = 0; j < N; j++) q[j] = div6_plus0(v[j]);
+        }
+#pragma unroll
+        for (int j = 0; j < N; j++) v[j] = q[j];
     };
     // generation 1 of plane zi from input slots (zi-1, zi, zi+1) into g1 slot d
     auto gen1 = [&](int zi, int sb, int sc, int sa, int d) {
         const bool zok = (unsigned)zi < (unsigned)nz;
+        float v[N1];
 #pragma unroll
-        for (int j = 0; j < N1; j++) {
-            const float v = cell(inp[j], inp[j + 1], inp[j + 2], inp[j + 1], inp[j + 1], sb, sc, sa);
-            g1[j][d] = (zok && ((iok >> (j + 1)) & 1u)) ? v : nv;
-        }
+        for (int j = 0; j < N1; j++) v[j] = sum7(inp[j], inp[j + 1], inp[j + 2], inp[j + 1], inp[j + 1], sb, sc, sa);
+        divide(v, std::integral_constant<int, N1>{});
+#pragma unroll
+        for (int j = 0; j < N1; j++) g1[j][d] = (zok && ((iok >> (j + 1)) & 1u)) ? v[j] : nv;
     };
 
 #pragma unroll
@@ -231,21 +252,18 @@ __device__ __forceinline__ void heat7x2_march(float *__restrict__ out, const flo
             const int zo = zi - 1;
             const int tb = (u + 3) & 3, tc = u & 3, ta = (u + 1) & 3;  // g1 slots of zo-1, zo, zo+1
             char *op = reinterpret_cast<char *>(out + (size_t)min(max(zo, 0), nz - 1) * plane);
+            float w[kT2Y];
+#pragma unroll
+            for (int j = 0; j < kT2Y; j++)
+                w[j] = kSingle ? g1[j + 1][tc] : sum7(g1[j], g1[j + 1], g1[j + 2], g1[j + 1], g1[j + 1], tb, tc, ta);
+            if constexpr (!kSingle) divide(w, std::integral_constant<int, kT2Y>{});
 #pragma unroll
             for (int j = 0; j < kT2Y; j++) {
-                const float v =
-                    kSingle ? g1[j + 1][tc] : cell(g1[j], g1[j + 1], g1[j + 2], g1[j + 1], g1[j + 1], tb, tc, ta);
+                const float v = w[j];
                 // output row y0+j is input row j+2: stored when in the cube
                 if (zo >= z0 && zo < z1 && lane >= 2 && lane <= 61 && ((iok >> (j + 2)) & 1u)) {
                     float *o = reinterpret_cast<float *>(op + ioff[j + 2]);
-                    if constexpr (NT)
-                        __builtin_nontemporal_store(v, o);
-                    else
-                        *o = v;
-                    if constexpr (kResidual) {
-                        const float dd = fabsf(__fsub_rn(v, g1[j + 1][tc]));
-                        *dmax = dd > *dmax ? dd : *dmax;
-                    }
+                    __builtin_nontemporal_store(v, o);
                 }
             }
         }

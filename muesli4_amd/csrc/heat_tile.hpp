@@ -1,0 +1,11 @@
+// Heat steps in LDS: 3-D tiles, several generations per launch (heat_tile.hip),
+// and the plane march of two generations (heat_pair.hip).
+#pragma once
+
+namespace mslhip {
+
+int heat_tile_step(float *out, const float *in, int nx, int ny, int nz, float nv, int steps, bool small,
+                   float *maxdiff);
+int heat_pair_step(float *out, const float *in, int nx, int ny, int nz, float nv, float *maxdiff);
+
+}  // namespace mslhip

@@ -197,9 +197,9 @@ __global__ __launch_bounds__(256) void serve_heat_kernel(const SHeat *__restrict
         const int z0 = (rest / g.ytiles) * g.zseg;
         const int z1 = min(z0 + g.zseg, g.nz);
         if (gens >= 2)
-            heat7x2_march<false, true>(dst, src, g.nx, g.ny, g.nz, g.nv, xt * kT2X, yt * kT2Y, z0, z1, nullptr);
+            heat7x2_march<false>(dst, src, g.nx, g.ny, g.nz, g.nv, xt * kT2X, yt * kT2Y, z0, z1);
         else
-            heat7x2_march<false, true, true>(dst, src, g.nx, g.ny, g.nz, g.nv, xt * kT2X, yt * kT2Y, z0, z1, nullptr);
+            heat7x2_march<true>(dst, src, g.nx, g.ny, g.nz, g.nv, xt * kT2X, yt * kT2Y, z0, z1);
     }
 }
 

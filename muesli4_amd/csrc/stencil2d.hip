@@ -466,8 +466,8 @@ __global__ void zero_u64_kernel(unsigned long long *p) { *p = 0ull; }
 // Every 32-bit pattern x: compare div_odd_square(x) (or div6, the heat
 // division, or div_plus0 against (0 + x) / d) with x / d bit for bit (NaN against NaN counts as equal);
 // one atomic per block.
-// kKind 0: div_odd_square, 1: div6, 2: div_plus0 and 3: div6_plus0, the last
-// two against (0 + x) / d
+// kKind 0: div_odd_square, 1: div6, 2: div_plus0, 3: div6_plus0 and 4:
+// div6_fast where div6_suspect passes it, the last three against (0 + x) / d
 template <int kKind>
 __global__ __launch_bounds__(256) void div_check_kernel(float d, float rcp, unsigned long long *count) {
     __shared__ unsigned int part[256];
@@ -483,6 +483,9 @@ __global__ __launch_bounds__(256) void div_check_kernel(float d, float rcp, unsi
             got = div_plus0(x, d, rcp);
         } else if constexpr (kKind == 3) {
             got = div6_plus0(x);
+        } else if constexpr (kKind == 4) {
+            got = div6_fast(x);
+            if (div6_suspect(got)) got = ref;
         } else {
             got = div_odd_square(x, d, rcp);
         }
@@ -591,6 +594,7 @@ int msl_selftest_div_six(uint64_t *h_mismatches) {
     zero_u64_kernel<<<1, 1, 0, ctx().stream>>>(d_count);
     div_check_kernel<1><<<ctx().num_cus * 8, 256, 0, ctx().stream>>>(6.0f, 1.0f / 6.0f, d_count);
     div_check_kernel<3><<<ctx().num_cus * 8, 256, 0, ctx().stream>>>(6.0f, 1.0f / 6.0f, d_count);
+    div_check_kernel<4><<<ctx().num_cus * 8, 256, 0, ctx().stream>>>(6.0f, 1.0f / 6.0f, d_count);
     rc = check_launch("msl_selftest_div_six");
     unsigned long long h = 0;
     hipError_t e = hipMemcpyAsync(&h, d_count, sizeof h, hipMemcpyDeviceToHost, ctx().stream);

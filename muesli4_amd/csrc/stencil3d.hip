@@ -8,7 +8,8 @@
 // Here one wavefront owns a 64 x 8 column of the cube and marches a segment
 // of z-planes with all neighbours in registers (heat7_march): each cell is
 // read from HBM once and written once (8 bytes per cell per step), in the
-// reference functor's operation order.  The optional fused residual folds
+// reference functor's operation order.  Small cubes and iterations run other
+// kernels (heat_tile.hip, heat_pair.hip; see heat_way).  The optional fused residual folds
 // max |v - in| into one device scalar with an integer atomic max (the bit
 // patterns of non-negative floats order like unsigned integers).
 #include <cstdlib>
@@ -19,6 +20,7 @@
 #include <vector>
 
 #include "heat.hpp"
+#include "heat_tile.hpp"
 
 namespace mslhip {
 
@@ -39,38 +41,6 @@ __global__ __launch_bounds__(256) void heat7_kernel(float *__restrict__ out, con
         const int z0 = zs * zseg;
         heat7_march<kResidual, false, NT>(out, in, nx, ny, nz, nv, xt * kTX, yt * kTY, z0, min(z0 + zseg, nz), &dmax,
                                           nullptr);
-    }
-    if (kResidual) {
-        __shared__ float wmax[4];
-#pragma unroll
-        for (int m = 32; m >= 1; m >>= 1) {
-            const float o = __shfl_xor(dmax, m);
-            dmax = o > dmax ? o : dmax;
-        }
-        if (lane == 0) wmax[threadIdx.x >> 6] = dmax;
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            const float m = fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));
-            atomicMax(reinterpret_cast<unsigned int *>(maxdiff), __float_as_uint(m));
-        }
-    }
-}
-
-// Two generations per launch (heat7x2_march); tiles of kT2X x kT2Y columns.
-template <bool kResidual, bool NT>
-__global__ __launch_bounds__(256) void heat7x2_kernel(float *__restrict__ out, const float *__restrict__ in, int nx,
-                                                      int ny, int nz, float nv, int zseg, int xtiles, int ytiles,
-                                                      int nitems, float *__restrict__ maxdiff) {
-    const int lane = threadIdx.x & 63;
-    const int item = __builtin_amdgcn_readfirstlane((int)xcd_tile(blockIdx.x, gridDim.x) * 4 + (threadIdx.x >> 6));
-    float dmax = 0.0f;
-    if (item < nitems) {
-        const int xt = item % xtiles;
-        const int rest = item / xtiles;
-        const int yt = rest % ytiles;
-        const int zs = rest / ytiles;
-        const int z0 = zs * zseg;
-        heat7x2_march<kResidual, NT>(out, in, nx, ny, nz, nv, xt * kT2X, yt * kT2Y, z0, min(z0 + zseg, nz), &dmax);
     }
     if (kResidual) {
         __shared__ float wmax[4];
@@ -110,35 +80,22 @@ inline HeatShape heat_shape(int nx, int ny, int nz) {
     return s;
 }
 
-// Cubes above this size run their iterations two generations per launch:
-// the pass reads and writes half the bytes per generation but computes 1.3x
-// the cells (tile halos), which pays where HBM or the Infinity Cache bounds
-// the single step (measured: 272^3 4.4 -> 5.4 TB/s, 320^3 5.0 -> 5.6 TB/s,
-// 512^3 4.9 -> 6.5 TB/s) and not on smaller cubes (256^3 5.6 -> 4.8 TB/s).
-constexpr size_t kHeatPairMinBytes = (size_t)64 << 20;
-
-// Two generations in one launch; maxdiff (if any) gets the second one's
-// max |change|.
-int heat_step2(float *out, const float *in, int nx, int ny, int nz, float nv, float *maxdiff) {
-    HeatShape s = heat_shape(nx, ny, nz);
-    s.xtiles = (nx + kT2X - 1) / kT2X;
-    s.ytiles = (ny + kT2Y - 1) / kT2Y;
-    s.nitems = s.xtiles * s.ytiles * s.zsegs;
-    const bool nt = stream_stores((size_t)nx * ny * nz * sizeof(float));
-    const int blocks = (s.nitems + 3) / 4;
-    if (maxdiff && nt)
-        heat7x2_kernel<true, true><<<blocks, 256, 0, ctx().stream>>>(out, in, nx, ny, nz, nv, s.zseg, s.xtiles,
-                                                                     s.ytiles, s.nitems, maxdiff);
-    else if (maxdiff)
-        heat7x2_kernel<true, false><<<blocks, 256, 0, ctx().stream>>>(out, in, nx, ny, nz, nv, s.zseg, s.xtiles,
-                                                                      s.ytiles, s.nitems, maxdiff);
-    else if (nt)
-        heat7x2_kernel<false, true><<<blocks, 256, 0, ctx().stream>>>(out, in, nx, ny, nz, nv, s.zseg, s.xtiles,
-                                                                      s.ytiles, s.nitems, nullptr);
-    else
-        heat7x2_kernel<false, false><<<blocks, 256, 0, ctx().stream>>>(out, in, nx, ny, nz, nv, s.zseg, s.xtiles,
-                                                                       s.ytiles, s.nitems, nullptr);
-    return check_launch("msl_heat7_iterate_f32");
+// How a cube's iterations run.  us per generation, one-step march / small
+// tiles / large tiles / pair kernel: 32^3 12.5 / 1.6 / 3.0 / 5.1, 64^3 12.9 /
+// 1.7 / 3.0 / 4.7, 80^3 13.1 / 2.7 / 3.3 / 4.8, 100^3 13.4 / 3.8 / 3.7 / 5.6,
+// 128^3 14.1 / 5.2 / 5.4 / 5.4, 150^3 14.6 / 8.5 / 6.9 / 8.7, 200^3 17.8 / 14.9
+// / 11.1 / 10.8, 256^3 22.6 / 27.6 / 18.4 / 14.0, 512^3 215 / 242 / 138 / 106
+// (tiles at the generations per launch given here).
+struct HeatWay {
+    int gens;          // most generations per launch
+    bool tile, small;  // tile kernel and its region; else the pair kernel
+};
+static HeatWay heat_way(int nx, int ny, int nz) {
+    const size_t cells = (size_t)nx * ny * nz;
+    if (cells <= 350000) return HeatWay{4, true, true};
+    if (cells <= 900000) return HeatWay{3, true, true};
+    if (cells <= 4200000) return HeatWay{3, true, false};
+    return HeatWay{2, false, false};
 }
 
 int heat_step(float *out, const float *in, int nx, int ny, int nz, float nv, float *maxdiff) {
@@ -149,6 +106,8 @@ int heat_step(float *out, const float *in, int nx, int ny, int nz, float nv, flo
     MSL_REQUIRE((int64_t)nx * ny < ((int64_t)1 << 30), "msl_heat7_f32: plane of 2^30 cells or more");
     if (nx == 0 || ny == 0 || nz == 0) return MSL_OK;
     MSL_REQUIRE(out && in && out != in, "msl_heat7_f32: null or aliased buffers");
+    const HeatWay way = heat_way(nx, ny, nz);
+    if (way.tile) return heat_tile_step(out, in, nx, ny, nz, nv, 1, way.small, maxdiff);
     HeatShape s = heat_shape(nx, ny, nz);
     const bool nt = stream_stores((size_t)nx * ny * nz * sizeof(float));
     const int blocks = (s.nitems + 3) / 4;
@@ -174,25 +133,37 @@ __global__ void zero_f32_kernel(float *p, int n) {
     if (i < n) p[i] = 0.0f;
 }
 
-// Generations per launch of msl_heat7_iterate_f32, in launch order.  Two
-// generations per launch on cubes above kHeatPairMinBytes (MSL_HEAT_GENS =
-// 1 or 2 forces one or two, read on every call so a process can compare
-// both).  A residual generation must be the last of its launch, and the
-// number of launches must have the parity of iters (the result ends in b
-// exactly when iters is odd, as with one launch per generation).
-static std::vector<int> heat_iterate_plan(int nx, int ny, int nz, int iters, int residual_every) {
+// Generations per launch of msl_heat7_iterate_f32, in launch order: the steps
+// up to each residual are dealt evenly to as few launches as heat_way allows
+// (a residual generation is the last of its launch; MSL_HEAT_GENS = 1 or 2
+// forces that many at most, through the one-step or the pair kernel, read on
+// every call so a process can compare both).  The number of launches must have
+// the parity of iters (the result ends in b exactly when iters is odd, as with
+// one launch per generation); when it does not, one launch is split in two.
+static int heat_gens_env() {
     const char *ge = getenv("MSL_HEAT_GENS");
-    const int gens_env = ge ? atoi(ge) : 0;
-    const bool pairs = gens_env == 2 || (gens_env != 1 && (size_t)nx * ny * nz * sizeof(float) > kHeatPairMinBytes);
-    auto is_res = [&](int it) { return residual_every > 0 && ((it + 1) % residual_every == 0); };
+    return ge ? atoi(ge) : 0;
+}
+
+static std::vector<int> heat_iterate_plan(int nx, int ny, int nz, int iters, int residual_every) {
+    const int env = heat_gens_env();
+    const int most = env == 1 || env == 2 ? env : heat_way(nx, ny, nz).gens;
     std::vector<int> plan;
-    for (int it = 0; it < iters; it += plan.back())
-        plan.push_back((pairs && it + 1 < iters && !is_res(it)) ? 2 : 1);
+    for (int it = 0; it < iters;) {
+        int seg = iters - it;
+        if (residual_every > 0) seg = std::min(seg, residual_every - it % residual_every);
+        it += seg;
+        for (int left = (seg + most - 1) / most; left > 0; left--) {
+            plan.push_back((seg + left - 1) / left);
+            seg -= plan.back();
+        }
+    }
     if ((int)(plan.size() & 1) != (iters & 1)) {
         for (size_t j = plan.size(); j-- > 0;)
-            if (plan[j] == 2) {
-                plan[j] = 1;
-                plan.insert(plan.begin() + j + 1, 1);
+            if (plan[j] >= 2) {
+                const int first = plan[j] / 2;
+                plan.insert(plan.begin() + j + 1, plan[j] - first);
+                plan[j] = first;
                 break;
             }
     }
@@ -236,11 +207,10 @@ int msl_heat7_iterate_f32(float *d_a, float *d_b, int nx, int ny, int nz, float 
     MSL_REQUIRE(nres == 0 || h_residuals != nullptr, "msl_heat7_iterate_f32: residual output required");
     if (h_result_in_b) *h_result_in_b = iters & 1;
     if (iters == 0 || nx == 0 || ny == 0 || nz == 0) return MSL_OK;
-    const std::vector<int> plan = heat_iterate_plan(nx, ny, nz, iters, residual_every);
-    const bool pairs = std::find(plan.begin(), plan.end(), 2) != plan.end();
+    const int env = heat_gens_env();
     char keybuf[256];
     snprintf(keybuf, sizeof keybuf, "heat7|%p|%p|%d|%d|%d|%08x|%d|%d|%d", (void *)d_a, (void *)d_b, nx, ny, nz,
-             __builtin_bit_cast(unsigned, nv), iters, residual_every, pairs ? 2 : 1);
+             __builtin_bit_cast(unsigned, nv), iters, residual_every, env);
     std::string key(keybuf);
     HeatGraph hg;
     {
@@ -262,14 +232,21 @@ int msl_heat7_iterate_f32(float *d_a, float *d_b, int nx, int ny, int nz, float 
             brc = check_launch("zero residuals");
         }
         auto is_res = [&](int it) { return residual_every > 0 && ((it + 1) % residual_every == 0); };
+        const std::vector<int> plan = heat_iterate_plan(nx, ny, nz, iters, residual_every);
+        const HeatWay way = heat_way(nx, ny, nz);
         int k = 0, it = 0;
         for (size_t j = 0; j < plan.size() && brc == MSL_OK; j++) {
             float *src = (j & 1) ? d_b : d_a;
             float *dst = (j & 1) ? d_a : d_b;
             it += plan[j];
             const bool res = is_res(it - 1);
-            brc = plan[j] == 2 ? heat_step2(dst, src, nx, ny, nz, nv, res ? d_res + (k++) : nullptr)
-                               : heat_step(dst, src, nx, ny, nz, nv, res ? d_res + (k++) : nullptr);
+            float *maxdiff = res ? d_res + (k++) : nullptr;
+            if (plan[j] == 1)
+                brc = heat_step(dst, src, nx, ny, nz, nv, maxdiff);
+            else if (way.tile && env == 0)
+                brc = heat_tile_step(dst, src, nx, ny, nz, nv, plan[j], way.small, maxdiff);
+            else
+                brc = heat_pair_step(dst, src, nx, ny, nz, nv, maxdiff);
         }
         void *g = nullptr;
         int erc = msl_graph_end(&g);
