@@ -60,7 +60,7 @@ def radius_figures(hip, a, b, r, t_ms):
     n = ROWS * COLS
     plan = hip.mean_iterate_plan(a.ptr, b.ptr, ROWS, COLS, r, BLUR_ITERS)
     gens = max(plan)
-    kname = ("mean3_multi_kernel<6, 16>" if r == 1 and gens > 1 else
+    kname = ("mean3_multi_kernel<6, 8, 8, 2>" if r == 1 and gens > 1 else
              f"strip2_mean_kernel<{r}, 0, true>" if gens == 2 else
              f"strip_stencil_kernel<MeanPolicy<{r}>, 0, true, 4>")
     out = {"kernel": kname, "plan_generations_per_launch": plan, "plan": plan,

@@ -28,6 +28,7 @@ SOURCES = [
     "elementwise.hip",
     "fold.hip",
     "stencil2d.hip",
+    "mean3.hip",
     "gol.hip",
     "blur_tile.hip",
     "stencil3d.hip",

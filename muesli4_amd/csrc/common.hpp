@@ -149,6 +149,39 @@ __device__ __forceinline__ float div_plus0(float x, float d, float rcp) {
     return __fmaf_rn(rc, rcp, q0);
 }
 
+// Correctly rounded x / d by two operations: 1/d = hi + lo with hi rounded
+// down (so lo >= 0), and RN(x * hi + RN(x * lo)) is the quotient as long as the
+// second product keeps its precision (Brisebarre and Muller, "Correctly
+// rounded multiplication by arbitrary precision constants"; for these d the
+// quotient stays at least ulp / 2d away from a rounding boundary).  For x = +0
+// and 2^-93 <= x <= 2^112 only: checked bit-for-bit against IEEE division on
+// all of them by msl_selftest_div_odd_square.
+struct RcpPair {
+    float hi, lo;
+};
+inline RcpPair rcp_pair(double d) {
+    const double q = 1.0 / d;
+    float hi = (float)q;
+    if ((double)hi > q) hi = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, hi) - 1u);
+    return RcpPair{hi, (float)(q - (double)hi)};
+}
+__device__ __forceinline__ float div_pair(float x, RcpPair p) { return __fmaf_rn(x, p.hi, __fmul_rn(x, p.lo)); }
+
+// Collects whether cells are all +0 or in [2^-60, 2^100], so that several
+// generations of means of them stay in the domain of div_pair: a mean of
+// (2r+1)^2 such cells is 0 or at least a (2r+1)^2-th of the smallest.
+struct PairDomain {
+    uint32_t most = 0u, least = ~0u;
+    __device__ __forceinline__ void push(float x) {
+        const uint32_t u = __float_as_uint(x);  // negative cells, -0 and NaN are above every bound
+        most = u > most ? u : most;
+        least = u - 1u < least ? u - 1u : least;  // +0 becomes the largest
+    }
+    __device__ __forceinline__ bool ok() const {
+        return most <= 0x71800000u && least >= 0x21800000u - 1u;  // 2^100, 2^-60
+    }
+};
+
 // Correctly rounded x / 6 (the heat functor's division) by the sequence of
 // div_odd_square with rcp = RN(1/6), plus one case that sequence misses: a
 // quotient exactly halfway between two subnormals (x = (6k+3) * 2^-149, where

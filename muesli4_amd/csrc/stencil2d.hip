@@ -241,6 +241,9 @@ static const MeanLauncher kMean2Launchers[] = {nullptr, nullptr, launch_mean2_r<
                                                launch_mean2_r<7>};
 constexpr int kMaxMean2R = 7;
 
+// Radius 1, up to kMean3Steps generations per launch (mean3.hip).
+int mean3_multi_step(float *out, const float *in, int rows, int cols, float nv, int steps);
+
 int mean_step(float *out, const float *in, int rows, int cols, int r, float nv, int seg) {
     int rc = ensure_ready();
     if (rc) return rc;
@@ -270,87 +273,7 @@ int gol_step(int32_t *out, const int32_t *in, int rows, int cols) {
     return launch_strip(out, in, rows, cols, (int32_t)0, pol, 0, "msl_gol_i32");
 }
 
-// Whole-wave lane shifts with the vacated lane reading 0 (bound_ctrl): no
-// 'old' operand to materialise, so the compiler folds the shift into the
-// add that consumes it (v_add_f32_dpp / v_add_u32_dpp).
-__device__ __forceinline__ int32_t lane_from_left(int32_t v) {  // lane l gets lane l-1 (lane 0: 0)
-    return __builtin_amdgcn_update_dpp(0, v, 0x138, 0xF, 0xF, true);
-}
-__device__ __forceinline__ int32_t lane_from_right(int32_t v) {  // lane l gets lane l+1 (lane 63: 0)
-    return __builtin_amdgcn_update_dpp(0, v, 0x130, 0xF, 0xF, true);
-}
-
-// Mean blur of radius 1, several generations per launch.  A block owns a
-// 64-column x (4 * RPW)-row window of the grid: lane l holds column l, wave w
-// rows [w*RPW, (w+1)*RPW) in registers.  The window edges lack neighbours, so
-// after s generations only cells at least s from every window edge are exact;
-// the block stores the central (64 - 2K) x (4*RPW - 2K) tile, exact after up
-// to K generations.  Row sums
-// ((0 + left) + centre) + right with the side cells by DPP, column sums
-// ((0 + above) + row) + below with the wave edge rows through LDS, then the
-// exact division by 9 -- the operation order of the one-step kernel (the
-// leading "0 +" of both sums folded into div_plus0), so every generation is
-// bit-identical to it.  Cells outside the grid hold nv
-// at every generation.
-template <int K, int RPW>
-__global__ __launch_bounds__(256) void mean3_multi_kernel(float *__restrict__ out, const float *__restrict__ in,
-                                                          int rows, int cols, float nv, int steps, int tiles_x,
-                                                          float denom, float rcp) {
-    constexpr int H = 4 * RPW, TW = 64 - 2 * K, TH = H - 2 * K;
-    __shared__ float edge[4][2][64];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int tx = blockIdx.x % tiles_x, ty = blockIdx.x / tiles_x;
-    const int gx = tx * TW - K + lane;
-    const int gy0 = ty * TH - K + wave * RPW;
-    const bool colok = (unsigned)gx < (unsigned)cols;
-    float c[RPW];
-#pragma unroll
-    for (int i = 0; i < RPW; i++) {
-        const int gy = gy0 + i;
-        c[i] = (colok && (unsigned)gy < (unsigned)rows) ? in[(size_t)gy * cols + gx] : nv;
-    }
-    // row sum of row i of the window (no leading +0: the column sum below
-    // is finished as if it started at +0, which makes a -0 row sum and a
-    // +0 one give the same result)
-    auto rowsum = [&](int i) {
-        const float l = __int_as_float(lane_from_left(__float_as_int(c[i])));
-        const float r = __int_as_float(lane_from_right(__float_as_int(c[i])));
-        return __fadd_rn(__fadd_rn(l, c[i]), r);
-    };
-    for (int s = 0; s < steps; s++) {
-        float rs[RPW + 2];  // row sums of rows gy0-1 .. gy0+RPW
-        // the wave's edge rows first: their sums go to the neighbouring
-        // waves; the inner rows' sums follow the exchange, in the block of
-        // the column sums, where each lane shift folds into its add
-        rs[1] = rowsum(0);
-        rs[RPW] = rowsum(RPW - 1);
-        edge[wave][0][lane] = rs[1];
-        edge[wave][1][lane] = rs[RPW];
-        __syncthreads();
-        rs[0] = wave > 0 ? edge[wave - 1][1][lane] : 0.0f;
-        rs[RPW + 1] = wave < 3 ? edge[wave + 1][0][lane] : 0.0f;
-        __syncthreads();
-#pragma unroll
-        for (int i = 1; i < RPW - 1; i++) rs[i + 1] = rowsum(i);
-#pragma unroll
-        for (int i = 0; i < RPW; i++) {
-            // the column sum without its leading +0, which div_plus0 restores
-            const float t = __fadd_rn(__fadd_rn(rs[i], rs[i + 1]), rs[i + 2]);
-            const int gy = gy0 + i;
-            c[i] = (colok && (unsigned)gy < (unsigned)rows) ? div_plus0(t, denom, rcp) : nv;
-        }
-    }
-    if (lane >= K && lane < 64 - K && colok) {
-#pragma unroll
-        for (int i = 0; i < RPW; i++) {
-            const int wy = wave * RPW + i, gy = gy0 + i;
-            if (wy >= K && wy < H - K && gy < rows) out[(size_t)gy * cols + gx] = c[i];
-        }
-    }
-}
-
-constexpr int kMean3Steps = 6;  // generations per launch of the radius-1 mean blur
-constexpr int kMean3Rows = 16;  // rows per wave: 64 x 64 windows, 52 x 52 tiles
+constexpr int kMean3Steps = 6;  // most generations per launch of the radius-1 kernel and of the tiles
 
 // Launch plan for `iters` generations of at most k per launch, alternating
 // buffers: the result must end in b exactly when iters is odd (as with one
@@ -381,17 +304,6 @@ static bool mean2_default(int r, int rows, int cols) {
     const size_t bytes = (size_t)rows * cols * sizeof(float);
     if (r < 2 || r > kMaxMean2R) return false;
     return r <= 4 ? bytes >= ((size_t)32 << 20) : stream_stores(bytes);
-}
-
-static int mean3_multi_step(float *out, const float *in, int rows, int cols, float nv, int steps) {
-    constexpr int TW = 64 - 2 * kMean3Steps, TH = 4 * kMean3Rows - 2 * kMean3Steps;
-    const int tiles_x = (cols + TW - 1) / TW;
-    const long blocks = (long)tiles_x * ((rows + TH - 1) / TH);
-    MSL_REQUIRE(blocks <= INT32_MAX, "msl_stencil2d_mean_iterate_f32: grid too large");
-    const MeanPolicy<1> pol = MeanPolicy<1>::make();
-    mean3_multi_kernel<kMean3Steps, kMean3Rows><<<(int)blocks, 256, 0, ctx().stream>>>(
-        out, in, rows, cols, nv, steps, tiles_x, pol.denom, pol.rcp);
-    return check_launch("msl_stencil2d_mean_iterate_f32");
 }
 
 // Grids whose iterations run in tiles (several generations per launch in
@@ -466,10 +378,12 @@ __global__ void zero_u64_kernel(unsigned long long *p) { *p = 0ull; }
 // Every 32-bit pattern x: compare div_odd_square(x) (or div6, the heat
 // division, or div_plus0 against (0 + x) / d) with x / d bit for bit (NaN against NaN counts as equal);
 // one atomic per block.
-// kKind 0: div_odd_square, 1: div6, 2: div_plus0, 3: div6_plus0 and 4:
-// div6_fast where div6_suspect passes it, the last three against (0 + x) / d
+// kKind 0: div_odd_square, 1: div6, 2: div_plus0, 3: div6_plus0, 4: div6_fast
+// where div6_suspect passes it and 5: div_pair on its domain, the last four
+// against (0 + x) / d
 template <int kKind>
-__global__ __launch_bounds__(256) void div_check_kernel(float d, float rcp, unsigned long long *count) {
+__global__ __launch_bounds__(256) void div_check_kernel(float d, float rcp, unsigned long long *count,
+                                                         RcpPair pair = RcpPair{}) {
     __shared__ unsigned int part[256];
     unsigned int bad = 0;
     const uint64_t stride = (uint64_t)gridDim.x * 256;
@@ -486,6 +400,8 @@ __global__ __launch_bounds__(256) void div_check_kernel(float d, float rcp, unsi
         } else if constexpr (kKind == 4) {
             got = div6_fast(x);
             if (div6_suspect(got)) got = ref;
+        } else if constexpr (kKind == 5) {
+            got = x == 0.0f || (x >= 0x1p-93f && x <= 0x1p112f) ? div_pair(__fadd_rn(0.0f, x), pair) : ref;
         } else {
             got = div_odd_square(x, d, rcp);
         }
@@ -574,6 +490,7 @@ int msl_selftest_div_odd_square(int r, uint64_t *h_mismatches) {
     const float d = (float)((2 * r + 1) * (2 * r + 1));
     div_check_kernel<0><<<ctx().num_cus * 8, 256, 0, ctx().stream>>>(d, 1.0f / d, d_count);
     div_check_kernel<2><<<ctx().num_cus * 8, 256, 0, ctx().stream>>>(d, 1.0f / d, d_count);
+    div_check_kernel<5><<<ctx().num_cus * 8, 256, 0, ctx().stream>>>(d, 1.0f / d, d_count, rcp_pair(d));
     rc = check_launch("msl_selftest_div_odd_square");
     unsigned long long h = 0;
     hipError_t e = hipMemcpyAsync(&h, d_count, sizeof h, hipMemcpyDeviceToHost, ctx().stream);
