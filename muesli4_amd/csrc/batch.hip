@@ -28,16 +28,21 @@
 // in the wave's LDS and the second generation is formed from them, so each
 // pair of generations reads and writes the grid once), in the launch plan
 // of the single-grid iterations (pairs, with one pair split so that the
-// number of launches keeps the parity of the step count); the other grids
-// run one generation per launch.  Each launch round is a pair kernel over
-// the pair items of that round and a step kernel over its single items.
+// number of launches keeps the parity of the step count); narrow grids (one
+// column per lane) of those radii run in LDS tiles (blur_tile.hpp), a workgroup
+// per tile and as many generations per round as their radius allows; the other
+// grids run one generation per launch.  Each launch round is a pair kernel
+// over the pair items of that round, a tile kernel over its tiles and a step
+// kernel over its single items.
 // Every cell keeps the operation order of one generation per launch, so the
 // states are bit-identical to the plain loop.
 //
 // Fold.  On the last step every lane keeps a TwoSum-compensated sum of the
 // values it stores; a wave combines its lanes in a fixed butterfly and
 // writes one (s, c) pair per item; a final kernel adds a grid's pairs in
-// FP64 in item order.  Deterministic for a given tiling.
+// FP64 in item order, or sums the final state of a grid that ended in tiles
+// (pushing a tile's stores took 1 ms more per round of the 4096-grid batch).
+// Deterministic for a given tiling.
 //
 // Autotuner.  The launch shape (workgroups per CU, static or atomic queue)
 // and the tile shape (C, seg) per width class and then per radius are chosen
@@ -53,6 +58,7 @@
 #include <vector>
 
 #include "blur_item.hpp"
+#include "blur_tile.hpp"
 
 namespace mslhip {
 
@@ -142,13 +148,14 @@ constexpr int kBatchPairMaxR = MSL_BATCH_PAIR_MAX_R;
 constexpr int kPairSeg = 128;  // rows per two-generation item
 constexpr int kPairLdsw = StripConsts<kBatchPairMaxR, 4>::LDSW;
 
-// One item of a launch round: grid g, strip at column xs, rows [y0, y1).
-// flags: kRUp march upwards, kRSrcB read state b (else a), kRFold fold the
-// stored values into partials[part].
+// One item of a launch round: grid g, strip at column xs, rows [y0, y1); or its
+// tile (xs, y0) and y1 generations.  flags: kRUp march upwards, kRSrcB read
+// state b (else a), kRFold fold the stored values into partials[part], kRTile64
+// 64-column tile.
 struct RItem {
     int g, xs, y0, y1, flags, part;
 };
-constexpr int kRUp = 1, kRSrcB = 2, kRFold = 4;
+constexpr int kRUp = 1, kRSrcB = 2, kRFold = 4, kRTile64 = 8;
 
 template <int R, bool kFold>
 __device__ __forceinline__ void pair_item(const float *src, float *dst, const BGrid &g, int xs, int y0, int y1,
@@ -216,24 +223,104 @@ __global__ __launch_bounds__(256) void batch_round_kernel(const BGrid *__restric
     }
 }
 
-// One wave per grid: FP64 sum of the (s, c) pairs of its last round's items
-// (fold[g] = {first partial, count}), in item order.
-__global__ __launch_bounds__(256) void batch_round_final_kernel(const int2 *__restrict__ fold, int ngrids,
+// Tiles of narrow grids.  128-column tiles (64-column ones where they cover
+// the grid with fewer lanes), as many generations per round as leave about
+// half of a tile.  10 steps of the 2621 grids narrower than 192 columns in the
+// 4096-grid batch: 0.82 ms, 2.0 in one-generation strips.  (Wide grids in tiles
+// take 470 us per generation, in two-generation strips 435.)
+constexpr int kTileGens[kBatchPairMaxR + 1] = {0, 6, 4, 4, 3, 3, 2, 2, 2};
+constexpr int kTileThreads = 512;    // W = 128, M = 4 or W = 64, M = 2
+constexpr int kTileBlocksPerCu = 3;  // 44 KB of LDS each
+constexpr size_t kTileLds = blur_tile_lds(kBatchPairMaxR, 128, kTileRows, 1);
+
+// Output columns and rows of a tile of w columns and gens generations.
+__host__ __device__ inline int tile_cols(int r, int w, int gens) { return (w - 2 * r * gens) / 4 * 4; }
+__host__ __device__ inline int tile_rows(int r, int gens) {
+    const int h = (kTileRows - 2 * r * (gens - 1)) / 8 * 8;
+    return h < 48 ? h : 48;
+}
+
+template <int W, int M, int R = 1>
+__device__ __forceinline__ void tile_item(const BGrid &g, const float *src, float *dst, const RItem &it, float *lds) {
+    if constexpr (R < kBatchPairMaxR) {
+        if (g.r != R) return tile_item<W, M, R + 1>(g, src, dst, it, lds);
+    }
+    blur_tile<R, W, M>(dst, src, g.rows, g.cols, g.nv, it.y1, tile_cols(R, W, it.y1), tile_rows(R, it.y1), it.xs,
+                       it.y0, lds);
+}
+
+// The tiles (xs, y0) of y1 generations of a round, a workgroup each; the next
+// one from the round's counter.  Bound by VALU issue.
+__global__ __launch_bounds__(kTileThreads) void batch_tile_kernel(const BGrid *__restrict__ grids,
+                                                                  const RItem *__restrict__ items, int nitems,
+                                                                  unsigned *__restrict__ ctr) {
+    extern __shared__ __attribute__((aligned(16))) float lds[];
+    __shared__ int next;
+    for (int i = (int)xcd_tile(blockIdx.x, gridDim.x); i < nitems;) {
+        const RItem it = items[i];
+        const BGrid g = grids[it.g];
+        const float *src = (it.flags & kRSrcB) ? g.b : g.a;
+        float *dst = (it.flags & kRSrcB) ? g.a : g.b;
+        if (it.flags & kRTile64)
+            tile_item<64, 2>(g, src, dst, it, lds);
+        else
+            tile_item<128, 4>(g, src, dst, it, lds);
+        if (threadIdx.x == 0) next = (int)(gridDim.x + atomicAdd(ctr, 1u));
+        __syncthreads();  // also: the tile's last reads of lds are done
+        i = __builtin_amdgcn_readfirstlane(next);
+        __syncthreads();
+    }
+}
+
+// One workgroup per grid.  FP64 sum of the (s, c) pairs of its last round's
+// items (fold[g] = {first partial, count}), in item order; a grid that ended
+// in tiles (count -1 - result buffer) is summed here from its final state:
+// each lane's quads in order, four loads in flight, the lanes' pairs in a fixed
+// butterfly and the waves' in FP64.
+__global__ __launch_bounds__(256) void batch_round_final_kernel(const BGrid *__restrict__ grids,
+                                                                const int2 *__restrict__ fold,
                                                                 const float2 *__restrict__ partials,
                                                                 double *__restrict__ sums) {
-    const int lane = threadIdx.x & 63;
-    const int gi = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (gi >= ngrids) return;
+    __shared__ double waves[4];
+    const int lane = threadIdx.x & 63, gi = blockIdx.x;
     const int2 f = fold[gi];
     double acc = 0.0;
-    for (int k = lane; k < f.y; k += 64) {
-        const float2 p = partials[f.x + k];
-        acc += (double)p.x;
-        acc += (double)p.y;
-    }
+    if (f.y >= 0) {
+        if (threadIdx.x >= 64) return;
+        for (int k = lane; k < f.y; k += 64) {
+            const float2 p = partials[f.x + k];
+            acc += (double)p.x;
+            acc += (double)p.y;
+        }
 #pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) acc += __shfl_xor(acc, m);
-    if (lane == 0) sums[gi] = acc;
+        for (int m = 32; m >= 1; m >>= 1) acc += __shfl_xor(acc, m);
+        if (lane == 0) sums[gi] = acc;
+        return;
+    }
+    const BGrid g = grids[gi];
+    const float *data = f.y == -2 ? g.b : g.a;
+    const int n = g.rows * g.cols, nq = n / 4;
+    LaneSum ls;
+    int t = threadIdx.x;
+    for (; t + 768 < nq; t += 1024) {
+        VecN<float, 4> v[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) v[u] = load_dword_aligned<float, 4>(data + 4 * (t + 256 * u));
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+#pragma unroll
+            for (int k = 0; k < 4; k++) ls.push(v[u].v[k]);
+    }
+    for (; t < nq; t += 256) {
+        const VecN<float, 4> v = load_dword_aligned<float, 4>(data + 4 * t);
+#pragma unroll
+        for (int k = 0; k < 4; k++) ls.push(v.v[k]);
+    }
+    if (4 * nq + (int)threadIdx.x < n) ls.push(data[4 * nq + threadIdx.x]);
+    wave_pair_reduce(ls);
+    if (lane == 0) waves[threadIdx.x >> 6] = (double)ls.s + (double)ls.c;
+    __syncthreads();
+    if (threadIdx.x == 0) sums[gi] = ((waves[0] + waves[1]) + waves[2]) + waves[3];
 }
 
 // One wave per grid: sum = sum over the grid's items, in item order, of
@@ -618,8 +705,22 @@ static std::vector<int> pair_plan(int iters) {
     return plan;
 }
 
+// Generations per round of a grid in tiles: dealt evenly to as few rounds as
+// `most` per round allows, one more where their number would not have the
+// parity of iters.
+static std::vector<int> tile_plan(int iters, int most) {
+    std::vector<int> plan;
+    int rounds = (iters + most - 1) / most;
+    if ((rounds ^ iters) & 1) rounds++;
+    for (; rounds > 0; rounds--) {
+        plan.push_back((iters + rounds - 1) / rounds);
+        iters -= plan.back();
+    }
+    return plan;
+}
+
 struct RoundRange {
-    int pair_off, pair_n, single_off, single_n;
+    int off[3], n[3];  // pair items, tiles, single items
 };
 
 // The launch rounds of msl_batch_run: per round the pair items and the
@@ -639,13 +740,15 @@ static void plan_rounds(const Batch &b, int iters, bool fold, RoundPlan &rp) {
     const int ng = (int)b.grids.size();
     std::vector<std::vector<int>> plan(ng);
     std::vector<int> kind(ng, kKindNarrow1), order;
+    std::vector<char> tiles(ng, 0);
     for (int g = 0; g < ng; g++) {
         const msl_batch_grid &G = b.grids[g];
         if (G.rows == 0 || G.cols == 0) continue;
         kind[g] = grid_kind(G, b.table[G.r][width_class(G.cols)].c);
-        const bool pair = b.pairs && G.r <= kBatchPairMaxR && kind[g] != kKindNarrow1;
-        plan[g] = pair ? pair_plan(iters) : std::vector<int>(iters, 1);
-        rp.pair_grids += pair ? 1 : 0;
+        const bool multi = b.pairs && G.r <= kBatchPairMaxR;
+        tiles[g] = multi && kind[g] == kKindNarrow1;
+        plan[g] = tiles[g] ? tile_plan(iters, kTileGens[G.r]) : multi ? pair_plan(iters) : std::vector<int>(iters, 1);
+        rp.pair_grids += multi ? 1 : 0;
         order.push_back(g);
     }
     // largest radius first: the costliest items start first and the cheap
@@ -665,42 +768,50 @@ static void plan_rounds(const Batch &b, int iters, bool fold, RoundPlan &rp) {
     std::vector<RoundRange> &rounds = rp.rounds;
     for (size_t j = 0; j < nrounds; j++) {
         RoundRange rr{};
-        for (int pass = 0; pass < 2; pass++) {  // pass 0: pair items, 1: single items
-            const int off = (int)items.size();
+        for (int pass = 0; pass < 3; pass++) {  // pair items, tiles, single items
+            rr.off[pass] = (int)items.size();
             for (int g : order) {
-                if (j >= plan[g].size() || (plan[g][j] == 2) != (pass == 0)) continue;
+                if (j >= plan[g].size()) continue;
+                const int gens = plan[g][j];
+                if ((gens == 1 ? 2 : tiles[g]) != pass) continue;
                 const msl_batch_grid &G = b.grids[g];
                 const bool last = fold && j + 1 == plan[g].size();
-                int sw, seg;
+                int sw, seg, flags = (j & 1) ? kRSrcB : 0;
                 if (pass == 0) {
                     const int halo = (G.r + 3) / 4 * 4;
                     sw = 256 - 2 * halo;
                     seg = b.pair_seg;
+                } else if (pass == 1) {
+                    auto lanes = [&](int w) {
+                        const int c = tile_cols(G.r, w, gens);
+                        return c < 16 ? INT32_MAX : (G.cols + c - 1) / c * w;
+                    };
+                    const int w = lanes(64) < lanes(128) ? 64 : 128;
+                    if (w == 64) flags |= kRTile64;
+                    sw = tile_cols(G.r, w, gens);
+                    seg = tile_rows(G.r, gens);
                 } else {
                     const Tile t = b.table[G.r][width_class(G.cols)];
                     sw = 64 * (kind[g] == kKindNarrow1 ? 1 : 4);
                     seg = std::max(1, t.seg);
                 }
-                if (last) hfold[g] = make_int2(nparts, 0);
+                if (last) hfold[g] = pass == 1 ? make_int2(0, (iters & 1) ? -2 : -1) : make_int2(nparts, 0);
                 for (int xs = 0; xs < G.cols; xs += sw)
                     for (int y0 = 0; y0 < G.rows; y0 += seg) {
-                        int flags = ((j & 1) ? kRSrcB : 0) | (((y0 / seg) & 1) ? kRUp : 0);
+                        if (pass == 1) {
+                            items.push_back(RItem{g, xs / sw, y0 / seg, gens, flags, 0});
+                            continue;
+                        }
                         int part = 0;
                         if (last) {
-                            flags |= kRFold;
                             part = nparts++;
                             hfold[g].y++;
                         }
-                        items.push_back(RItem{g, xs, y0, std::min(y0 + seg, G.rows), flags, part});
+                        items.push_back(RItem{g, xs, y0, std::min(y0 + seg, G.rows),
+                                              flags | (((y0 / seg) & 1) ? kRUp : 0) | (last ? kRFold : 0), part});
                     }
             }
-            if (pass == 0) {
-                rr.pair_off = off;
-                rr.pair_n = (int)items.size() - off;
-            } else {
-                rr.single_off = off;
-                rr.single_n = (int)items.size() - off;
-            }
+            rr.n[pass] = (int)items.size() - rr.off[pass];
         }
         rounds.push_back(rr);
     }
@@ -718,7 +829,7 @@ static int build_rounds(Batch &b, int iters, bool fold, RunGraph &rg, std::vecto
     MSL_HIP_TRY(hipMalloc(&rg.d_items, sizeof(RItem) * std::max<size_t>(items.size(), 1)));
     MSL_HIP_TRY(hipMalloc(&rg.d_fold, sizeof(int2) * hfold.size()));
     MSL_HIP_TRY(hipMalloc(&rg.d_partials, sizeof(float2) * std::max(nparts, 1)));
-    MSL_HIP_TRY(hipMalloc(&rg.d_ctr, sizeof(unsigned) * std::max<size_t>(2 * nrounds, 1)));
+    MSL_HIP_TRY(hipMalloc(&rg.d_ctr, sizeof(unsigned) * std::max<size_t>(3 * nrounds, 1)));
     if (!items.empty())
         MSL_HIP_TRY(hipMemcpyAsync(rg.d_items, items.data(), sizeof(RItem) * items.size(), hipMemcpyHostToDevice,
                                    ctx().stream));
@@ -732,7 +843,7 @@ static int build_rounds(Batch &b, int iters, bool fold, RunGraph &rg, std::vecto
 // and the per-grid fold combine.
 static int enqueue_rounds(Batch &b, const std::vector<RoundRange> &rounds, double *d_sums, const RunGraph &rg) {
     hipStream_t s = ctx().stream;
-    const int nc = (int)(2 * rounds.size());
+    const int nc = (int)(3 * rounds.size());
     if (nc > 0) {
         batch_zero_kernel<<<(nc + 255) / 256, 256, 0, s>>>(rg.d_ctr, nc);
         int rc = check_launch("msl_batch_run");
@@ -741,23 +852,26 @@ static int enqueue_rounds(Batch &b, const std::vector<RoundRange> &rounds, doubl
     const int cus = ctx().num_cus;
     for (size_t j = 0; j < rounds.size(); j++) {
         const RoundRange &rr = rounds[j];
-        if (rr.pair_n) {
-            const int blocks = std::max(1, std::min((rr.pair_n + 3) / 4, cus * b.max_pair_blocks_per_cu));
-            batch_round_kernel<true><<<blocks, 256, 0, s>>>(b.d_grids, rg.d_items + rr.pair_off, rr.pair_n,
-                                                            rg.d_partials, rg.d_ctr + 2 * j);
+        if (rr.n[0]) {
+            const int blocks = std::max(1, std::min((rr.n[0] + 3) / 4, cus * b.max_pair_blocks_per_cu));
+            batch_round_kernel<true><<<blocks, 256, 0, s>>>(b.d_grids, rg.d_items + rr.off[0], rr.n[0], rg.d_partials,
+                                                            rg.d_ctr + 3 * j);
         }
-        if (rr.single_n) {
+        if (rr.n[1])
+            batch_tile_kernel<<<std::min(rr.n[1], cus * kTileBlocksPerCu), kTileThreads, kTileLds, s>>>(
+                b.d_grids, rg.d_items + rr.off[1], rr.n[1], rg.d_ctr + 3 * j + 1);
+        if (rr.n[2]) {
             const int bpc = std::max(1, std::min(b.blocks_per_cu, b.max_blocks_per_cu));
-            const int blocks = std::max(1, std::min((rr.single_n + 3) / 4, cus * bpc));
-            batch_round_kernel<false><<<blocks, 256, 0, s>>>(b.d_grids, rg.d_items + rr.single_off, rr.single_n,
-                                                             rg.d_partials, rg.d_ctr + 2 * j + 1);
+            const int blocks = std::max(1, std::min((rr.n[2] + 3) / 4, cus * bpc));
+            batch_round_kernel<false><<<blocks, 256, 0, s>>>(b.d_grids, rg.d_items + rr.off[2], rr.n[2], rg.d_partials,
+                                                             rg.d_ctr + 3 * j + 2);
         }
         int rc = check_launch("msl_batch_run");
         if (rc) return rc;
     }
     if (d_sums) {
         const int ng = (int)b.grids.size();
-        batch_round_final_kernel<<<(ng + 3) / 4, 256, 0, s>>>(rg.d_fold, ng, rg.d_partials, d_sums);
+        batch_round_final_kernel<<<ng, 256, 0, s>>>(b.d_grids, rg.d_fold, rg.d_partials, d_sums);
         return check_launch("msl_batch_run");
     }
     return MSL_OK;
@@ -913,7 +1027,7 @@ int msl_batch_run_plan(const void *batch, int iters, int with_fold, int *h_round
     RoundPlan rp;
     plan_rounds(*b, iters, with_fold != 0, rp);
     int launches = rp.rounds.empty() ? 0 : 1;  // counter clear
-    for (const RoundRange &rr : rp.rounds) launches += (rr.pair_n > 0) + (rr.single_n > 0);
+    for (const RoundRange &rr : rp.rounds) for (int n : rr.n) launches += n > 0;
     if (with_fold && iters > 0) launches++;
     if (h_rounds) *h_rounds = (int)rp.rounds.size();
     if (h_launches) *h_launches = launches;

@@ -40,30 +40,49 @@ __device__ __forceinline__ void blur_tile(float *__restrict__ out, const float *
     int x0 = ox - R * steps, y0 = oy - R * steps;       // grid cell of LDS (0, 0)
     const bool inside = x0 >= 0 && x0 + W <= cols && y0 >= 0 && y0 + h <= rows;
 
-    {
-        const int c0 = x0 + 4 * q;
+    // The tile's cells, all loads at once.  Tiles over the grid's edge are
+    // filled with nv first, and each quad that overlaps the grid is loaded and
+    // stored shifted to lie in it (overlapping quads store equal values):
+    // cheaper than selecting per cell, and most tiles of small grids are such.
+    if (inside || cols >= 4) {
+        const int c0 = x0 + 4 * q, cc = min(max(c0, 0), cols - 4);
         VecN<float, 4> v[ROUNDS];
 #pragma unroll
         for (int i = 0; i < ROUNDS; i++) {
-            const int y = y0 + min(rr + RPR * i, h - 1);
-            if (inside) {
-                v[i] = load_dword_aligned<float, 4>(in + (size_t)y * cols + c0);
-            } else {
-                const float *row = in + (size_t)min(max(y, 0), rows - 1) * cols;
+            const int y = min(max(y0 + min(rr + RPR * i, h - 1), 0), rows - 1);
+            v[i] = load_dword_aligned<float, 4>(in + (size_t)y * cols + cc);
+        }
+        if (inside) {
 #pragma unroll
-                for (int k = 0; k < 4; k++) v[i].v[k] = row[min(max(c0 + k, 0), cols - 1)];
+            for (int i = 0; i < ROUNDS; i++)
+                if (rr + RPR * i < h)
+                    *reinterpret_cast<V *>(lds + (rr + RPR * i) * W + 4 * q) = to_native<float, 4>(v[i]);
+        } else {
+            for (int row = rr; row < h; row += RPR) *reinterpret_cast<V *>(lds + row * W + 4 * q) = V{nv, nv, nv, nv};
+            __syncthreads();
+            const int p = cc - x0;
+            if (c0 < cols && c0 + 4 > 0) {
+#pragma unroll
+                for (int i = 0; i < ROUNDS; i++) {
+                    const int row = rr + RPR * i;
+                    if (row < h && (unsigned)(y0 + row) < (unsigned)rows) {
+#pragma unroll
+                        for (int k = 0; k < 4; k++)
+                            if (p + k >= 0) lds[row * W + p + k] = v[i].v[k];
+                    }
+                }
             }
         }
+    } else {
+        const int c0 = x0 + 4 * q;
+        for (int row = rr; row < h; row += RPR) {
+            const bool rowok = (unsigned)(y0 + row) < (unsigned)rows;
+            const float *src = in + (size_t)min(max(y0 + row, 0), rows - 1) * cols;
 #pragma unroll
-        for (int i = 0; i < ROUNDS; i++) {
-            const int row = rr + RPR * i;
-            if (!inside) {
-                const bool rowok = (unsigned)(y0 + row) < (unsigned)rows;
-#pragma unroll
-                for (int k = 0; k < 4; k++)
-                    v[i].v[k] = rowok && (unsigned)(c0 + k) < (unsigned)cols ? v[i].v[k] : nv;
+            for (int k = 0; k < 4; k++) {
+                const float f = src[min(max(c0 + k, 0), cols - 1)];
+                lds[row * W + 4 * q + k] = rowok && (unsigned)(c0 + k) < (unsigned)cols ? f : nv;
             }
-            if (row < h) *reinterpret_cast<V *>(lds + row * W + 4 * q) = to_native<float, 4>(v[i]);
         }
     }
     __syncthreads();

@@ -167,7 +167,7 @@ inline RcpPair rcp_pair(double d) {
 }
 __device__ __forceinline__ float div_pair(float x, RcpPair p) { return __fmaf_rn(x, p.hi, __fmul_rn(x, p.lo)); }
 
-// Collects whether cells are all +0 or in [2^-60, 2^100], so that several
+// Collects whether cells are all +0 or in [2^-40, 2^100], so that several
 // generations of means of them stay in the domain of div_pair: a mean of
 // (2r+1)^2 such cells is 0 or at least a (2r+1)^2-th of the smallest.
 struct PairDomain {
@@ -178,7 +178,7 @@ struct PairDomain {
         least = u - 1u < least ? u - 1u : least;  // +0 becomes the largest
     }
     __device__ __forceinline__ bool ok() const {
-        return most <= 0x71800000u && least >= 0x21800000u - 1u;  // 2^100, 2^-60
+        return most <= 0x71800000u && least >= 0x2B800000u - 1u;  // 2^100, 2^-40
     }
 };
 

@@ -294,27 +294,40 @@ static std::vector<int> generation_plan(int iters, int k) {
     return plan;
 }
 
+// The same parity with the generations dealt evenly to as few launches as at
+// most k each allow (LDS tiles: a launch's cost grows with its generations).
+static std::vector<int> even_plan(int iters, int k) {
+    std::vector<int> plan;
+    int launches = (iters + k - 1) / k;
+    if ((launches ^ iters) & 1) launches++;
+    for (; launches > 0; launches--) {
+        plan.push_back((iters + launches - 1) / launches);
+        iters -= plan.back();
+    }
+    return plan;
+}
+
 // Whether iterations of radius r run two generations per launch by default.
-// Measured (GB/s, one vs two generations per launch): radii 2-4 gain from
-// 4096^2 on (r = 2: 5.7 -> 9.0 TB/s), radii 5-7 only on grids streamed from
-// HBM (8192^2: r = 5 4.7 -> 7.2, r = 7 4.5 -> 6.1); on grids that stay in
-// the Infinity Cache their longer halo recomputation costs more than the
-// saved traffic (5792^2: r = 5 5.2 -> 4.6).
+// Measured (GB/s, one vs two generations per launch): radius 4 gains from
+// 4096^2 on, radii 5-7 only on grids streamed from HBM (8192^2: r = 5 4.7 ->
+// 7.2, r = 7 4.5 -> 6.1); on grids that stay in the Infinity Cache their longer
+// halo recomputation costs more than the saved traffic (5792^2: r = 5 5.2 ->
+// 4.6).
 static bool mean2_default(int r, int rows, int cols) {
     const size_t bytes = (size_t)rows * cols * sizeof(float);
-    if (r < 2 || r > kMaxMean2R) return false;
+    if (r < 4 || r > kMaxMean2R) return false;
     return r <= 4 ? bytes >= ((size_t)32 << 20) : stream_stores(bytes);
 }
 
 // Grids whose iterations run in tiles (several generations per launch in
-// LDS): radius 2 and above up to these many cells, unless the two-generation
-// march takes them (mean2_default).  us per generation of the best tile and
-// of the march: 4096^2 r = 5 20.4 / 26.4, 6 21.6 / 26.0, 8 28.0 / 28.3;
-// 3000^2 r = 8 16.9 / 20.3, 9 20.6 / 22.5, 10 23.8 / 22.2; 2048^2 r = 10
-// 13.0 / 17.7; 500 x 517 r = 3 2.1 / 4.9.
+// LDS): radii 2 and 3 always, 4 to 8 up to 2^24 cells, above up to 2^22.2.
+// us per generation of the best tile and of the march: 8192^2 r = 2 42.7 / 59.0,
+// 3 57.8 / 60.3, 4 63.9 / 60.9, 5 79.9 / 63.2; 4096^2 r = 4 17.0 / 19.3, 5 20.4
+// / 26.4, 6 21.6 / 26.0, 8 28.0 / 28.3; 3000^2 r = 8 16.9 / 20.3, 9 20.6 / 22.5,
+// 10 23.8 / 22.2; 2048^2 r = 10 13.0 / 17.7; 500 x 517 r = 3 2.1 / 4.9.
 static bool tile_default(int r, int rows, int cols) {
     const long cells = (long)rows * cols;
-    return r >= 2 && !mean2_default(r, rows, cols) && cells <= (r <= 8 ? 1L << 24 : 9L << 19);
+    return r >= 2 && (r <= 3 || cells <= (r <= 8 ? 1L << 24 : 9L << 19));
 }
 
 enum LaunchKind { kLaunchStep, kLaunchMulti3, kLaunchPair, kLaunchTile };
@@ -326,10 +339,10 @@ struct MeanLaunch {
 };
 
 // The launches of msl_stencil2d_mean_iterate_f32, in order: the
-// six-generation register-window kernel at r = 1, the two-generation march at
-// r = 2 .. kMaxMean2R on large grids with rows of 4 or more cells, tiles with
-// the number of generations that the model prices lowest on smaller ones,
-// else the one-step kernel.  MSL_MEAN_GENS = 1 or 2 forces one or two
+// six-generation register-window kernel at r = 1, tiles with the number of
+// generations that the model prices lowest (tile_default), the two-generation
+// march up to kMaxMean2R on larger grids with rows of 4 or more cells, else the
+// one-step kernel.  MSL_MEAN_GENS = 1 or 2 forces one or two
 // generations per launch for r >= 2 (read on every call, so a process can
 // compare both).
 static int mean_gens_env() {
@@ -346,17 +359,18 @@ static std::vector<MeanLaunch> mean_iterate_plan(const float *d_a, const float *
     };
     if (r == 1) return launches(generation_plan(iters, kMean3Steps), kLaunchMulti3);
     const int gens_env = mean_gens_env();
-    const bool pairs = r <= kMaxMean2R && row_mode(d_a, d_b, cols) != kScalar &&
+    const bool tiles = gens_env == 0 && iters > 1 && tile_default(r, rows, cols);
+    const bool pairs = !tiles && r <= kMaxMean2R && row_mode(d_a, d_b, cols) != kScalar &&
                        (gens_env == 2 || (gens_env != 1 && mean2_default(r, rows, cols)));
     if (pairs) return launches(generation_plan(iters, 2), kLaunchPair);
-    if (gens_env == 0 && iters > 1 && tile_default(r, rows, cols)) {
+    if (tiles) {
         TileShape shape[kMean3Steps + 1];
         std::vector<int> best;
         double best_us = 1e30;
         for (int k = 1; k <= kMean3Steps; k++) {
             shape[k] = tile_shape(rows, cols, r, k);
             if (shape[k].w == 0) break;
-            const std::vector<int> gens = generation_plan(iters, k);
+            const std::vector<int> gens = even_plan(iters, k);
             double us = 0.0;
             for (int g : gens) us += shape[g].us;
             if (us < best_us) {
