@@ -15,7 +15,8 @@
  *  - Pointers named d_* are device pointers (from msl_malloc or any HIP
  *    allocation on the current device); h_* are host pointers.
  *  - All launches are stream-ordered on the library stream (msl_stream()).
- *    Entry points that return a value to the host synchronise that stream.
+ *    Entry points that return a value to the host wait until it is there
+ *    (all earlier work of that stream is done by then).
  *  - x = column, y = row, z = depth.  DM layout row*cols+col, DC layout
  *    (z*rows+y)*cols+x (reference include/nplmatrix.h:141-143,
  *    include/plcube.h:121-123).

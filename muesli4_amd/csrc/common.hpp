@@ -47,6 +47,12 @@ int check_launch(const char *what);
 
 // Scratch workspace owned by the context (grown outside graph capture only).
 int workspace(size_t bytes, void **ptr);
+// Results that a kernel posts to the host itself.  host_post_slot gives a
+// 16-byte entry of pinned memory and a sequence number for one launch, whose
+// last thread calls post_result; host_post_wait returns the posted 64 bits.
+int host_post_slot(void **slot, uint32_t *seq);
+int host_post_wait(const void *slot, uint32_t seq, uint64_t *bits, const char *name);
+
 // Looks up, with `device` current, the device address of the fixed scratch
 // array of the allocation-free fold (fold.hip); called once per device by
 // msl_init.
@@ -87,6 +93,18 @@ __host__ __device__ inline uint64_t hash64(uint64_t seed, uint64_t idx) {
     z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ULL;
     z = (z ^ (z >> 27)) * 0x94D049BB133111EBULL;
     return z ^ (z >> 31);
+}
+
+// One 16-byte store of the value, its sequence number and a check word over
+// both: the host takes the entry only when the three agree, so the order in
+// which its bytes arrive does not matter.
+__host__ __device__ inline uint32_t post_check(uint64_t bits, uint32_t seq) {
+    return ((uint32_t)bits * 0x9E3779B1u) ^ ((uint32_t)(bits >> 32) * 0x85EBCA77u) ^ (seq * 0xC2B2AE3Du) ^ 0x27D4EB2Fu;
+}
+__device__ __forceinline__ void post_result(void *slot, uint32_t seq, uint64_t bits) {
+    typedef uint32_t post_t __attribute__((ext_vector_type(4)));
+    const post_t v = {(uint32_t)bits, (uint32_t)(bits >> 32), seq, post_check(bits, seq)};
+    __builtin_nontemporal_store(v, static_cast<post_t *>(slot));
 }
 
 // IEEE single operations that the compiler may not contract into an FMA.

@@ -14,6 +14,8 @@
 // accumulated in c); partial pairs are merged with TwoSum as well.  The final
 // combine converts each (s, c) to FP64 and adds them in block order - the
 // only FP64 arithmetic in the fold.
+#include <cstring>
+
 #include "common.hpp"
 
 namespace mslhip {
@@ -148,13 +150,27 @@ __global__ __launch_bounds__(kFoldThreads) void fold_kernel(const typename P::In
     if (threadIdx.x == 0) partials[blockIdx.x] = r;
 }
 
+// The fold's value to *result (device memory), or posted to the host when seq
+// is not 0.
+template <typename T>
+__device__ __forceinline__ void put_result(void *result, uint32_t seq, T value) {
+    if (seq) {
+        uint64_t bits = 0;
+        __builtin_memcpy(&bits, &value, sizeof(value));
+        post_result(result, seq, bits);
+    } else {
+        *reinterpret_cast<T *>(result) = value;
+    }
+}
+
 // Final combine (second launch, one block): partials in block order.  A
 // second launch is used instead of a last-block-done counter because the
 // agent-scope release fence that counter needs writes back the whole L2 of
 // each XCD and costs more than the extra launch.
 template <typename P, bool kF64Final>
 __global__ __launch_bounds__(kFoldThreads) void fold_final_kernel(const typename P::Part *__restrict__ partials,
-                                                                  int nparts, void *__restrict__ result) {
+                                                                  int nparts, void *__restrict__ result,
+                                                                  uint32_t seq) {
     if constexpr (kF64Final) {
         // Compensated sum: FP64 combine of the (s, c) partials, the only FP64
         // arithmetic of the fold (thread t takes partials t, t+256, ...).
@@ -172,13 +188,13 @@ __global__ __launch_bounds__(kFoldThreads) void fold_final_kernel(const typename
         if (threadIdx.x == 0) {
             double t = lds[0];
             for (int w = 1; w < kFoldWaves; w++) t += lds[w];
-            *reinterpret_cast<double *>(result) = t;
+            put_result(result, seq, t);
         }
     } else {
         typename P::Part a = P::init();
         for (int k = threadIdx.x; k < nparts; k += kFoldThreads) a = P::combine(a, partials[k]);
         const typename P::Part t = block_reduce<P>(a);
-        if (threadIdx.x == 0) *reinterpret_cast<typename P::Part *>(result) = t;
+        if (threadIdx.x == 0) put_result(result, seq, t);
     }
 }
 
@@ -187,16 +203,16 @@ __global__ __launch_bounds__(kFoldThreads) void fold_final_kernel(const typename
 // that fold_kernel would have had, group g those of blocks g, g + 4, ..., and
 // combines them in the order of fold_kernel and fold_final_kernel, so the
 // result is bit-identical to theirs.  Bound by launch and load latency: the
-// whole call (result on the host) takes 13.9 us at 10007 floats and 15.9 at
-// 40960, two launches 16.3 at any size up to 2^20 (the compensated sum; the
-// line lies where it meets them, the integer sum and max would gain to 16
-// partials).  With a third launch that copied the scalar it was 18.1.
+// whole call (result on the host) takes 8.7 us at 10007 floats and 10.4 at
+// 40960, two launches 11.4 at any size up to 2^20 (the compensated sum; the
+// line lies just below where it meets them).  With a third launch that copied
+// the scalar and a wait for the stream it was 17.3.
 constexpr int kSmallParts = 10;
 constexpr int kSmallThreads = 4 * kFoldThreads;
 
 template <typename P, bool kF64Final>
 __global__ __launch_bounds__(kSmallThreads) void fold_small_kernel(const typename P::In *__restrict__ in, size_t n,
-                                                                   int nparts, void *__restrict__ result,
+                                                                   int nparts, void *__restrict__ result, uint32_t seq,
                                                                    int vec_ok) {
     using Part = typename P::Part;
     __shared__ Part lds[kSmallParts][kFoldWaves];
@@ -220,10 +236,10 @@ __global__ __launch_bounds__(kSmallThreads) void fold_small_kernel(const typenam
         d += (double)p.c;
 #pragma unroll
         for (int m = 32; m >= 1; m >>= 1) d += __shfl_xor(d, m);
-        if (threadIdx.x == 0) *reinterpret_cast<double *>(result) = d;
+        if (threadIdx.x == 0) put_result(result, seq, d);
     } else {
         p = wave_reduce<P>(P::combine(P::init(), p));
-        if (threadIdx.x == 0) *reinterpret_cast<Part *>(result) = p;
+        if (threadIdx.x == 0) put_result(result, seq, p);
     }
 }
 
@@ -243,21 +259,21 @@ inline int fold_blocks(size_t n) {
 // fold_blocks(n)) is only used when the array takes two launches.
 template <typename P, bool kF64Final>
 int launch_fold(const typename P::In *in, size_t n, int blocks, typename P::Part *partials, void *result,
-                const char *name) {
+                uint32_t seq, const char *name) {
     const int vec_ok = (((uintptr_t)in) & 15u) == 0;
     if (blocks <= kSmallParts) {
-        fold_small_kernel<P, kF64Final><<<1, kSmallThreads, 0, ctx().stream>>>(in, n, blocks, result, vec_ok);
+        fold_small_kernel<P, kF64Final><<<1, kSmallThreads, 0, ctx().stream>>>(in, n, blocks, result, seq, vec_ok);
         return check_launch(name);
     }
     fold_kernel<P><<<blocks, kFoldThreads, 0, ctx().stream>>>(in, n, partials, vec_ok);
     int rc = check_launch(name);
     if (rc) return rc;
-    fold_final_kernel<P, kF64Final><<<1, kFoldThreads, 0, ctx().stream>>>(partials, blocks, result);
+    fold_final_kernel<P, kF64Final><<<1, kFoldThreads, 0, ctx().stream>>>(partials, blocks, result, seq);
     return check_launch(name);
 }
 
 template <typename P, bool kF64Final>
-int run_fold(const typename P::In *in, size_t n, void *d_result, const char *name) {
+int run_fold(const typename P::In *in, size_t n, void *result, uint32_t seq, const char *name) {
     int rc = ensure_ready();
     if (rc) return rc;
     MSL_REQUIRE(in != nullptr || n == 0, std::string(name) + ": null input");
@@ -267,20 +283,23 @@ int run_fold(const typename P::In *in, size_t n, void *d_result, const char *nam
         rc = workspace((size_t)blocks * sizeof(typename P::Part), &ws);
         if (rc) return rc;
     }
-    return launch_fold<P, kF64Final>(in, n, blocks, static_cast<typename P::Part *>(ws), d_result, name);
+    return launch_fold<P, kF64Final>(in, n, blocks, static_cast<typename P::Part *>(ws), result, seq, name);
 }
 
-// Folds into the pinned result slot and waits: the last kernel stores the
-// scalar to host memory itself, with no copy launch behind it.
+// Folds and waits: the last kernel posts the scalar to the host itself, with no
+// copy launch behind it and no wait for the kernel's own end.
 template <typename P, bool kF64Final, typename R>
 int run_fold_host(const typename P::In *in, size_t n, R *h_result, const char *name) {
     void *slot = nullptr;
-    int rc = msl_result_slot(&slot, nullptr);
+    uint32_t seq = 0;
+    int rc = host_post_slot(&slot, &seq);
     if (rc) return rc;
-    rc = run_fold<P, kF64Final>(in, n, slot, name);
+    rc = run_fold<P, kF64Final>(in, n, slot, seq, name);
     if (rc) return rc;
-    MSL_HIP_TRY(hipStreamSynchronize(ctx().stream));
-    *h_result = *static_cast<const R *>(slot);
+    uint64_t bits = 0;
+    rc = host_post_wait(slot, seq, &bits, name);
+    if (rc) return rc;
+    std::memcpy(h_result, &bits, sizeof(*h_result));
     return MSL_OK;
 }
 
@@ -318,7 +337,7 @@ extern "C" {
 
 int msl_fold_sum_f32(const float *d_in, size_t n, double *d_result) {
     MSL_REQUIRE(d_result != nullptr, "msl_fold_sum_f32: null result pointer");
-    return run_fold<CompSumPolicy, true>(d_in, n, d_result, "msl_fold_sum_f32");
+    return run_fold<CompSumPolicy, true>(d_in, n, d_result, 0, "msl_fold_sum_f32");
 }
 
 int msl_fold_sum_f32_noalloc(const float *d_in, size_t n, double *d_result) {
@@ -333,7 +352,7 @@ int msl_fold_sum_f32_noalloc(const float *d_in, size_t n, double *d_result) {
                                        "(lower MSL_FOLD_BLOCKS_PER_CU)");
     Pair *partials = reinterpret_cast<Pair *>(g_scratch_ptr[ctx().device]);
     MSL_REQUIRE(partials != nullptr, "msl_fold_sum_f32_noalloc: scratch not set up on this device");
-    return launch_fold<CompSumPolicy, true>(d_in, n, blocks, partials, d_result, "msl_fold_sum_f32_noalloc");
+    return launch_fold<CompSumPolicy, true>(d_in, n, blocks, partials, d_result, 0, "msl_fold_sum_f32_noalloc");
 }
 
 int msl_fold_sum_f32_host(const float *d_in, size_t n, double *h_sum64, float *h_sum32) {
