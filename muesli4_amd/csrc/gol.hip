@@ -41,7 +41,8 @@ constexpr int kFirstRows = 8;
 __global__ __launch_bounds__(64) void gol_first_kernel(uint32_t *__restrict__ out, const int32_t *__restrict__ in,
                                                        int rows, int cols, int words, int tiles_x) {
     const int lane = threadIdx.x;
-    const int tx = blockIdx.x % tiles_x, ty = blockIdx.x / tiles_x;
+    const int tile = (int)xcd_tile(blockIdx.x, gridDim.x);
+    const int tx = tile % tiles_x, ty = tile / tiles_x;
     const int x = tx * 64 + lane, y0 = ty * kFirstRows;
     const int xl = max(min(x - 1, cols - 1), 0), xc = min(x, cols - 1), xr = min(x + 1, cols - 1);
     uint32_t l[kFirstRows + 2], c[kFirstRows + 2], r[kFirstRows + 2];
@@ -96,7 +97,8 @@ template <bool kUnpack>
 __global__ __launch_bounds__(64) void gol_bits_kernel(void *__restrict__ out, const uint32_t *__restrict__ in,
                                                       int rows, int cols, int words, int steps, int tiles_x) {
     const int lane = threadIdx.x;
-    const int tx = blockIdx.x % tiles_x, ty = blockIdx.x / tiles_x;
+    const int tile = (int)xcd_tile(blockIdx.x, gridDim.x);
+    const int tx = tile % tiles_x, ty = tile / tiles_x;
     const int w0 = tx * kBitInner - 1;
     const int y = ty * kBitRows - kBitSteps + lane;
     const bool rowok = (unsigned)y < (unsigned)rows;
