@@ -58,10 +58,10 @@ int blur_tile_step(float *out, const float *in, int rows, int cols, int r, float
 // Tile of a launch of `steps` generations: columns, rows per thread of the
 // column pass (the workgroup has 16 w / m threads) and output rows, by the
 // smallest modelled time.  The model is the kernel's structure with six
-// coefficients fitted to 9000 timings (64^2 .. 4096^2, r = 1 .. 10, 1 .. 6
-// generations; its choice is 3 % slower than the best shape on average, 22 %
+// coefficients fitted to 8000 timings (64^2 .. 4096^2, r = 2 .. 13, 1 .. 6
+// generations; its choice is 1 % slower than the best shape on average, 14 %
 // at worst):
-//   3.1 us         per launch (drain, launch, first load, last store)
+//   1.9 us         per launch (drain, launch, first load, last store)
 //   0.6 us         per generation (two barriers)
 //   lat            the dependent chain of one wave: its rounds of row sums
 //                  and its column sums
@@ -87,8 +87,8 @@ TileShape tile_shape(int rows, int cols, int r, int steps) {
             const double tiles =
                 (double)((cols + tile_w - 1) / tile_w) * (double)((rows + th - 1) / th) / cus;
             const double b = tiles <= 1.0 ? 1.0 : 0.5 * (std::ceil(tiles) + tiles);
-            const double us = 3.14 + 0.592 * steps + 0.00938 * lat +
-                              b * (1.31e-6 * vw + 2.19e-4 * (th + 2 * r * steps) * w + 0.0163 * steps * (w / (4 * m)));
+            const double us = 1.90 + 0.613 * steps + 0.00719 * lat +
+                              b * (2.12e-6 * vw + 1.70e-4 * (th + 2 * r * steps) * w + 0.0145 * steps * (w / (4 * m)));
             if (us < best.us) best = TileShape{w, m, th, us};
         }
     }

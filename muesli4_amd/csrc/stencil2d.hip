@@ -103,13 +103,38 @@ inline int row_mode(const T *in, const T *out, int cols) {
     return kScalar;
 }
 
-// Single steps of radius kTile1MinR and above on grids of at most
-// kTile1MaxCells run the tile kernel (blur_tile.hip): us per step, strip
-// march / tile: 500 x 517 r = 4 5.7 / 4.8, 5 6.5 / 5.0, 10 11.1 / 5.3;
-// 1024^2 r = 4 5.9 / 6.4, 5 6.8 / 6.3, 10 11.7 / 7.1; 2048^2 r = 4 9.3 / 10.7,
-// 6 12.9 / 11.2, 10 17.7 / 13.2; 3000^2 r = 6 17.6 / 19.3, 10 22.1 / 24.4.
-constexpr int kTile1MinR = 5;
-constexpr long kTile1MaxCells = 9L << 19;  // 4.7 million
+// Grids whose single steps run the tile kernel (blur_tile.hip), and their
+// tiles: 16-wave tiles (one row per thread) of the fewest rows that give at most
+// one per CU, else 8-wave tiles of 64 rows once those give two per CU and of 32
+// below; 128-column tiles, which read the fewest LDS cells per output, above
+// kTile1WideCells and at radii above 10 (whose 64-column tiles hold few
+// outputs) from four tiles per CU.  us per step, strip march / tile: 300 x
+// 1000 r = 2 4.1 / 3.6, 4 5.1 / 3.7; 1201 x 1999 r = 2 8.1 / 5.8, 4 9.2 / 6.4;
+// 2048^2 r = 2 7.5 / 7.8, 4 9.1 / 8.8, 10 17.7 / 11.7, 13 - / 14.6; 3000^2
+// r = 5 18.2 / 15.4, 7 22.0 / 16.7, 10 21.8 / 21.0, 13 30.7 / 24.0; 4096^2
+// r = 2 23.4 / 23.5, 5 27.8 / 25.4, 8 29.1 / 28.6, 10 30.7 / 30.9, 13 49.5 / 38.4;
+// 5000 x 5001 r = 5 42.9 / 33.3, 10 48.1 / 44.8, 16 81.0 / 68.6; 5792^2 r = 5
+// 47.0 / 42.4, 8 49.4 / 49.9, 10 52.3 / 58.8, 16 77.5 / 87.8.
+// Radius 10 on aligned rows marches above 10.5 million cells (one-call us from
+// memory, march / tile: 3000^2 21.3 / 18.6, 3400 x 3600 26.0 / 27.0; unaligned
+// rows 4095^2 42.5 / 35.8), and so do radii 5 and 6 at row strides of 4 KB
+// multiples, where the tiles' loads meet in few memory channels (r = 5,
+// 4096 x 4100 32.9 / 30.8, 4096^2 32.0 / 33.5).
+constexpr long kTile1WideCells = 9L << 19;
+static bool tile1_default(const float *in, const float *out, int r, int rows, int cols) {
+    if (r < 2) return false;
+    const bool march = (r == 10 && row_mode(in, out, cols) == kAligned) || (r <= 6 && cols % 1024 == 0);
+    return (long)rows * cols <= (r <= 4 ? 3L << 20 : march ? 10L << 20 : 25L << 20);
+}
+
+static TileShape tile1_shape(int rows, int cols, int r) {
+    const int cus = ctx().num_cus, tile_w = (64 - 2 * r) / 4 * 4;
+    auto tiles = [&](int h) { return (long)((cols + tile_w - 1) / tile_w) * ((rows + h - 1) / h); };
+    for (int h = 8; h <= 32; h *= 2)
+        if (tiles(h) <= cus) return TileShape{64, 1, h, 0.0};
+    if ((long)rows * cols > kTile1WideCells || (r > 10 && tiles(64) > 4L * cus)) return TileShape{128, 4, 64, 0.0};
+    return TileShape{64, 2, tiles(64) < 2L * cus ? 32 : 64, 0.0};
+}
 
 struct StripShape {
     int seg, strips_x, segs, nitems, c;
@@ -128,7 +153,7 @@ inline StripShape strip_shape(int rows, int cols, int r, int seg, bool streamed)
     StripShape s;
     const long cus = ctx().num_cus;
     const long strips4 = (cols + kStripW - 1) / kStripW;
-    s.c = r < kTile1MinR && strips4 * ((rows + 7) / 8) < 8 * cus ? 1 : 4;
+    s.c = r == 1 && strips4 * ((rows + 7) / 8) < 8 * cus ? 1 : 4;
     const int sw = 64 * s.c;
     s.strips_x = (cols + sw - 1) / sw;
     if (seg <= 0) seg = tune_int("MSL_STRIP_SEG", 0);
@@ -158,7 +183,7 @@ int launch_strip(typename Pol::T *out, const typename Pol::T *in, int rows, int 
     StripShape s = strip_shape(rows, cols, Pol::R, seg, nt);
     const int blocks = (s.nitems + 3) / 4;
     const int mode = row_mode(in, out, cols);
-    if constexpr (Pol::R < kTile1MinR) {
+    if constexpr (Pol::R == 1) {
         if (s.c == 1) {
             strip_stencil_kernel<Pol, kAligned, false, 1><<<blocks, 256, 0, ctx().stream>>>(
                 out, in, rows, cols, nv, s.seg, s.strips_x, s.nitems, pol);
@@ -252,12 +277,8 @@ int mean_step(float *out, const float *in, int rows, int cols, int r, float nv, 
     MSL_REQUIRE((int64_t)rows * cols <= INT32_MAX && cols < (1 << 30), "msl_stencil2d_mean_f32: grid too large");
     if (rows == 0 || cols == 0) return MSL_OK;
     MSL_REQUIRE(out && in && out != in, "msl_stencil2d_mean_f32: null or aliased buffers");
-    if (r >= kTile1MinR && (long)rows * cols <= kTile1MaxCells && seg <= 0) {
-        // 64-row tiles once they give two workgroups per CU, else 32-row ones
-        const int tile_w = (64 - 2 * r) / 4 * 4;
-        const long tiles = (long)((cols + tile_w - 1) / tile_w) * ((rows + 63) / 64);
-        return blur_tile_step(out, in, rows, cols, r, nv, 1, TileShape{64, 2, tiles < 2L * ctx().num_cus ? 32 : 64, 0.0});
-    }
+    if (seg <= 0 && tile1_default(in, out, r, rows, cols))
+        return blur_tile_step(out, in, rows, cols, r, nv, 1, tile1_shape(rows, cols, r));
     return kMeanLaunchers[r](out, in, rows, cols, nv, seg);
 }
 

@@ -71,3 +71,14 @@ def test_blur_tile_special_values(r, iters):
         y[rng.integers(0, 150, 6), rng.integers(0, 260, 6)] = v
         got, ref = _iterate(y, r, 0.0, iters)
         np.testing.assert_array_equal(got, ref)
+
+
+@pytest.mark.parametrize("shape,r", [((2200, 2201), 5), ((2200, 2201), 10), ((2201, 2204), 9), ((1030, 4099), 12)])
+def test_blur_tile_wide_single_steps(shape, r):
+    """Single steps in 128-column tiles: grids above 4.7 million cells, and
+    radii above 10 from four 64-column tiles per CU."""
+    print(f"[case] blur tile wide {shape} r={r}", flush=True)
+    hip.init(0)
+    x = R.fill_uniform_f32(shape[0] * shape[1], 11).reshape(shape)
+    got, ref = _iterate(x, r, 1.5, 1, shift=1)
+    np.testing.assert_array_equal(got.view(np.uint32), ref.view(np.uint32))
