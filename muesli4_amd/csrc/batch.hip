@@ -323,27 +323,6 @@ __global__ __launch_bounds__(256) void batch_round_final_kernel(const BGrid *__r
     if (threadIdx.x == 0) sums[gi] = ((waves[0] + waves[1]) + waves[2]) + waves[3];
 }
 
-// One wave per grid: sum = sum over the grid's items, in item order, of
-// (double)s + (double)c; lanes take items l, l+64, ... and are combined in a
-// fixed butterfly.
-__global__ __launch_bounds__(256) void batch_fold_final_kernel(const BGrid *__restrict__ grids, int ngrids,
-                                                               const float2 *__restrict__ partials,
-                                                               double *__restrict__ sums) {
-    const int lane = threadIdx.x & 63;
-    const int gi = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (gi >= ngrids) return;
-    const BGrid g = grids[gi];
-    double acc = 0.0;
-    for (int k = lane; k < g.nitems; k += 64) {
-        const float2 p = partials[g.item0 + k];
-        acc += (double)p.x;
-        acc += (double)p.y;
-    }
-#pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) acc += __shfl_xor(acc, m);
-    if (lane == 0) sums[gi] = acc;
-}
-
 __global__ void batch_zero_kernel(unsigned *p, int n) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) p[i] = 0u;

@@ -38,12 +38,10 @@ __device__ __forceinline__ float from_right(float v, float edge) {
 }
 
 // March the tile (x0 = 64 * xtile, rows y0 .. y0+kTY-1) over planes
-// z0 .. z1-1.  kResidual: fold max |v - in| into *dmax.  kSum: push every
-// stored value into *sum.
-template <bool kResidual, bool kSum, bool NT = true>
+// z0 .. z1-1.  kResidual: fold max |v - in| into *dmax.
+template <bool kResidual, bool NT = true>
 __device__ __forceinline__ void heat7_march(float *__restrict__ out, const float *__restrict__ in, int nx, int ny,
-                                            int nz, float nv, int x0, int y0, int z0, int z1, float *dmax,
-                                            LaneSum *sum) {
+                                            int nz, float nv, int x0, int y0, int z0, int z1, float *dmax) {
     const int lane = threadIdx.x & 63;
     const int x = x0 + lane;
     const int hxl = lane == 0 ? x - 1 : (lane == 63 ? x + 1 : x);  // x-halo column
@@ -129,7 +127,6 @@ __device__ __forceinline__ void heat7_march(float *__restrict__ out, const float
                         const float d = fabsf(__fsub_rn(v, c));
                         *dmax = d > *dmax ? d : *dmax;
                     }
-                    if constexpr (kSum) sum->push(v);
                 }
             }
         }
@@ -150,8 +147,8 @@ __device__ __forceinline__ void heat7_march(float *__restrict__ out, const float
 constexpr int kT2X = kTX - 4;  // output columns of a two-generation wave tile
 // Output rows of a two-generation wave tile: 5 rows (90 VGPRs, five waves
 // per SIMD) beat 8 (124, four) although the y halo grows from 4/8 to 4/5
-// (512^3, 200 iterations: 8 rows 32.5 ms, 7 32.6, 6 31.8, 5 30.5, 4 35.1;
-// 320^3: 8 rows 7.13 ms, 5 6.90).
+// (200 iterations of a 320^3 cube alone: 8 rows 7.13 ms, 5 6.90).  The serving
+// engine's items use it; single cubes run heat_tile.hip and heat_pair.hip.
 constexpr int kT2Y = 5;
 
 template <bool kSingle>

@@ -504,8 +504,6 @@ int msl_stencil2d_mean_iterate_plan(const float *d_a, const float *d_b, int rows
     MSL_REQUIRE(iters >= 0 && rows >= 0 && cols >= 0, "msl_stencil2d_mean_iterate_plan: negative argument");
     MSL_REQUIRE(r >= 1 && r <= kMaxMeanR, "msl_stencil2d_mean_iterate_plan: radius must be in [1, 16]");
     MSL_REQUIRE(h_launches != nullptr && capacity >= 0, "msl_stencil2d_mean_iterate_plan: bad output arguments");
-    int rc = ensure_ready();  // the tile model counts the device's CUs
-    if (rc) return rc;
     std::vector<MeanLaunch> plan;
     if (iters > 0 && rows > 0 && cols > 0) plan = mean_iterate_plan(d_a, d_b, rows, cols, r, iters);
     *h_launches = (int)plan.size();

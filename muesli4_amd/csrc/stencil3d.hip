@@ -39,8 +39,7 @@ __global__ __launch_bounds__(256) void heat7_kernel(float *__restrict__ out, con
         const int yt = rest % ytiles;
         const int zs = rest / ytiles;
         const int z0 = zs * zseg;
-        heat7_march<kResidual, false, NT>(out, in, nx, ny, nz, nv, xt * kTX, yt * kTY, z0, min(z0 + zseg, nz), &dmax,
-                                          nullptr);
+        heat7_march<kResidual, NT>(out, in, nx, ny, nz, nv, xt * kTX, yt * kTY, z0, min(z0 + zseg, nz), &dmax);
     }
     if (kResidual) {
         __shared__ float wmax[4];
