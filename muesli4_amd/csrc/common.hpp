@@ -254,4 +254,13 @@ __device__ __forceinline__ unsigned xcd_tile(unsigned bid, unsigned nblocks) {
     return xcd * (nblocks / kXcd) + (xcd < rest ? xcd : rest) + bid / kXcd;
 }
 
+// The same for launches whose tiles differ in cost (the hardware hands out
+// workgroups in order as others end, so costs balance by themselves): within
+// each 64 workgroups, every XCD takes 8 neighbours.
+__device__ __forceinline__ unsigned xcd_mixed_tile(unsigned bid, unsigned nblocks) {
+    constexpr unsigned kXcd = 8, kNear = 8, kGroup = kXcd * kNear;
+    const unsigned base = bid / kGroup * kGroup, k = bid - base;
+    return base + kGroup > nblocks ? bid : base + k % kXcd * kNear + k / kXcd;
+}
+
 }  // namespace mslhip

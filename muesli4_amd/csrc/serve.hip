@@ -15,7 +15,7 @@
 //     first-fit allocator with coalescing (no per-job hipMalloc, no
 //     fragmentation growth beyond the free list);
 //   * every round advances each active stencil job by several steps in one
-//     or more launches: one persistent launch covers all active blur jobs'
+//     or more launches: one launch covers all active blur jobs'
 //     tiles and advances each by the generations its radius allows in LDS
 //     (blur_tile.hpp), one covers all heat jobs' (tile, z-segment) items, two
 //     generations each, one covers the chunks of the map+fold jobs admitted
@@ -23,7 +23,7 @@
 //     The number of launches (at most kMaxSub) aims at kRoundUs of work, so
 //     that the per-round host work and small launches stay a modest share;
 //   * after a job's last step its final state is folded (compensated FP32
-//     pairs per fixed 64K-element chunk, combined in FP64 in chunk order;
+//     pairs per fixed 8K-element chunk, combined in FP64 in chunk order;
 //     wrapping u32 for map+fold) and the round's results are copied to
 //     pinned host memory;
 //   * up to kRing rounds are in flight; a round's event retires its
@@ -98,13 +98,9 @@ struct SFinal {
     int kind, item0, nitems, slot;
 };
 
-// item_desc[i] = largest j with starts[j] <= i (starts ascending, starts[0] = 0);
-// also clears the round's nctr work-queue counters of this kind, one per launch
-// (the work kernels run after this one on the same stream).
-__global__ void serve_expand_kernel(const int *__restrict__ starts, int ndesc, int nitems, int *__restrict__ item_desc,
-                                    unsigned *__restrict__ ctr, int nctr) {
+// item_desc[i] = largest j with starts[j] <= i (starts ascending, starts[0] = 0).
+__global__ void serve_expand_kernel(const int *__restrict__ starts, int ndesc, int nitems, int *__restrict__ item_desc) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < nctr) ctr[i] = 0u;
     if (i >= nitems) return;
     int lo = 0, hi = ndesc - 1;
     while (lo < hi) {
@@ -113,15 +109,6 @@ __global__ void serve_expand_kernel(const int *__restrict__ starts, int ndesc, i
         else hi = mid - 1;
     }
     item_desc[i] = lo;
-}
-
-// Each wave takes its first item statically and every further one from the
-// round's atomic counter (items differ in cost by radius and shape, so a
-// static split leaves a long tail).
-__device__ __forceinline__ int serve_next_item(unsigned *ctr, int stride) {
-    unsigned nx = 0;
-    if ((threadIdx.x & 63) == 0) nx = atomicAdd(ctr, 1u);
-    return stride + __builtin_amdgcn_readfirstlane((int)nx);
 }
 
 // Most generations of a blur job per launch: as many as the LDS tile still
@@ -149,58 +136,49 @@ __device__ __forceinline__ void serve_blur_tile(const SBlur &g, const float *src
 constexpr size_t serve_tile_lds(int w) { return blur_tile_lds(kBatchMaxR, w, kTileRows, 1); }
 
 // Launch k of the round over every tile of every active blur job (tiles of
-// jobs that are done in this round are skipped); one workgroup per tile, the
-// next tile from the launch's counter.  Bound by VALU issue at load and by
-// the latency of a tile's barriers and loads otherwise.  128 jobs at once:
-// 42 ms of one-step strip items (486 launches of 86 us) before.
+// jobs that are done in this round are skipped), one workgroup per tile.  Bound
+// by VALU issue at load and by the latency of a tile's barriers and loads
+// otherwise.  128 jobs at once: 42 ms of one-step strip items (486 launches of
+// 86 us), 14.5 with persistent workgroups that took tiles from a counter
+// (two more barriers and an atomic's latency per tile), and all launches of
+// the run 31.8 -> 27.0 ms with one workgroup per tile or heat item.
 template <int W, int M>
 __global__ __launch_bounds__(16 * W / M) void serve_blur_kernel(const SBlur *__restrict__ descs,
-                                                                const int *__restrict__ item_desc, int nitems,
-                                                                unsigned *__restrict__ ctr, int k_launch) {
+                                                                const int *__restrict__ item_desc, int k_launch) {
     extern __shared__ __attribute__((aligned(16))) float lds[];
-    __shared__ int next;
-    for (int i = (int)xcd_tile(blockIdx.x, gridDim.x); i < nitems;) {
-        const SBlur g = descs[__builtin_amdgcn_readfirstlane(item_desc[i])];
-        const int gens = min(g.gens, g.steps - k_launch * g.gens);
-        if (gens > 0) {
-            const bool odd = (g.parity0 + k_launch) & 1;
-            const int k = i - g.item0;
-            serve_blur_tile<W, M>(g, odd ? g.b : g.a, odd ? g.a : g.b, gens, k % g.tiles_x, k / g.tiles_x, lds);
-        }
-        if (threadIdx.x == 0) next = (int)(gridDim.x + atomicAdd(ctr, 1u));
-        __syncthreads();  // also: the tile's last reads of lds are done
-        i = __builtin_amdgcn_readfirstlane(next);
-        __syncthreads();
-    }
+    const int i = (int)xcd_mixed_tile(blockIdx.x, gridDim.x);
+    const SBlur g = descs[__builtin_amdgcn_readfirstlane(item_desc[i])];
+    const int gens = min(g.gens, g.steps - k_launch * g.gens);
+    if (gens <= 0) return;
+    const bool odd = (g.parity0 + k_launch) & 1;
+    const int k = i - g.item0;
+    serve_blur_tile<W, M>(g, odd ? g.b : g.a, odd ? g.a : g.b, gens, k % g.tiles_x, k / g.tiles_x, lds);
 }
 
 // Launch k of the round over every item of every active heat job: two
 // generations, or the last one of an odd count.
 __global__ __launch_bounds__(256) void serve_heat_kernel(const SHeat *__restrict__ descs,
                                                          const int *__restrict__ item_desc, int nitems,
-                                                         unsigned *__restrict__ ctr, int k_launch) {
-    const int wave = threadIdx.x >> 6;
-    const int nw = gridDim.x * 4;
-    for (int i = __builtin_amdgcn_readfirstlane((int)xcd_tile(blockIdx.x, gridDim.x) * 4 + wave); i < nitems;
-         i = serve_next_item(ctr, nw)) {
-        const int j = __builtin_amdgcn_readfirstlane(item_desc[i]);
-        const SHeat g = descs[j];
-        const int gens = g.steps - 2 * k_launch;
-        if (gens <= 0) continue;
-        const bool odd = (g.parity0 + k_launch) & 1;
-        const float *src = odd ? g.b : g.a;
-        float *dst = odd ? g.a : g.b;
-        const int k = i - g.item0;
-        const int xt = k % g.xtiles;
-        const int rest = k / g.xtiles;
-        const int yt = rest % g.ytiles;
-        const int z0 = (rest / g.ytiles) * g.zseg;
-        const int z1 = min(z0 + g.zseg, g.nz);
-        if (gens >= 2)
-            heat7x2_march<false>(dst, src, g.nx, g.ny, g.nz, g.nv, xt * kT2X, yt * kT2Y, z0, z1);
-        else
-            heat7x2_march<true>(dst, src, g.nx, g.ny, g.nz, g.nv, xt * kT2X, yt * kT2Y, z0, z1);
-    }
+                                                         int k_launch) {
+    const int i = __builtin_amdgcn_readfirstlane((int)(xcd_mixed_tile(blockIdx.x, gridDim.x) * 4 + (threadIdx.x >> 6)));
+    if (i >= nitems) return;
+    const int j = __builtin_amdgcn_readfirstlane(item_desc[i]);
+    const SHeat g = descs[j];
+    const int gens = g.steps - 2 * k_launch;
+    if (gens <= 0) return;
+    const bool odd = (g.parity0 + k_launch) & 1;
+    const float *src = odd ? g.b : g.a;
+    float *dst = odd ? g.a : g.b;
+    const int k = i - g.item0;
+    const int xt = k % g.xtiles;
+    const int rest = k / g.xtiles;
+    const int yt = rest % g.ytiles;
+    const int z0 = (rest / g.ytiles) * g.zseg;
+    const int z1 = min(z0 + g.zseg, g.nz);
+    if (gens >= 2)
+        heat7x2_march<false>(dst, src, g.nx, g.ny, g.nz, g.nv, xt * kT2X, yt * kT2Y, z0, z1);
+    else
+        heat7x2_march<true>(dst, src, g.nx, g.ny, g.nz, g.nv, xt * kT2X, yt * kT2Y, z0, z1);
 }
 
 typedef uint32_t v4u_t __attribute__((ext_vector_type(4)));
@@ -402,7 +380,6 @@ struct RoundSlot {
     int *d_item_desc[4] = {nullptr, nullptr, nullptr, nullptr};
     float2 *d_ps = nullptr;  // sum chunk partials
     uint32_t *d_pm = nullptr;
-    unsigned *d_ctr = nullptr;  // work-queue counters, kMaxSub each: blur, heat, then map
     double *d_rf = nullptr, *h_rf = nullptr;
     uint32_t *d_ru = nullptr, *h_ru = nullptr;
     std::vector<std::pair<SJob *, int>> finishing;
@@ -499,7 +476,6 @@ static void slot_free(RoundSlot &R) {
         if (R.d_item_desc[k]) (void)hipFree(R.d_item_desc[k]);
     if (R.d_ps) (void)hipFree(R.d_ps);
     if (R.d_pm) (void)hipFree(R.d_pm);
-    if (R.d_ctr) (void)hipFree(R.d_ctr);
     if (R.d_rf) (void)hipFree(R.d_rf);
     if (R.d_ru) (void)hipFree(R.d_ru);
     if (R.h_rf) (void)hipHostFree(R.h_rf);
@@ -509,7 +485,6 @@ static void slot_free(RoundSlot &R) {
 
 // Grows a slot's buffers (only called while the slot is not in flight).
 static int slot_reserve(RoundSlot &R, size_t stage_bytes, const int items[4]) {
-    if (!R.d_ctr) MSL_HIP_TRY(hipMalloc(&R.d_ctr, sizeof(unsigned) * 4 * kMaxSub));
     if (stage_bytes > R.stage_cap) {
         if (R.h_stage) MSL_HIP_TRY(hipHostFree(R.h_stage));
         if (R.d_stage) MSL_HIP_TRY(hipFree(R.d_stage));
@@ -785,32 +760,28 @@ static int run_round(Server &S, int *did_work) {
     // (map+fold jobs run before the stencil steps: they are single-pass and
     // must not wait behind several steps of the stencil jobs)
     if (items[2]) {
-        serve_expand_kernel<<<(items[2] + 255) / 256, 256, 0, st>>>(gsm, (int)dm.size(), items[2], R.d_item_desc[2],
-                                                                    R.d_ctr + 2 * kMaxSub, 1);
+        serve_expand_kernel<<<(items[2] + 255) / 256, 256, 0, st>>>(gsm, (int)dm.size(), items[2], R.d_item_desc[2]);
         serve_map_kernel<<<persistent(items[2], 4), 256, 0, st>>>(gm, R.d_item_desc[2], items[2], R.d_pm);
     }
     if (items[0])
-        serve_expand_kernel<<<(items[0] + 255) / 256, 256, 0, st>>>(gsb, (int)db.size(), items[0], R.d_item_desc[0],
-                                                                    R.d_ctr, nsub_max[0]);
+        serve_expand_kernel<<<(items[0] + 255) / 256, 256, 0, st>>>(gsb, (int)db.size(), items[0], R.d_item_desc[0]);
     if (items[1])
-        serve_expand_kernel<<<(items[1] + 255) / 256, 256, 0, st>>>(gsh, (int)dh.size(), items[1], R.d_item_desc[1],
-                                                                    R.d_ctr + kMaxSub, nsub_max[1]);
+        serve_expand_kernel<<<(items[1] + 255) / 256, 256, 0, st>>>(gsh, (int)dh.size(), items[1], R.d_item_desc[1]);
     for (int k = 0; k < std::max(nsub_max[0], nsub_max[1]); k++) {
         if (k < nsub_max[0] && light)
             serve_blur_kernel<kLightW, kLightM>
-                <<<std::min(items[0], cus), 16 * kLightW / kLightM, serve_tile_lds(kLightW), st>>>(
-                    gb, R.d_item_desc[0], items[0], R.d_ctr + k, k);
+                <<<items[0], 16 * kLightW / kLightM, serve_tile_lds(kLightW), st>>>(
+                    gb, R.d_item_desc[0], k);
         else if (k < nsub_max[0])
             serve_blur_kernel<kHeavyW, kHeavyM>
-                <<<std::min(items[0], cus * 3), 16 * kHeavyW / kHeavyM, serve_tile_lds(kHeavyW), st>>>(
-                    gb, R.d_item_desc[0], items[0], R.d_ctr + k, k);
+                <<<items[0], 16 * kHeavyW / kHeavyM, serve_tile_lds(kHeavyW), st>>>(
+                    gb, R.d_item_desc[0], k);
         if (k < nsub_max[1])
-            serve_heat_kernel<<<persistent(items[1], 3), 256, 0, st>>>(gh, R.d_item_desc[1], items[1],
-                                                                       R.d_ctr + kMaxSub + k, k);
+            serve_heat_kernel<<<(items[1] + 3) / 4, 256, 0, st>>>(gh, R.d_item_desc[1], items[1], k);
     }
     if (items[3]) {
         serve_expand_kernel<<<(items[3] + 255) / 256, 256, 0, st>>>(gss_start, (int)ds.size(), items[3],
-                                                                    R.d_item_desc[3], R.d_ctr + 3 * kMaxSub, 1);
+                                                                    R.d_item_desc[3]);
         serve_sum_kernel<<<persistent(items[3], 4), 256, 0, st>>>(gss, R.d_item_desc[3], items[3], R.d_ps);
     }
     if (!fin.empty()) {
