@@ -230,7 +230,6 @@ __global__ __launch_bounds__(256) void batch_round_kernel(const BGrid *__restric
 // take 470 us per generation, in two-generation strips 435.)
 constexpr int kTileGens[kBatchPairMaxR + 1] = {0, 6, 4, 4, 3, 3, 2, 2, 2};
 constexpr int kTileThreads = 512;    // W = 128, M = 4 or W = 64, M = 2
-constexpr int kTileBlocksPerCu = 3;  // 44 KB of LDS each
 constexpr size_t kTileLds = blur_tile_lds(kBatchPairMaxR, 128, kTileRows, 1);
 
 // Output columns and rows of a tile of w columns and gens generations.
@@ -249,27 +248,21 @@ __device__ __forceinline__ void tile_item(const BGrid &g, const float *src, floa
                        it.y0, lds);
 }
 
-// The tiles (xs, y0) of y1 generations of a round, a workgroup each; the next
-// one from the round's counter.  Bound by VALU issue.
+// The tiles (xs, y0) of y1 generations of a round, a workgroup each.  Bound by
+// VALU issue.  (Persistent workgroups that took tiles from a counter: the 4096-
+// grid batch 5.05 ms, now 4.91.  The strip items stay persistent: their waves
+// end at different times, and one workgroup per four of them took 5.36.)
 __global__ __launch_bounds__(kTileThreads) void batch_tile_kernel(const BGrid *__restrict__ grids,
-                                                                  const RItem *__restrict__ items, int nitems,
-                                                                  unsigned *__restrict__ ctr) {
+                                                                  const RItem *__restrict__ items) {
     extern __shared__ __attribute__((aligned(16))) float lds[];
-    __shared__ int next;
-    for (int i = (int)xcd_tile(blockIdx.x, gridDim.x); i < nitems;) {
-        const RItem it = items[i];
-        const BGrid g = grids[it.g];
-        const float *src = (it.flags & kRSrcB) ? g.b : g.a;
-        float *dst = (it.flags & kRSrcB) ? g.a : g.b;
-        if (it.flags & kRTile64)
-            tile_item<64, 2>(g, src, dst, it, lds);
-        else
-            tile_item<128, 4>(g, src, dst, it, lds);
-        if (threadIdx.x == 0) next = (int)(gridDim.x + atomicAdd(ctr, 1u));
-        __syncthreads();  // also: the tile's last reads of lds are done
-        i = __builtin_amdgcn_readfirstlane(next);
-        __syncthreads();
-    }
+    const RItem it = items[xcd_mixed_tile(blockIdx.x, gridDim.x)];
+    const BGrid g = grids[it.g];
+    const float *src = (it.flags & kRSrcB) ? g.b : g.a;
+    float *dst = (it.flags & kRSrcB) ? g.a : g.b;
+    if (it.flags & kRTile64)
+        tile_item<64, 2>(g, src, dst, it, lds);
+    else
+        tile_item<128, 4>(g, src, dst, it, lds);
 }
 
 // One workgroup per grid.  FP64 sum of the (s, c) pairs of its last round's
@@ -808,7 +801,7 @@ static int build_rounds(Batch &b, int iters, bool fold, RunGraph &rg, std::vecto
     MSL_HIP_TRY(hipMalloc(&rg.d_items, sizeof(RItem) * std::max<size_t>(items.size(), 1)));
     MSL_HIP_TRY(hipMalloc(&rg.d_fold, sizeof(int2) * hfold.size()));
     MSL_HIP_TRY(hipMalloc(&rg.d_partials, sizeof(float2) * std::max(nparts, 1)));
-    MSL_HIP_TRY(hipMalloc(&rg.d_ctr, sizeof(unsigned) * std::max<size_t>(3 * nrounds, 1)));
+    MSL_HIP_TRY(hipMalloc(&rg.d_ctr, sizeof(unsigned) * std::max<size_t>(2 * nrounds, 1)));
     if (!items.empty())
         MSL_HIP_TRY(hipMemcpyAsync(rg.d_items, items.data(), sizeof(RItem) * items.size(), hipMemcpyHostToDevice,
                                    ctx().stream));
@@ -822,7 +815,7 @@ static int build_rounds(Batch &b, int iters, bool fold, RunGraph &rg, std::vecto
 // and the per-grid fold combine.
 static int enqueue_rounds(Batch &b, const std::vector<RoundRange> &rounds, double *d_sums, const RunGraph &rg) {
     hipStream_t s = ctx().stream;
-    const int nc = (int)(3 * rounds.size());
+    const int nc = (int)(2 * rounds.size());
     if (nc > 0) {
         batch_zero_kernel<<<(nc + 255) / 256, 256, 0, s>>>(rg.d_ctr, nc);
         int rc = check_launch("msl_batch_run");
@@ -834,16 +827,15 @@ static int enqueue_rounds(Batch &b, const std::vector<RoundRange> &rounds, doubl
         if (rr.n[0]) {
             const int blocks = std::max(1, std::min((rr.n[0] + 3) / 4, cus * b.max_pair_blocks_per_cu));
             batch_round_kernel<true><<<blocks, 256, 0, s>>>(b.d_grids, rg.d_items + rr.off[0], rr.n[0], rg.d_partials,
-                                                            rg.d_ctr + 3 * j);
+                                                            rg.d_ctr + 2 * j);
         }
         if (rr.n[1])
-            batch_tile_kernel<<<std::min(rr.n[1], cus * kTileBlocksPerCu), kTileThreads, kTileLds, s>>>(
-                b.d_grids, rg.d_items + rr.off[1], rr.n[1], rg.d_ctr + 3 * j + 1);
+            batch_tile_kernel<<<rr.n[1], kTileThreads, kTileLds, s>>>(b.d_grids, rg.d_items + rr.off[1]);
         if (rr.n[2]) {
             const int bpc = std::max(1, std::min(b.blocks_per_cu, b.max_blocks_per_cu));
             const int blocks = std::max(1, std::min((rr.n[2] + 3) / 4, cus * bpc));
             batch_round_kernel<false><<<blocks, 256, 0, s>>>(b.d_grids, rg.d_items + rr.off[2], rr.n[2], rg.d_partials,
-                                                             rg.d_ctr + 3 * j + 2);
+                                                             rg.d_ctr + 2 * j + 1);
         }
         int rc = check_launch("msl_batch_run");
         if (rc) return rc;
