@@ -10,7 +10,7 @@
 // of its launches unpacks to ints.  The packed grids (1/32 of the cells each)
 // live in the caller's two buffers, in the one that does not hold the data
 // being read or the result.  100 generations of 1024^2 and a fold, which 13
-// launches of an int-per-cell register window took 210 us for, take 67 us
+// launches of an int-per-cell register window took 210 us for, take 58 us
 // (windows of 64 x 64 ints: 14 us per 8 generations; here 5.4 us per 14,
 // mostly launch and load latency; 4096 x 4000: 1.9 us per generation, 10.7
 // before).

@@ -31,9 +31,9 @@ __device__ __forceinline__ float lane_from_right(float v) {  // lane l gets lane
 // divide in two operations instead of four (div_pair; the block votes once
 // per launch): 6.2 VALU operations per cell and generation of a window, 9.1
 // before.  8 rows per wave keep 59 VGPRs, eight waves per SIMD (16 rows: 104).
-// 8192^2 x 20: 653 -> 533 us, of which 4 passes over HBM take 420 at the rate
-// of a copy and the VALU issue 287; with the next window's cells loaded ahead
-// by persistent blocks it took 685 (99 VGPRs).
+// 8192^2 x 20: 653 -> 533 us (502 with every XCD on a contiguous range), of
+// which 4 passes over HBM take 420 at the rate of a copy and the VALU issue 381;
+// with the next window's cells loaded ahead by persistent blocks 685 (99 VGPRs).
 template <int K, int RPW, int NW, int NC>
 __global__ __launch_bounds__(64 * NW) void mean3_multi_kernel(float *__restrict__ out, const float *__restrict__ in,
                                                               int rows, int cols, float nv, int steps, int tiles_x,
