@@ -634,6 +634,10 @@ static int autotune(Batch &b, int *entries) {
         for (int r = 1; r <= kBatchMaxR; r++) used |= present[r][wc];
         if (!used) continue;
         for (const Tile &cand : kClassCands) {
+            // runs put narrow classes of one column per lane in LDS tiles, which the
+            // one-step objective does not see (4096 grids, 10 steps, with the
+            // classes it then picked 256-column strips for: 5.10 ms, in tiles 4.96)
+            if (b.pairs && wc < 2 && cand.c != 1) continue;
             Tile saved[kBatchMaxR + 1];
             for (int r = 0; r <= kBatchMaxR; r++) saved[r] = b.table[r][wc];
             rc = try_change([&] { for (int r = 1; r <= kBatchMaxR; r++) b.table[r][wc] = cand; },
