@@ -366,9 +366,10 @@ struct MeanLaunch {
 // one-step kernel.  MSL_MEAN_GENS = 1 or 2 forces one or two
 // generations per launch for r >= 2 (read on every call, so a process can
 // compare both).
-static int mean_gens_env() {
+static int mean_gens_env() {  // 0: not forced (unset, or any other value)
     const char *ge = getenv("MSL_MEAN_GENS");
-    return ge ? atoi(ge) : 0;
+    const int gens = ge ? atoi(ge) : 0;
+    return gens == 1 || gens == 2 ? gens : 0;
 }
 
 static std::vector<MeanLaunch> mean_iterate_plan(const float *d_a, const float *d_b, int rows, int cols, int r,

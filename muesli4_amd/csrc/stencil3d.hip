@@ -139,14 +139,15 @@ __global__ void zero_f32_kernel(float *p, int n) {
 // every call so a process can compare both).  The number of launches must have
 // the parity of iters (the result ends in b exactly when iters is odd, as with
 // one launch per generation); when it does not, one launch is split in two.
-static int heat_gens_env() {
+static int heat_gens_env() {  // 0: not forced (unset, or any other value)
     const char *ge = getenv("MSL_HEAT_GENS");
-    return ge ? atoi(ge) : 0;
+    const int gens = ge ? atoi(ge) : 0;
+    return gens == 1 || gens == 2 ? gens : 0;
 }
 
 static std::vector<int> heat_iterate_plan(int nx, int ny, int nz, int iters, int residual_every) {
     const int env = heat_gens_env();
-    const int most = env == 1 || env == 2 ? env : heat_way(nx, ny, nz).gens;
+    const int most = env ? env : heat_way(nx, ny, nz).gens;
     std::vector<int> plan;
     for (int it = 0; it < iters;) {
         int seg = iters - it;
