@@ -103,7 +103,7 @@ def program_flags() -> list:
             "-L", LIBDIR, "-lmsl_hip", f"-Wl,-rpath,{LIBDIR}"]
 
 
-def build_program(src: str, out: str, rpath_origin: str | None = None) -> str:
+def build_program(src: str, out: str, rpath_origin: str | None = None, extra: tuple = ()) -> str:
     """Compile one C++ skeleton program (e.g. an example written against the
     msl:: API) into an executable linked to libmsl_hip.so.  rpath_origin, if
     given, is the library directory relative to the executable ($ORIGIN), so
@@ -113,15 +113,19 @@ def build_program(src: str, out: str, rpath_origin: str | None = None) -> str:
     if rpath_origin is not None:
         flags = [f for f in flags if not f.startswith("-Wl,-rpath")] + [f"-Wl,-rpath,$ORIGIN/{rpath_origin}"]
     tmp = out + ".tmp"
-    _run([HIPCC, *flags, src, "-o", tmp])
+    _run([HIPCC, *flags, *extra, src, "-o", tmp])
     os.replace(tmp, out)
     return out
 
 
 def build_cpp_tests() -> str:
-    """The C++ API test driver run by tests/test_gpu_cpp_api.py."""
+    """The C++ API test driver run by tests/test_gpu_cpp_api.py, and the
+    allocation-failure test of the serving engine (its own hipMalloc is the one
+    that the library calls, hence -rdynamic)."""
     out = os.path.join(CPP_TESTS, "build", "skeletons_test")
     rel = os.path.relpath(LIBDIR, os.path.dirname(out))
+    build_program(os.path.join(CPP_TESTS, "serve_retry_test.cpp"),
+                  os.path.join(CPP_TESTS, "build", "serve_retry_test"), rpath_origin=rel, extra=("-rdynamic", "-ldl"))
     return build_program(os.path.join(CPP_TESTS, "skeletons_test.cpp"), out, rpath_origin=rel)
 
 

@@ -363,8 +363,10 @@ struct SJob {
     uint32_t *u = nullptr;
     int steps_done = 0;
     int in_b = 0;     // 1: the state after steps_done steps is in b
-    // the round being planned: steps, generations per launch, tiling
-    int steps = 0, gens = 0;
+    // the round being planned: steps, the buffer of the state after them
+    // (steps_done and in_b follow once its launches are enqueued, so a round
+    // that fails before can be run again), generations per launch, tiling
+    int steps = 0, to_b = 0, gens = 0;
     int tile_w = 0, tile_h = 0, tiles_x = 0, xtiles = 0, ytiles = 0, zseg = 0, nitems = 0;
     double sum = 0.0;
     uint32_t sum_u32 = 0;
@@ -490,6 +492,7 @@ static int slot_reserve(RoundSlot &R, size_t stage_bytes, const int items[4]) {
         if (R.d_stage) MSL_HIP_TRY(hipFree(R.d_stage));
         R.h_stage = nullptr;
         R.d_stage = nullptr;
+        R.stage_cap = 0;
         const size_t cap = std::max(stage_bytes * 2, (size_t)1 << 16);
         MSL_HIP_TRY(hipHostMalloc((void **)&R.h_stage, cap, hipHostMallocDefault));
         MSL_HIP_TRY(hipMalloc(&R.d_stage, cap));
@@ -500,6 +503,7 @@ static int slot_reserve(RoundSlot &R, size_t stage_bytes, const int items[4]) {
         const int cap = std::max(items[k] + items[k] / 2, 4096);
         if (R.d_item_desc[k]) MSL_HIP_TRY(hipFree(R.d_item_desc[k]));
         R.d_item_desc[k] = nullptr;
+        R.item_cap[k] = 0;
         MSL_HIP_TRY(hipMalloc(&R.d_item_desc[k], sizeof(int) * cap));
         if (k == 2) {
             if (R.d_pm) MSL_HIP_TRY(hipFree(R.d_pm));
@@ -691,28 +695,26 @@ static int run_round(Server &S, int *did_work) {
         J->steps = std::min(gens * nsub, J->spec.steps - J->steps_done);
         const int launches = (J->steps + gens - 1) / gens;
         *most = std::max(*most, launches);
-        return (J->in_b + launches) & 1;
+        J->to_b = (J->in_b + launches) & 1;
     };
     for (SJob *J : S.blur) {
         const msl_job &s = J->spec;
-        const int to_b = plan_steps(J, J->gens, &nsub_max[0]);
+        plan_steps(J, J->gens, &nsub_max[0]);
         db.push_back(SBlur{J->a, J->b, s.d0, s.d1, s.r, s.nv, J->tiles_x, J->tile_w, J->tile_h, items[0], J->nitems,
                            J->in_b, J->gens, J->steps});
         sb.push_back(items[0]);
-        J->in_b = to_b;
         if (J->steps_done + J->steps == s.steps)
-            add_sum(J, to_b ? J->b : J->a, (long long)s.d0 * s.d1, (int)fin.size());
+            add_sum(J, J->to_b ? J->b : J->a, (long long)s.d0 * s.d1, (int)fin.size());
         items[0] += J->nitems;
     }
     for (SJob *J : S.heat) {
         const msl_job &s = J->spec;
-        const int to_b = plan_steps(J, 2, &nsub_max[1]);
+        plan_steps(J, 2, &nsub_max[1]);
         dh.push_back(SHeat{J->a, J->b, s.d0, s.d1, s.d2, s.nv, J->xtiles, J->ytiles, J->zseg, items[1], J->nitems,
                            J->in_b, J->steps});
         sh.push_back(items[1]);
-        J->in_b = to_b;
         if (J->steps_done + J->steps == s.steps)
-            add_sum(J, to_b ? J->b : J->a, (long long)s.d0 * s.d1 * s.d2, (int)fin.size());
+            add_sum(J, J->to_b ? J->b : J->a, (long long)s.d0 * s.d1 * s.d2, (int)fin.size());
         items[1] += J->nitems;
     }
     for (SJob *J : maps) {
@@ -802,6 +804,7 @@ static int run_round(Server &S, int *did_work) {
         size_t w = 0;
         for (SJob *J : v) {
             J->steps_done += J->steps;
+            J->in_b = J->to_b;
             if (J->steps_done < J->spec.steps) v[w++] = J;
         }
         v.resize(w);
