@@ -39,9 +39,10 @@
 //
 // Fold.  On the last step every lane keeps a TwoSum-compensated sum of the
 // values it stores; a wave combines its lanes in a fixed butterfly and
-// writes one (s, c) pair per item; a final kernel adds a grid's pairs in
-// FP64 in item order, or sums the final state of a grid that ended in tiles
-// (pushing a tile's stores took 1 ms more per round of the 4096-grid batch).
+// writes one (s, c) pair per item.  A grid that ended in tiles gets its pairs
+// from its final state, one per 4096 cells (pushing a tile's stores took 1 ms
+// more per round of the 4096-grid batch).  A final kernel adds a grid's pairs
+// in FP64 in item order.
 // Deterministic for a given tiling.
 //
 // Autotuner.  The launch shape (workgroups per CU, static or atomic queue)
@@ -265,55 +266,64 @@ __global__ __launch_bounds__(kTileThreads) void batch_tile_kernel(const BGrid *_
         tile_item<128, 4>(g, src, dst, it, lds);
 }
 
-// One workgroup per grid.  FP64 sum of the (s, c) pairs of its last round's
-// items (fold[g] = {first partial, count}), in item order; a grid that ended
-// in tiles (count -1 - result buffer) is summed here from its final state:
-// each lane's quads in order, four loads in flight, the lanes' pairs in a fixed
-// butterfly and the waves' in FP64.
-__global__ __launch_bounds__(256) void batch_round_final_kernel(const BGrid *__restrict__ grids,
-                                                                const int2 *__restrict__ fold,
-                                                                const float2 *__restrict__ partials,
-                                                                double *__restrict__ sums) {
-    __shared__ double waves[4];
-    const int lane = threadIdx.x & 63, gi = blockIdx.x;
-    const int2 f = fold[gi];
-    double acc = 0.0;
-    if (f.y >= 0) {
-        if (threadIdx.x >= 64) return;
-        for (int k = lane; k < f.y; k += 64) {
-            const float2 p = partials[f.x + k];
-            acc += (double)p.x;
-            acc += (double)p.y;
-        }
-#pragma unroll
-        for (int m = 32; m >= 1; m >>= 1) acc += __shfl_xor(acc, m);
-        if (lane == 0) sums[gi] = acc;
-        return;
-    }
-    const BGrid g = grids[gi];
-    const float *data = f.y == -2 ? g.b : g.a;
-    const int n = g.rows * g.cols, nq = n / 4;
+// Partials of the grids that ended in tiles: one wave per item {grid, first
+// cell xs, end y0} of kSumChunk cells of the final state (kRSrcB: in b), four
+// 16-byte loads in flight per lane.  A lane adds 64 cells, no more than in a
+// strip item of 64 rows, so the sums lose nothing to longer chains, and a grid
+// of any size is read by the whole device (6 steps of one 300000 x 190 grid
+// and its fold: 0.46 ms, with one workgroup for the sum of a grid 10.1, and
+// 5.7 million equal cells summed with an error of 4e-8).
+constexpr int kSumChunk = 1 << 12;
+
+__global__ __launch_bounds__(256) void batch_sum_kernel(const BGrid *__restrict__ grids,
+                                                        const RItem *__restrict__ items, int nitems,
+                                                        float2 *__restrict__ partials) {
+    const int lane = threadIdx.x & 63;
+    const int i = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4 + (threadIdx.x >> 6)));
+    if (i >= nitems) return;
+    const RItem it = items[i];
+    const BGrid g = grids[it.g];
+    const float *data = ((it.flags & kRSrcB) ? g.b : g.a) + it.xs;
+    const int n = it.y0 - it.xs, nq = n / 4;
     LaneSum ls;
-    int t = threadIdx.x;
-    for (; t + 768 < nq; t += 1024) {
+    int t = lane;
+    for (; t + 192 < nq; t += 256) {
         VecN<float, 4> v[4];
 #pragma unroll
-        for (int u = 0; u < 4; u++) v[u] = load_dword_aligned<float, 4>(data + 4 * (t + 256 * u));
+        for (int u = 0; u < 4; u++) v[u] = load_dword_aligned<float, 4>(data + 4 * (t + 64 * u));
 #pragma unroll
         for (int u = 0; u < 4; u++)
 #pragma unroll
             for (int k = 0; k < 4; k++) ls.push(v[u].v[k]);
     }
-    for (; t < nq; t += 256) {
+    for (; t < nq; t += 64) {
         const VecN<float, 4> v = load_dword_aligned<float, 4>(data + 4 * t);
 #pragma unroll
         for (int k = 0; k < 4; k++) ls.push(v.v[k]);
     }
-    if (4 * nq + (int)threadIdx.x < n) ls.push(data[4 * nq + threadIdx.x]);
+    if (4 * nq + lane < n) ls.push(data[4 * nq + lane]);
     wave_pair_reduce(ls);
-    if (lane == 0) waves[threadIdx.x >> 6] = (double)ls.s + (double)ls.c;
-    __syncthreads();
-    if (threadIdx.x == 0) sums[gi] = ((waves[0] + waves[1]) + waves[2]) + waves[3];
+    if (lane == 0) partials[it.part] = make_float2(ls.s, ls.c);
+}
+
+// One wave per grid: FP64 sum of the (s, c) pairs of its items (fold[g] =
+// {first partial, count}), in item order.
+__global__ __launch_bounds__(256) void batch_round_final_kernel(const int2 *__restrict__ fold, int ngrids,
+                                                                const float2 *__restrict__ partials,
+                                                                double *__restrict__ sums) {
+    const int lane = threadIdx.x & 63;
+    const int gi = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (gi >= ngrids) return;
+    const int2 f = fold[gi];
+    double acc = 0.0;
+    for (int k = lane; k < f.y; k += 64) {
+        const float2 p = partials[f.x + k];
+        acc += (double)p.x;
+        acc += (double)p.y;
+    }
+#pragma unroll
+    for (int m = 32; m >= 1; m >>= 1) acc += __shfl_xor(acc, m);
+    if (lane == 0) sums[gi] = acc;
 }
 
 __global__ void batch_zero_kernel(unsigned *p, int n) {
@@ -708,6 +718,7 @@ struct RoundPlan {
     std::vector<RItem> items;
     std::vector<int2> fold;  // per grid {first partial, count}
     std::vector<RoundRange> rounds;
+    int sum_off = 0, sum_n = 0;  // items of batch_sum_kernel
     int nparts = 0;
     int pair_grids = 0;
 };
@@ -771,7 +782,7 @@ static void plan_rounds(const Batch &b, int iters, bool fold, RoundPlan &rp) {
                     sw = 64 * (kind[g] == kKindNarrow1 ? 1 : 4);
                     seg = std::max(1, t.seg);
                 }
-                if (last) hfold[g] = pass == 1 ? make_int2(0, (iters & 1) ? -2 : -1) : make_int2(nparts, 0);
+                if (last && pass != 1) hfold[g] = make_int2(nparts, 0);
                 for (int xs = 0; xs < G.cols; xs += sw)
                     for (int y0 = 0; y0 < G.rows; y0 += seg) {
                         if (pass == 1) {
@@ -791,13 +802,22 @@ static void plan_rounds(const Batch &b, int iters, bool fold, RoundPlan &rp) {
         }
         rounds.push_back(rr);
     }
+    rp.sum_off = (int)items.size();
+    for (int g : order) {
+        if (!fold || !tiles[g] || plan[g].empty() || plan[g].back() == 1) continue;
+        const int cells = b.grids[g].rows * b.grids[g].cols;
+        hfold[g] = make_int2(nparts, (cells - 1) / kSumChunk + 1);
+        for (int k = 0; k < hfold[g].y; k++)
+            items.push_back(RItem{g, k * kSumChunk, (int)std::min((k + 1L) * kSumChunk, (long)cells), 0,
+                                  (iters & 1) ? kRSrcB : 0, nparts++});
+    }
+    rp.sum_n = (int)items.size() - rp.sum_off;
 }
 
 // Plans the rounds and uploads items and fold ranges into rg's buffers.
-static int build_rounds(Batch &b, int iters, bool fold, RunGraph &rg, std::vector<RoundRange> &rounds) {
-    RoundPlan rp;
+static int build_rounds(Batch &b, int iters, bool fold, RunGraph &rg, RoundPlan &rp) {
     plan_rounds(b, iters, fold, rp);
-    rounds = rp.rounds;
+    const std::vector<RoundRange> &rounds = rp.rounds;
     const std::vector<RItem> &items = rp.items;
     const std::vector<int2> &hfold = rp.fold;
     const int nparts = rp.nparts;
@@ -817,8 +837,9 @@ static int build_rounds(Batch &b, int iters, bool fold, RunGraph &rg, std::vecto
 
 // Enqueues the rounds (counters cleared by a kernel, never a memset node)
 // and the per-grid fold combine.
-static int enqueue_rounds(Batch &b, const std::vector<RoundRange> &rounds, double *d_sums, const RunGraph &rg) {
+static int enqueue_rounds(Batch &b, const RoundPlan &rp, double *d_sums, const RunGraph &rg) {
     hipStream_t s = ctx().stream;
+    const std::vector<RoundRange> &rounds = rp.rounds;
     const int nc = (int)(2 * rounds.size());
     if (nc > 0) {
         batch_zero_kernel<<<(nc + 255) / 256, 256, 0, s>>>(rg.d_ctr, nc);
@@ -846,7 +867,10 @@ static int enqueue_rounds(Batch &b, const std::vector<RoundRange> &rounds, doubl
     }
     if (d_sums) {
         const int ng = (int)b.grids.size();
-        batch_round_final_kernel<<<ng, 256, 0, s>>>(b.d_grids, rg.d_fold, rg.d_partials, d_sums);
+        if (rp.sum_n)
+            batch_sum_kernel<<<(rp.sum_n + 3) / 4, 256, 0, s>>>(b.d_grids, rg.d_items + rp.sum_off, rp.sum_n,
+                                                                rg.d_partials);
+        batch_round_final_kernel<<<(ng + 3) / 4, 256, 0, s>>>(rg.d_fold, ng, rg.d_partials, d_sums);
         return check_launch("msl_batch_run");
     }
     return MSL_OK;
@@ -1003,11 +1027,11 @@ int msl_batch_run_plan(const void *batch, int iters, int with_fold, int *h_round
     plan_rounds(*b, iters, with_fold != 0, rp);
     int launches = rp.rounds.empty() ? 0 : 1;  // counter clear
     for (const RoundRange &rr : rp.rounds) for (int n : rr.n) launches += n > 0;
-    if (with_fold && iters > 0) launches++;
+    if (with_fold && iters > 0) launches += 1 + (rp.sum_n > 0);
     if (h_rounds) *h_rounds = (int)rp.rounds.size();
     if (h_launches) *h_launches = launches;
     if (h_pair_grids) *h_pair_grids = rp.pair_grids;
-    if (h_items) *h_items = (int)rp.items.size();
+    if (h_items) *h_items = rp.sum_off;
     return MSL_OK;
 }
 
@@ -1024,8 +1048,8 @@ int msl_batch_run(void *batch, int iters, double *d_sums, int *h_result_in_b) {
     hipGraphExec_t exec = it == b->graphs.end() ? nullptr : it->second.exec;
     if (!exec) {
         RunGraph rg;
-        std::vector<RoundRange> rounds;
-        rc = build_rounds(*b, iters, d_sums != nullptr, rg, rounds);
+        RoundPlan rp;
+        rc = build_rounds(*b, iters, d_sums != nullptr, rg, rp);
         if (!rc) rc = msl_graph_begin();
         if (rc) {
             if (rg.d_items) (void)hipFree(rg.d_items);
@@ -1034,7 +1058,7 @@ int msl_batch_run(void *batch, int iters, double *d_sums, int *h_result_in_b) {
             if (rg.d_ctr) (void)hipFree(rg.d_ctr);
             return rc;
         }
-        int brc = enqueue_rounds(*b, rounds, d_sums, rg);
+        int brc = enqueue_rounds(*b, rp, d_sums, rg);
         void *g = nullptr;
         int erc = msl_graph_end(&g);
         if (brc || erc) {
