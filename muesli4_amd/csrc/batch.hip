@@ -28,9 +28,10 @@
 // in the wave's LDS and the second generation is formed from them, so each
 // pair of generations reads and writes the grid once), in the launch plan
 // of the single-grid iterations (pairs, with one pair split so that the
-// number of launches keeps the parity of the step count); narrow grids (one
-// column per lane) of those radii run in LDS tiles (blur_tile.hpp), a workgroup
-// per tile and as many generations per round as their radius allows; the other
+// number of launches keeps the parity of the step count); narrow grids (of
+// fewer than 192 columns, or one column per lane) of those radii run in LDS tiles
+// (blur_tile.hpp), a workgroup per tile and as many generations per round as
+// their radius allows; the other
 // grids run one generation per launch.  Each launch round is a pair kernel
 // over the pair items of that round, a tile kernel over its tiles and a step
 // kernel over its single items.
@@ -644,10 +645,6 @@ static int autotune(Batch &b, int *entries) {
         for (int r = 1; r <= kBatchMaxR; r++) used |= present[r][wc];
         if (!used) continue;
         for (const Tile &cand : kClassCands) {
-            // runs put narrow classes of one column per lane in LDS tiles, which the
-            // one-step objective does not see (4096 grids, 10 steps, with the
-            // classes it then picked 256-column strips for: 5.10 ms, in tiles 4.96)
-            if (b.pairs && wc < 2 && cand.c != 1) continue;
             Tile saved[kBatchMaxR + 1];
             for (int r = 0; r <= kBatchMaxR; r++) saved[r] = b.table[r][wc];
             rc = try_change([&] { for (int r = 1; r <= kBatchMaxR; r++) b.table[r][wc] = cand; },
@@ -733,7 +730,14 @@ static void plan_rounds(const Batch &b, int iters, bool fold, RoundPlan &rp) {
         if (G.rows == 0 || G.cols == 0) continue;
         kind[g] = grid_kind(G, b.table[G.r][width_class(G.cols)].c);
         const bool multi = b.pairs && G.r <= kBatchPairMaxR;
-        tiles[g] = multi && kind[g] == kKindNarrow1;
+        // Rounds of several generations of narrow grids are tiles whatever the
+        // columns per lane of their strips, which then serve rounds of one
+        // generation, as the tuner times them.  us of 10 steps, tiles / strip
+        // pairs, 33 million cells at most: 30 columns r = 1 145 / 846, 8 438 /
+        // 1595; 100 columns 248 / 724, 1149 / 1367; 190 columns 296 / 555, 814 /
+        // 1058.  (One step of strips at 190 columns, one / four columns per
+        // lane: r = 1 181 / 85, 8 152 / 98.)
+        tiles[g] = multi && (kind[g] == kKindNarrow1 || width_class(G.cols) < 2);
         plan[g] = tiles[g] ? tile_plan(iters, kTileGens[G.r]) : multi ? pair_plan(iters) : std::vector<int>(iters, 1);
         rp.pair_grids += multi ? 1 : 0;
         order.push_back(g);

@@ -1,5 +1,5 @@
-"""Narrow grids of a batch in LDS tiles: folds as exact as those of the strip
-items, whatever the grid's size."""
+"""Narrow grids of a batch in LDS tiles: which grids run there, and folds as
+exact as those of the strip items, whatever the grid's size."""
 import ctypes as C
 
 import numpy as np
@@ -7,6 +7,7 @@ import pytest
 
 from muesli4_amd import hip
 from muesli4_amd.hip import BatchGrid, DeviceArray, call
+from oracle import refcpu as R
 
 pytestmark = pytest.mark.gpu
 
@@ -34,8 +35,28 @@ class Grids:
         call("msl_batch_run", self.handle, iters, self.sums.ptr, C.byref(inb))
         return [x.to_host() for x in (self.b if inb.value else self.a)], self.sums.to_host()
 
+    def rounds(self, iters):
+        n = C.c_int()
+        call("msl_batch_run_plan", self.handle, iters, 1, C.byref(n), None, None, None)
+        return n.value
+
+    def set_columns(self, c):
+        for r in range(1, 11):
+            for wc in range(4):
+                call("msl_batch_set_tile", self.handle, r, wc, c, 64)
+
     def close(self):
         call("msl_batch_destroy", self.handle)
+
+
+def _uniform(shapes, seed=3):
+    return [R.fill_uniform_f32(s[0] * s[1], seed + k).reshape(s) for k, s in enumerate(shapes)]
+
+
+def _oracle(x, r, nv, iters):
+    for _ in range(iters):
+        x = R.stencil2d_mean_f32(x, r, nv)
+    return x
 
 
 @pytest.mark.parametrize("iters", [3, 6])
@@ -52,3 +73,34 @@ def test_fold_of_tile_grids_keeps_its_precision(iters):
     for x, s, shape in zip(states, sums, shapes):
         ref = float(np.sum(x.astype(np.float64)))
         assert abs(s - ref) <= FOLD_TOL * float(np.sum(np.abs(x.astype(np.float64)))), (shape, s, ref)
+
+
+def test_narrow_grids_run_in_tiles_whatever_their_strips(tmp_path):
+    """The columns per lane of a narrow class shape its one-generation rounds
+    only, also when they come from a saved table."""
+    print("[case] batch narrow grids with either strip width", flush=True)
+    hip.init(0)
+    shapes, radii, iters = [(70, 40), (33, 95), (120, 100), (65, 191), (9, 5)], [1, 2, 4, 3, 5], 12
+    grids = _uniform(shapes)
+    b = Grids(grids, radii, 0.5)
+    rounds = b.rounds(iters)
+    assert rounds == 4  # three generations a round at r = 2..5 (in strips: six pairs)
+    for c in (1, 4):
+        b.set_columns(c)
+        assert b.rounds(iters) == rounds
+    table = tmp_path / "tiles.txt"
+    n = C.c_int()
+    call("msl_batch_autotune", b.handle, str(table).encode(), C.byref(n))
+    assert n.value == len(radii)
+    lines = [ln.split() for ln in table.read_text().splitlines()]
+    for ln in lines:
+        if ln[0] == "tile":
+            ln[3] = "4"
+    table.write_text("".join(" ".join(ln) + "\n" for ln in lines))
+    call("msl_batch_autotune", b.handle, str(table).encode(), C.byref(n))
+    assert n.value < 0  # loaded
+    assert b.rounds(iters) == rounds
+    states, _ = b.run(iters)
+    b.close()
+    for x, got, r in zip(grids, states, radii):
+        np.testing.assert_array_equal(got, _oracle(x, r, 0.5, iters), err_msg=f"r={r}")
