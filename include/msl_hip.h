@@ -149,6 +149,14 @@ int msl_stencil2d_mean_iterate_f32(float *d_a, float *d_b, int rows, int cols, i
  * skeleton call); it lets callers and tests see which kernels run.      */
 int msl_stencil2d_mean_iterate_plan(const float *d_a, const float *d_b, int rows, int cols, int r, int iters,
                                     int *h_gens, int capacity, int *h_launches);
+/* The kernel of each of those launches (a single msl_stencil2d_mean_f32 step
+ * runs the one of iters = 1).                                            */
+#define MSL_MEAN_MARCH 0  /* one generation, strips marched down the rows     */
+#define MSL_MEAN_WINDOW 1 /* r = 1: up to six generations in register windows */
+#define MSL_MEAN_PAIR 2   /* two generations, strips marched down the rows    */
+#define MSL_MEAN_TILE 3   /* one to six generations in LDS tiles              */
+int msl_stencil2d_mean_iterate_kernels(const float *d_a, const float *d_b, int rows, int cols, int r, int iters,
+                                       int *h_kernels, int capacity, int *h_launches);
 /* Game of Life B3/S23, cells outside are 0 (reference:
  * examples/gameoflife.cpp:18-43 through DM::mapStencilMM,
  * src/dm.cpp:615-1208).                                                 */

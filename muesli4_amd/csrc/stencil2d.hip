@@ -121,8 +121,19 @@ inline int row_mode(const T *in, const T *out, int cols) {
 // multiples, where the tiles' loads meet in few memory channels (r = 5,
 // 4096 x 4100 32.9 / 30.8, 4096^2 32.0 / 33.5).
 constexpr long kTile1WideCells = 9L << 19;
+
+// Whether the environment sets the shape of the march (strip_shape): the mean
+// blur then marches at every size.
+static bool march_forced() {
+    static const bool forced = [] {
+        const int c = tune_int("MSL_STRIP_C", 0);
+        return tune_int("MSL_STRIP_SEG", 0) > 0 || c == 1 || c == 4;
+    }();
+    return forced;
+}
+
 static bool tile1_default(const float *in, const float *out, int r, int rows, int cols) {
-    if (r < 2) return false;
+    if (r < 2 || march_forced()) return false;
     const bool march = (r == 10 && row_mode(in, out, cols) == kAligned) || (r <= 6 && cols % 1024 == 0);
     return (long)rows * cols <= (r <= 4 ? 3L << 20 : march ? 10L << 20 : 25L << 20);
 }
@@ -153,7 +164,8 @@ inline StripShape strip_shape(int rows, int cols, int r, int seg, bool streamed)
     StripShape s;
     const long cus = ctx().num_cus;
     const long strips4 = (cols + kStripW - 1) / kStripW;
-    s.c = r == 1 && strips4 * ((rows + 7) / 8) < 8 * cus ? 1 : 4;
+    s.c = tune_int("MSL_STRIP_C", 0);
+    if (s.c != 1 && s.c != 4) s.c = r == 1 && strips4 * ((rows + 7) / 8) < 8 * cus ? 1 : 4;
     const int sw = 64 * s.c;
     s.strips_x = (cols + sw - 1) / sw;
     if (seg <= 0) seg = tune_int("MSL_STRIP_SEG", 0);
@@ -183,14 +195,10 @@ int launch_strip(typename Pol::T *out, const typename Pol::T *in, int rows, int 
     StripShape s = strip_shape(rows, cols, Pol::R, seg, nt);
     const int blocks = (s.nitems + 3) / 4;
     const int mode = row_mode(in, out, cols);
-    if constexpr (Pol::R == 1) {
-        if (s.c == 1) {
-            strip_stencil_kernel<Pol, kAligned, false, 1><<<blocks, 256, 0, ctx().stream>>>(
-                out, in, rows, cols, nv, s.seg, s.strips_x, s.nitems, pol);
-            return check_launch(name);
-        }
-    }
-    if (mode == kAligned && nt)
+    if (s.c == 1)  // (above R = 1 only where MSL_STRIP_C asks for it)
+        strip_stencil_kernel<Pol, kAligned, false, 1><<<blocks, 256, 0, ctx().stream>>>(out, in, rows, cols, nv, s.seg,
+                                                                                          s.strips_x, s.nitems, pol);
+    else if (mode == kAligned && nt)
         strip_stencil_kernel<Pol, kAligned, true><<<blocks, 256, 0, ctx().stream>>>(out, in, rows, cols, nv, s.seg,
                                                                                       s.strips_x, s.nitems, pol);
     else if (mode == kAligned)
@@ -336,7 +344,7 @@ static std::vector<int> even_plan(int iters, int k) {
 // 4.6).
 static bool mean2_default(int r, int rows, int cols) {
     const size_t bytes = (size_t)rows * cols * sizeof(float);
-    if (r < 4 || r > kMaxMean2R) return false;
+    if (r < (march_forced() ? 2 : 4) || r > kMaxMean2R) return false;
     return r <= 4 ? bytes >= ((size_t)32 << 20) : stream_stores(bytes);
 }
 
@@ -348,9 +356,10 @@ static bool mean2_default(int r, int rows, int cols) {
 // 10 23.8 / 22.2; 2048^2 r = 10 13.0 / 17.7; 500 x 517 r = 3 2.1 / 4.9.
 static bool tile_default(int r, int rows, int cols) {
     const long cells = (long)rows * cols;
-    return r >= 2 && (r <= 3 || cells <= (r <= 8 ? 1L << 24 : 9L << 19));
+    return r >= 2 && !march_forced() && (r <= 3 || cells <= (r <= 8 ? 1L << 24 : 9L << 19));
 }
 
+// Launches of an iteration; kLaunchStep is one generation by mean_step.
 enum LaunchKind { kLaunchStep, kLaunchMulti3, kLaunchPair, kLaunchTile };
 
 struct MeanLaunch {
@@ -510,6 +519,28 @@ int msl_stencil2d_mean_iterate_plan(const float *d_a, const float *d_b, int rows
     *h_launches = (int)plan.size();
     MSL_REQUIRE(h_gens != nullptr || plan.empty() || capacity == 0, "msl_stencil2d_mean_iterate_plan: null output");
     for (size_t k = 0; k < plan.size() && (int)k < capacity; k++) h_gens[k] = plan[k].gens;
+    return MSL_OK;
+}
+
+int msl_stencil2d_mean_iterate_kernels(const float *d_a, const float *d_b, int rows, int cols, int r, int iters,
+                                       int *h_kernels, int capacity, int *h_launches) {
+    MSL_REQUIRE(iters >= 0 && rows >= 0 && cols >= 0, "msl_stencil2d_mean_iterate_kernels: negative argument");
+    MSL_REQUIRE(r >= 1 && r <= kMaxMeanR, "msl_stencil2d_mean_iterate_kernels: radius must be in [1, 16]");
+    MSL_REQUIRE(h_launches != nullptr && capacity >= 0, "msl_stencil2d_mean_iterate_kernels: bad output arguments");
+    std::vector<MeanLaunch> plan;
+    if (iters > 0 && rows > 0 && cols > 0) plan = mean_iterate_plan(d_a, d_b, rows, cols, r, iters);
+    *h_launches = (int)plan.size();
+    MSL_REQUIRE(h_kernels != nullptr || plan.empty() || capacity == 0, "msl_stencil2d_mean_iterate_kernels: null output");
+    for (size_t k = 0; k < plan.size() && (int)k < capacity; k++) {
+        switch (plan[k].kind) {
+            case kLaunchStep:
+                h_kernels[k] = tile1_default(d_a, d_b, r, rows, cols) ? MSL_MEAN_TILE : MSL_MEAN_MARCH;
+                break;
+            case kLaunchMulti3: h_kernels[k] = MSL_MEAN_WINDOW; break;
+            case kLaunchPair: h_kernels[k] = MSL_MEAN_PAIR; break;
+            case kLaunchTile: h_kernels[k] = MSL_MEAN_TILE; break;
+        }
+    }
     return MSL_OK;
 }
 

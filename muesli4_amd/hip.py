@@ -105,6 +105,7 @@ SIGNATURES = {
     "msl_stencil2d_mean_f32": [p, p, i32, i32, i32, f32],
     "msl_stencil2d_mean_iterate_f32": [p, p, i32, i32, i32, f32, i32, PI],
     "msl_stencil2d_mean_iterate_plan": [p, p, i32, i32, i32, i32, PI, i32, PI],
+    "msl_stencil2d_mean_iterate_kernels": [p, p, i32, i32, i32, i32, PI, i32, PI],
     "msl_gol_i32": [p, p, i32, i32],
     "msl_gol_iterate_i32": [p, p, i32, i32, i32, PI],
     "msl_heat7_f32": [p, p, i32, i32, i32, f32],
@@ -190,6 +191,18 @@ def mean_iterate_plan(d_a, d_b, rows: int, cols: int, r: int, iters: int) -> lis
     n = C.c_int()
     call("msl_stencil2d_mean_iterate_plan", d_a, d_b, rows, cols, r, iters, gens, cap, C.byref(n))
     return list(gens)[: n.value]
+
+
+MEAN_KERNELS = ("march", "window", "pair", "tile")  # MSL_MEAN_*
+
+
+def mean_iterate_kernels(d_a, d_b, rows: int, cols: int, r: int, iters: int) -> list:
+    """Kernels of the launches of mean_iterate_plan, as MEAN_KERNELS names."""
+    cap = max(iters, 1)
+    kinds = (C.c_int * cap)()
+    n = C.c_int()
+    call("msl_stencil2d_mean_iterate_kernels", d_a, d_b, rows, cols, r, iters, kinds, cap, C.byref(n))
+    return [MEAN_KERNELS[k] for k in list(kinds)[: n.value]]
 
 
 def heat_iterate_plan(nx: int, ny: int, nz: int, iters: int, every: int) -> list:

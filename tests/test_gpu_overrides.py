@@ -1,6 +1,9 @@
 """Environment overrides of the kernel choice: results stay bit-identical to
 the oracle under each of them."""
 import ctypes as C
+import os
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -40,3 +43,39 @@ def test_generation_overrides_other_than_1_and_2(value, monkeypatch):
     np.testing.assert_array_equal((b if inb.value else a).to_host(), want)
     assert [hip.heat_iterate_plan(nx, ny, nz, iters, 0),
             hip.mean_iterate_plan(None, None, 90, 130, 3, iters)] == plans
+
+
+MARCH = r"""
+import numpy as np
+from muesli4_amd import hip
+from muesli4_amd.hip import DeviceArray, call
+from oracle import refcpu as R
+import ctypes as C
+hip.init(0)
+for r in (1, 2, 3, 5, 7, 9, 10, 12, 16):
+    for shape in [(200, 301), (130, 260), (333, 3), (1, 700), (70, 1028)]:
+        n = shape[0] * shape[1]
+        x = R.fill_uniform_f32(n, 3 + r).reshape(shape)
+        a, b = DeviceArray.from_host(x), DeviceArray(shape, np.float32)
+        assert hip.mean_iterate_kernels(a.ptr, b.ptr, *shape, r, 1) == ["march"], (shape, r)
+        call("msl_stencil2d_mean_f32", b.ptr, a.ptr, *shape, r, 1.5)
+        np.testing.assert_array_equal(b.to_host(), R.stencil2d_mean_f32(x, r, 1.5), err_msg=f"{shape} r={r}")
+        inb = C.c_int()
+        call("msl_stencil2d_mean_iterate_f32", a.ptr, b.ptr, *shape, r, 1.5, 3, C.byref(inb))
+        want = x
+        for _ in range(3):
+            want = R.stencil2d_mean_f32(want, r, 1.5)
+        np.testing.assert_array_equal(b.to_host(), want, err_msg=f"{shape} r={r} x3")
+"""
+
+
+# The overrides of the march's shape (read once per process) march at every
+# size: every radius and row mode of it, with both strip widths.
+@pytest.mark.parametrize("env", [{"MSL_STRIP_SEG": "24"}, {"MSL_STRIP_C": "4"}, {"MSL_STRIP_C": "1"},
+                                 {"MSL_STRIP_C": "1", "MSL_STRIP_SEG": "7"}])
+def test_march_shape_overrides(env):
+    print(f"[case] march with {env}", flush=True)
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    res = subprocess.run([sys.executable, "-c", MARCH], cwd=root, env={**os.environ, **env}, stdout=subprocess.PIPE,
+                         stderr=subprocess.STDOUT, text=True, timeout=100)
+    assert res.returncode == 0, res.stdout
