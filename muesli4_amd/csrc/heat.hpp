@@ -143,17 +143,22 @@ __device__ __forceinline__ void heat7_march(float *__restrict__ out, const float
 // Generation-1 cells outside the cube are nv, as the second step reads them.
 // Every cell is computed in the one-step order, so the result is
 // bit-identical to two single steps.  kSingle: generation 1 only, of the same
-// tile (the odd step of a job whose items are laid out for two).
+// tile (the odd step of a job whose items are laid out for two).  kResidual:
+// max |generation 2 - generation 1| into *dmax.  kFull: every division in its
+// full form (on thin cubes, which wait for memory, 5-10 % faster than the
+// short form and its check).
 constexpr int kT2X = kTX - 4;  // output columns of a two-generation wave tile
 // Output rows of a two-generation wave tile: 5 rows (90 VGPRs, five waves
 // per SIMD) beat 8 (124, four) although the y halo grows from 4/8 to 4/5
 // (200 iterations of a 320^3 cube alone: 8 rows 7.13 ms, 5 6.90).  The serving
-// engine's items use it; single cubes run heat_tile.hip and heat_pair.hip.
+// engine's items use it, and large thin cubes (heat_way); other cubes run
+// heat_tile.hip and heat_pair.hip.
 constexpr int kT2Y = 5;
 
-template <bool kSingle>
+template <bool kSingle, bool kFull = false, bool kResidual = false, bool NT = true>
 __device__ __forceinline__ void heat7x2_march(float *__restrict__ out, const float *__restrict__ in, int nx, int ny,
-                                              int nz, float nv, int x0, int y0, int z0, int z1) {
+                                              int nz, float nv, int x0, int y0, int z0, int z1,
+                                              float *dmax = nullptr) {
     constexpr int NI = kT2Y + 4;  // input rows y0-2 .. y0+kT2Y+1
     constexpr int N1 = kT2Y + 2;  // generation-1 rows y0-1 .. y0+kT2Y
     const int lane = threadIdx.x & 63;
@@ -202,6 +207,11 @@ __device__ __forceinline__ void heat7x2_march(float *__restrict__ out, const flo
     // sums are still in registers).
     auto divide = [&](auto &v, auto n) {
         constexpr int N = decltype(n)::value;
+        if constexpr (kFull) {
+#pragma unroll
+            for (int j = 0; j < N; j++) v[j] = div6_plus0(v[j]);
+            return;
+        }
         float q[N];
         bool suspect = false;
 #pragma unroll
@@ -260,7 +270,14 @@ __device__ __forceinline__ void heat7x2_march(float *__restrict__ out, const flo
                 // output row y0+j is input row j+2: stored when in the cube
                 if (zo >= z0 && zo < z1 && lane >= 2 && lane <= 61 && ((iok >> (j + 2)) & 1u)) {
                     float *o = reinterpret_cast<float *>(op + ioff[j + 2]);
-                    __builtin_nontemporal_store(v, o);
+                    if constexpr (NT)
+                        __builtin_nontemporal_store(v, o);
+                    else
+                        *o = v;
+                    if constexpr (kResidual) {
+                        const float d = fabsf(__fsub_rn(v, g1[j + 1][tc]));
+                        *dmax = d > *dmax ? d : *dmax;
+                    }
                 }
             }
         }

@@ -195,12 +195,22 @@ __global__ __launch_bounds__(kHeatThreads) __attribute__((amdgpu_waves_per_eu(8,
     }
 }
 
+template <int kHY, int kHZ>
+static long tile_blocks(int nx, int ny, int nz, int steps) {
+    const int tx = kHX - 2 * steps, ty = kHY - 2 * steps, tz = kHZ - 2 * steps;
+    return (long)((nx + tx - 1) / tx) * ((ny + ty - 1) / ty) * ((nz + tz - 1) / tz);
+}
+
+long heat_tile_blocks(int nx, int ny, int nz, int steps, bool small) {
+    return small ? tile_blocks<16, 12>(nx, ny, nz, steps) : tile_blocks<24, 20>(nx, ny, nz, steps);
+}
+
 template <int kHY, int kHZ, int kHZP>
 static int launch_heat_tile(float *out, const float *in, int nx, int ny, int nz, float nv, int steps, float *maxdiff) {
     const int tx = kHX - 2 * steps, ty = kHY - 2 * steps, tz = kHZ - 2 * steps;
     MSL_REQUIRE(steps >= 1 && tz >= 1, "msl_heat7_f32: generations per launch out of range");
     const int tiles_x = (nx + tx - 1) / tx, tiles_y = (ny + ty - 1) / ty;
-    const long blocks = (long)tiles_x * tiles_y * ((nz + tz - 1) / tz);
+    const long blocks = tile_blocks<kHY, kHZ>(nx, ny, nz, steps);
     MSL_REQUIRE(blocks <= INT32_MAX, "msl_heat7_f32: cube too large");
     if (maxdiff)
         heat_tile_kernel<kHY, kHZ, kHZP, true><<<(int)blocks, kHeatThreads, 0, ctx().stream>>>(

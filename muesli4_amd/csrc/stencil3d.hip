@@ -24,9 +24,10 @@
 
 namespace mslhip {
 
-// One wave per (64 x kTY column tile, z-segment); four independent waves per
-// workgroup, no LDS and no barrier.
-template <bool kResidual, bool NT>
+// One wave per (64 x kTY column tile, z-segment), or per kT2X x kT2Y tile of
+// two generations (kPair); four independent waves per workgroup, no LDS and no
+// barrier.
+template <bool kPair, bool kResidual, bool NT>
 __global__ __launch_bounds__(256) void heat7_kernel(float *__restrict__ out, const float *__restrict__ in, int nx,
                                                     int ny, int nz, float nv, int zseg, int xtiles, int ytiles,
                                                     int nitems, float *__restrict__ maxdiff) {
@@ -39,7 +40,11 @@ __global__ __launch_bounds__(256) void heat7_kernel(float *__restrict__ out, con
         const int yt = rest % ytiles;
         const int zs = rest / ytiles;
         const int z0 = zs * zseg;
-        heat7_march<kResidual, NT>(out, in, nx, ny, nz, nv, xt * kTX, yt * kTY, z0, min(z0 + zseg, nz), &dmax);
+        const int z1 = min(z0 + zseg, nz);
+        if constexpr (kPair)
+            heat7x2_march<false, true, kResidual, NT>(out, in, nx, ny, nz, nv, xt * kT2X, yt * kT2Y, z0, z1, &dmax);
+        else
+            heat7_march<kResidual, NT>(out, in, nx, ny, nz, nv, xt * kTX, yt * kTY, z0, z1, &dmax);
     }
     if (kResidual) {
         __shared__ float wmax[4];
@@ -61,7 +66,7 @@ struct HeatShape {
     int zseg, xtiles, ytiles, zsegs, nitems;
 };
 
-inline HeatShape heat_shape(int nx, int ny, int nz) {
+inline HeatShape heat_shape(int nx, int ny, int nz, bool pair) {
     HeatShape s;
     s.xtiles = (nx + kTX - 1) / kTX;
     s.ytiles = (ny + kTY - 1) / kTY;
@@ -75,8 +80,49 @@ inline HeatShape heat_shape(int nx, int ny, int nz) {
     if (int z = tune_int("MSL_HEAT_ZSEG", 0)) zseg = z;
     s.zseg = zseg;
     s.zsegs = (nz + zseg - 1) / zseg;
+    if (pair) {
+        s.xtiles = (nx + kT2X - 1) / kT2X;
+        s.ytiles = (ny + kT2Y - 1) / kT2Y;
+    }
     s.nitems = s.xtiles * s.ytiles * s.zsegs;
     return s;
+}
+
+template <bool kPair>
+static int launch_heat_march(float *out, const float *in, int nx, int ny, int nz, float nv, float *maxdiff) {
+    const HeatShape s = heat_shape(nx, ny, nz, kPair);
+    const bool nt = stream_stores((size_t)nx * ny * nz * sizeof(float));
+    const int blocks = (s.nitems + 3) / 4;
+    if (maxdiff && nt)
+        heat7_kernel<kPair, true, true><<<blocks, 256, 0, ctx().stream>>>(out, in, nx, ny, nz, nv, s.zseg, s.xtiles,
+                                                                          s.ytiles, s.nitems, maxdiff);
+    else if (maxdiff)
+        heat7_kernel<kPair, true, false><<<blocks, 256, 0, ctx().stream>>>(out, in, nx, ny, nz, nv, s.zseg, s.xtiles,
+                                                                           s.ytiles, s.nitems, maxdiff);
+    else if (nt)
+        heat7_kernel<kPair, false, true><<<blocks, 256, 0, ctx().stream>>>(out, in, nx, ny, nz, nv, s.zseg, s.xtiles,
+                                                                           s.ytiles, s.nitems, nullptr);
+    else
+        heat7_kernel<kPair, false, false><<<blocks, 256, 0, ctx().stream>>>(out, in, nx, ny, nz, nv, s.zseg, s.xtiles,
+                                                                            s.ytiles, s.nitems, nullptr);
+    return check_launch("msl_heat7_f32");
+}
+
+// Times of a launch in us, fitted to 340 cubes of 0.2 to 4.2 million cells with
+// an extent of 1 to 24 (both within 12 % on average): a tile costs the same
+// however few of its planes or rows lie in the cube, the march only the planes
+// and rows that do.
+static double heat_march_us(int nx, int ny, int nz) {
+    const HeatShape s = heat_shape(nx, ny, nz, false);
+    auto whole = [](int planes) { return (planes + kP - 1) / kP * kP; };
+    const double chain = whole(std::min(s.zseg, nz));
+    const double planes = (double)(s.zsegs - 1) * whole(s.zseg) + whole(nz - (s.zsegs - 1) * s.zseg);
+    return 3.74 + std::max(0.566 * chain, 3.22e-4 * s.xtiles * s.ytiles * planes);
+}
+static double heat_tile_us(int nx, int ny, int nz, int gens, bool small, bool residual) {
+    const double blocks = (double)heat_tile_blocks(nx, ny, nz, gens, small);
+    const double each = (small ? 0.00582 : 0.0105) * (1.0 + 0.5 * (gens - 1)) + (residual ? (small ? 0.010 : 0.006) : 0.0);
+    return (small ? 3.48 : 6.64) + each * blocks;
 }
 
 // How a cube's iterations run.  us per generation, one-step march / small
@@ -85,16 +131,33 @@ inline HeatShape heat_shape(int nx, int ny, int nz) {
 // 128^3 14.1 / 5.2 / 5.4 / 5.4, 150^3 14.6 / 8.5 / 6.9 / 8.7, 200^3 17.8 / 14.9
 // / 11.1 / 10.8, 256^3 22.6 / 27.6 / 18.4 / 14.0, 512^3 215 / 242 / 138 / 106
 // (tiles at the generations per launch given here).
+// Thin cubes leave most of a tile or of the pair kernel's planes empty: up to
+// 4.2 million cells they march wherever that is modelled as faster (2000 x
+// 2000 x 1, tiles / march: 47 / 15; 1000 x 1000 x 3 14 / 9), and larger ones run
+// the march of one wave per tile, two generations per launch where the cube
+// exceeds 64 MiB (pair kernel / that march, 25 million cells: 5000 x 1 x 5000
+// 235 / 74, 2000 x 10 x 1250 33 / 29, 2000 x 12 x 1041 29 / 29; 16 x 300 x 5208 63 /
+// 60, 32 x 300 x 2604 35 / 36; 2000 x 6250 x 2 36 / 31, 2000 x 3125 x 4 25 / 27).
+enum HeatKernel { kHeatMarch, kHeatSmallTile, kHeatTile, kHeatPair, kHeatMarchPair };
 struct HeatWay {
-    int gens;          // most generations per launch
-    bool tile, small;  // tile kernel and its region; else the pair kernel
+    int gens;  // most generations per launch
+    HeatKernel kernel;
 };
+constexpr size_t kHeatTileCells = 4200000, kHeatSmallTileCells = 900000;
+constexpr size_t kHeatMarchPairMinBytes = (size_t)64 << 20;
+
 static HeatWay heat_way(int nx, int ny, int nz) {
     const size_t cells = (size_t)nx * ny * nz;
-    if (cells <= 350000) return HeatWay{4, true, true};
-    if (cells <= 900000) return HeatWay{3, true, true};
-    if (cells <= 4200000) return HeatWay{3, true, false};
-    return HeatWay{2, false, false};
+    if (cells <= kHeatTileCells) {
+        const bool small = cells <= kHeatSmallTileCells;
+        const int gens = cells <= 350000 ? 4 : 3;
+        if (heat_tile_us(nx, ny, nz, gens, small, false) < gens * heat_march_us(nx, ny, nz))
+            return HeatWay{gens, small ? kHeatSmallTile : kHeatTile};
+        return HeatWay{1, kHeatMarch};
+    }
+    if (nx < 32 || ny <= 10 || nz <= 2)
+        return cells * sizeof(float) > kHeatMarchPairMinBytes ? HeatWay{2, kHeatMarchPair} : HeatWay{1, kHeatMarch};
+    return HeatWay{2, kHeatPair};
 }
 
 int heat_step(float *out, const float *in, int nx, int ny, int nz, float nv, float *maxdiff) {
@@ -105,24 +168,12 @@ int heat_step(float *out, const float *in, int nx, int ny, int nz, float nv, flo
     MSL_REQUIRE((int64_t)nx * ny < ((int64_t)1 << 30), "msl_heat7_f32: plane of 2^30 cells or more");
     if (nx == 0 || ny == 0 || nz == 0) return MSL_OK;
     MSL_REQUIRE(out && in && out != in, "msl_heat7_f32: null or aliased buffers");
-    const HeatWay way = heat_way(nx, ny, nz);
-    if (way.tile) return heat_tile_step(out, in, nx, ny, nz, nv, 1, way.small, maxdiff);
-    HeatShape s = heat_shape(nx, ny, nz);
-    const bool nt = stream_stores((size_t)nx * ny * nz * sizeof(float));
-    const int blocks = (s.nitems + 3) / 4;
-    if (maxdiff && nt)
-        heat7_kernel<true, true><<<blocks, 256, 0, ctx().stream>>>(out, in, nx, ny, nz, nv, s.zseg, s.xtiles, s.ytiles,
-                                                                   s.nitems, maxdiff);
-    else if (maxdiff)
-        heat7_kernel<true, false><<<blocks, 256, 0, ctx().stream>>>(out, in, nx, ny, nz, nv, s.zseg, s.xtiles, s.ytiles,
-                                                                    s.nitems, maxdiff);
-    else if (nt)
-        heat7_kernel<false, true><<<blocks, 256, 0, ctx().stream>>>(out, in, nx, ny, nz, nv, s.zseg, s.xtiles, s.ytiles,
-                                                                    s.nitems, nullptr);
-    else
-        heat7_kernel<false, false><<<blocks, 256, 0, ctx().stream>>>(out, in, nx, ny, nz, nv, s.zseg, s.xtiles,
-                                                                     s.ytiles, s.nitems, nullptr);
-    return check_launch("msl_heat7_f32");
+    const size_t cells = (size_t)nx * ny * nz;
+    const bool small = cells <= kHeatSmallTileCells;
+    if (cells <= kHeatTileCells &&
+        1.05 * heat_tile_us(nx, ny, nz, 1, small, maxdiff != nullptr) < heat_march_us(nx, ny, nz))
+        return heat_tile_step(out, in, nx, ny, nz, nv, 1, small, maxdiff);
+    return launch_heat_march<false>(out, in, nx, ny, nz, nv, maxdiff);
 }
 
 // Small fill used instead of hipMemsetAsync so that captured graphs contain
@@ -233,7 +284,7 @@ int msl_heat7_iterate_f32(float *d_a, float *d_b, int nx, int ny, int nz, float 
         }
         auto is_res = [&](int it) { return residual_every > 0 && ((it + 1) % residual_every == 0); };
         const std::vector<int> plan = heat_iterate_plan(nx, ny, nz, iters, residual_every);
-        const HeatWay way = heat_way(nx, ny, nz);
+        const HeatKernel kernel = env ? kHeatPair : heat_way(nx, ny, nz).kernel;
         int k = 0, it = 0;
         for (size_t j = 0; j < plan.size() && brc == MSL_OK; j++) {
             float *src = (j & 1) ? d_b : d_a;
@@ -243,10 +294,12 @@ int msl_heat7_iterate_f32(float *d_a, float *d_b, int nx, int ny, int nz, float 
             float *maxdiff = res ? d_res + (k++) : nullptr;
             if (plan[j] == 1)
                 brc = heat_step(dst, src, nx, ny, nz, nv, maxdiff);
-            else if (way.tile && env == 0)
-                brc = heat_tile_step(dst, src, nx, ny, nz, nv, plan[j], way.small, maxdiff);
-            else
+            else if (kernel == kHeatPair)
                 brc = heat_pair_step(dst, src, nx, ny, nz, nv, maxdiff);
+            else if (kernel == kHeatMarchPair)
+                brc = launch_heat_march<true>(dst, src, nx, ny, nz, nv, maxdiff);
+            else
+                brc = heat_tile_step(dst, src, nx, ny, nz, nv, plan[j], kernel == kHeatSmallTile, maxdiff);
         }
         void *g = nullptr;
         int erc = msl_graph_end(&g);
