@@ -132,8 +132,30 @@ static bool march_forced() {
     return forced;
 }
 
+// Grids of few rows: a tile costs about the same however few of its rows lie
+// in the grid, a strip only the rows that do, so once there are several tiles
+// per CU the march wins.  us per step, march / tile: 1 x 300000 r = 2 3.5 / 9.1,
+// 10 8.7 / 17.4; 3 x 100000 4.0 / 4.7, 9.6 / 7.6; 4 x 750000 6.8 / 20.3, 19.5 /
+// 40.4; 16 x 187500 6.8 / 8.1, 17.0 / 15.4; 24 x 125000 6.0 / 6.9, 17.1 / 12.3;
+// r = 13 8 x 375000 24.7 / 24.4, 10 x 2000000 94 / 122, 12 x 1666666 102 / 104.
+static bool thin_step(int rows, int cols, int r) {
+    const int tiles = cols / (r > 10 ? 128 - 2 * r : 64 - 2 * r), cus = ctx().num_cus;
+    return tiles >= 8 * cus && rows <= (r <= 10 ? 16 : (tiles >= 48 * cus ? 12 : 8));
+}
+
+// The same for iterations, whose tiles take several generations at once.  us
+// per generation, march / tile: 1 x 300000 r = 2 3.8 / 5.8, 10 9.1 / 17.9; 2 x
+// 150000 4.4 / 3.6, 9.5 / 10.6; 6 x 500000 6.3 / 10.4, 12.7 / 29.5; 10 x 300000
+// 7.6 / 6.7, 14.7 / 21.4; 12 x 250000 8.0 / 6.3, 15.5 / 18.7; 16 x 187500 8.5 /
+// 5.1, 17.4 / 15.8; two-generation march: 8 x 2500000 r = 2 18 / 44, 16 x 1250000 15
+// / 25, 24 x 833333 20 / 20.
+static bool thin_iterate(int rows, int cols, int r) {
+    const int tiles = cols / (64 - 2 * r), cus = ctx().num_cus;
+    return tiles >= 16 * cus && rows <= (tiles >= 64 * cus ? 16 : (r >= 8 ? 12 : 8));
+}
+
 static bool tile1_default(const float *in, const float *out, int r, int rows, int cols) {
-    if (r < 2 || march_forced()) return false;
+    if (r < 2 || march_forced() || thin_step(rows, cols, r)) return false;
     const bool march = (r == 10 && row_mode(in, out, cols) == kAligned) || (r <= 6 && cols % 1024 == 0);
     return (long)rows * cols <= (r <= 4 ? 3L << 20 : march ? 10L << 20 : 25L << 20);
 }
@@ -337,26 +359,27 @@ static std::vector<int> even_plan(int iters, int k) {
 }
 
 // Whether iterations of radius r run two generations per launch by default.
-// Measured (GB/s, one vs two generations per launch): radius 4 gains from
-// 4096^2 on, radii 5-7 only on grids streamed from HBM (8192^2: r = 5 4.7 ->
-// 7.2, r = 7 4.5 -> 6.1); on grids that stay in the Infinity Cache their longer
-// halo recomputation costs more than the saved traffic (5792^2: r = 5 5.2 ->
-// 4.6).
+// Measured (GB/s, one vs two generations per launch): radii 2-4 gain from
+// 4096^2 on (2 and 3 are asked for thin grids only, see tile_default), radii 5-7
+// only on grids streamed from HBM (8192^2: r = 5 4.7 -> 7.2, r = 7 4.5 -> 6.1);
+// on grids that stay in the Infinity Cache their longer halo recomputation
+// costs more than the saved traffic (5792^2: r = 5 5.2 -> 4.6).
 static bool mean2_default(int r, int rows, int cols) {
     const size_t bytes = (size_t)rows * cols * sizeof(float);
-    if (r < (march_forced() ? 2 : 4) || r > kMaxMean2R) return false;
+    if (r < 2 || r > kMaxMean2R) return false;
     return r <= 4 ? bytes >= ((size_t)32 << 20) : stream_stores(bytes);
 }
 
 // Grids whose iterations run in tiles (several generations per launch in
-// LDS): radii 2 and 3 always, 4 to 8 up to 2^24 cells, above up to 2^22.2.
+// LDS): radii 2 and 3 at every size, 4 to 8 up to 2^24 cells, above up to 2^22.2,
+// thin grids apart.
 // us per generation of the best tile and of the march: 8192^2 r = 2 42.7 / 59.0,
 // 3 57.8 / 60.3, 4 63.9 / 60.9, 5 79.9 / 63.2; 4096^2 r = 4 17.0 / 19.3, 5 20.4
 // / 26.4, 6 21.6 / 26.0, 8 28.0 / 28.3; 3000^2 r = 8 16.9 / 20.3, 9 20.6 / 22.5,
 // 10 23.8 / 22.2; 2048^2 r = 10 13.0 / 17.7; 500 x 517 r = 3 2.1 / 4.9.
 static bool tile_default(int r, int rows, int cols) {
     const long cells = (long)rows * cols;
-    return r >= 2 && !march_forced() && (r <= 3 || cells <= (r <= 8 ? 1L << 24 : 9L << 19));
+    return r >= 2 && !march_forced() && !thin_iterate(rows, cols, r) && (r <= 3 || cells <= (r <= 8 ? 1L << 24 : 9L << 19));
 }
 
 // Launches of an iteration; kLaunchStep is one generation by mean_step.

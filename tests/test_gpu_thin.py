@@ -58,3 +58,31 @@ def _heat(shape, iters, every):
     got = (b if inb.value else a).to_host()
     np.testing.assert_array_equal(got.view(np.uint32), host.view(np.uint32))
     assert list(res)[: len(want_res)] == want_res
+
+
+# Grids of few rows: the widths on both sides of the rules (for 256 CUs), by
+# the kernel that a single step and an iteration run.
+@pytest.mark.parametrize("r,shape,step,iterate", [
+    (2, (1, 122881), "march", "tile"), (2, (1, 122700), "tile", "tile"),
+    (2, (8, 245761), "march", "march"), (2, (9, 245761), "march", "tile"),
+    (2, (16, 983041), "march", "pair"), (3, (17, 983041), "march", "tile"),
+    (5, (16, 110600), "march", "tile"), (8, (12, 196609), "march", "march"), (8, (13, 196609), "march", "march"),
+    (10, (2, 90113), "march", "march"), (13, (8, 208897), "march", "march"), (13, (9, 208897), "tile", "tile"),
+    (16, (3, 196609), "march", "march"), (4, (5, 1000003), "march", "march"),
+])
+def test_mean_thin_grids(r, shape, step, iterate):
+    print(f"[case] mean r={r} thin {shape}", flush=True)
+    hip.init(0)
+    rows, cols = shape
+    x = R.fill_uniform_f32(rows * cols, 4).reshape(shape)
+    a, b = DeviceArray.from_host(x), DeviceArray(shape, np.float32)
+    assert hip.mean_iterate_kernels(a.ptr, b.ptr, rows, cols, r, 1) == [step]
+    assert hip.mean_iterate_kernels(a.ptr, b.ptr, rows, cols, r, 4)[0] == iterate
+    inb = C.c_int()
+    for iters in (1, 4):
+        a = DeviceArray.from_host(x)
+        call("msl_stencil2d_mean_iterate_f32", a.ptr, b.ptr, rows, cols, r, 1.5, iters, C.byref(inb))
+        want = x
+        for _ in range(iters):
+            want = R.stencil2d_mean_f32(want, r, 1.5)
+        np.testing.assert_array_equal((b if inb.value else a).to_host(), want)
