@@ -377,8 +377,16 @@ static bool mean2_default(int r, int rows, int cols) {
 // 3 57.8 / 60.3, 4 63.9 / 60.9, 5 79.9 / 63.2; 4096^2 r = 4 17.0 / 19.3, 5 20.4
 // / 26.4, 6 21.6 / 26.0, 8 28.0 / 28.3; 3000^2 r = 8 16.9 / 20.3, 9 20.6 / 22.5,
 // 10 23.8 / 22.2; 2048^2 r = 10 13.0 / 17.7; 500 x 517 r = 3 2.1 / 4.9.
+// At radii 2 and 3 from 32 MiB on, rows that one strip of the two-generation
+// march (248 columns) holds stay with it, tiles / march: 125000 x 160 r = 2 20.0 /
+// 18.8, 3 25.4 / 23.2; 250000 x 240 2 47 / 50, 3 69 / 54; 80000 x 250 3 23 / 38.
+static bool one_strip(int r, int rows, int cols) {
+    return r <= 3 && cols >= 150 && cols <= (r == 2 ? 190 : 248) && (long)rows * cols >= 8L << 20;
+}
+
 static bool tile_default(int r, int rows, int cols) {
     const long cells = (long)rows * cols;
+    if (one_strip(r, rows, cols)) return false;
     return r >= 2 && !march_forced() && !thin_iterate(rows, cols, r) && (r <= 3 || cells <= (r <= 8 ? 1L << 24 : 9L << 19));
 }
 
@@ -432,9 +440,16 @@ static std::vector<MeanLaunch> mean_iterate_plan(const float *d_a, const float *
                 best = gens;
             }
         }
+        // one generation by itself: as a single step runs it, but narrow rows in the
+        // tile that was priced, where the step would march mostly empty strips (us
+        // per generation, march / tile: 500000 x 120 r = 3 115 / 70, 1071428 x 56 182 /
+        // 76)
+        const bool step = cols >= 192 || tile1_default(d_a, d_b, r, rows, cols);
         std::vector<MeanLaunch> plan = launches(best, kLaunchTile);
-        for (MeanLaunch &l : plan)
+        for (MeanLaunch &l : plan) {
+            if (l.gens == 1 && !step) l.kind = kLaunchTile;
             if (l.kind == kLaunchTile) l.tile = shape[l.gens];
+        }
         return plan;
     }
     return launches(std::vector<int>(iters, 1), kLaunchStep);

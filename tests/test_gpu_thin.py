@@ -86,3 +86,48 @@ def test_mean_thin_grids(r, shape, step, iterate):
         for _ in range(iters):
             want = R.stencil2d_mean_f32(want, r, 1.5)
         np.testing.assert_array_equal((b if inb.value else a).to_host(), want)
+
+
+# Narrow grids: rows that one strip of the two-generation march holds, and
+# tile plans with launches of one generation.
+@pytest.mark.parametrize("r,shape,kernel", [(2, (70000, 160), "pair"), (2, (70000, 191), "tile"), (3, (40000, 240), "pair"),
+                                            (3, (40000, 250), "tile"), (3, (160000, 56), "tile"), (2, (150000, 60), "tile")])
+@pytest.mark.parametrize("iters", [2, 6])
+def test_mean_narrow_grids(r, shape, kernel, iters):
+    print(f"[case] mean r={r} narrow {shape} x{iters}", flush=True)
+    hip.init(0)
+    rows, cols = shape
+    x = R.fill_uniform_f32(rows * cols, 6).reshape(shape)
+    a, b = DeviceArray.from_host(x), DeviceArray(shape, np.float32)
+    if iters > 2:
+        assert set(hip.mean_iterate_kernels(a.ptr, b.ptr, rows, cols, r, iters)) <= {kernel, "march" if kernel == "pair" else kernel}
+    inb = C.c_int()
+    call("msl_stencil2d_mean_iterate_f32", a.ptr, b.ptr, rows, cols, r, 1.5, iters, C.byref(inb))
+    for _ in range(iters):
+        x = R.stencil2d_mean_f32(x, r, 1.5)
+    np.testing.assert_array_equal((b if inb.value else a).to_host(), x)
+
+
+# Radius-1 windows over the grid's edge: every window shape on narrow and flat
+# grids, odd widths, waves without rows in the grid, cells of either sign and
+# neutral values that are no ordinary number.
+@pytest.mark.parametrize("shape", [(13400, 60), (27000, 52), (27000, 104), (27000, 105), (9000, 117), (1, 30000), (7, 20001),
+                                   (53, 9000), (70000, 1), (40000, 3), (200, 64), (1700, 1801)])
+def test_mean3_edge_windows(shape):
+    print(f"[case] mean3 edges {shape}", flush=True)
+    hip.init(0)
+    rows, cols = shape
+    x = R.fill_uniform_f32(rows * cols, 8).reshape(shape)
+    for data, nv in ((x, 3.5), (x - np.float32(127.5), 0.0), (x, -np.inf), (x, np.nan)):
+        for iters in (3, 6):
+            a, b = DeviceArray.from_host(data), DeviceArray(shape, np.float32)
+            assert hip.mean_iterate_kernels(a.ptr, b.ptr, rows, cols, 1, iters)[0] == "window"
+            inb = C.c_int()
+            call("msl_stencil2d_mean_iterate_f32", a.ptr, b.ptr, rows, cols, 1, nv, iters, C.byref(inb))
+            want = data
+            for _ in range(iters):
+                want = R.stencil2d_mean_f32(want, 1, nv)
+            got = (b if inb.value else a).to_host()
+            np.testing.assert_array_equal(got, want)
+            keep = ~np.isnan(want)
+            np.testing.assert_array_equal(got.view(np.uint32)[keep], want.view(np.uint32)[keep])
