@@ -30,10 +30,14 @@ __device__ __forceinline__ float lane_from_right(float v) {  // lane l gets lane
 // ones compute 1.51, and whole windows of non-negative cells of ordinary size
 // divide in two operations instead of four (div_pair; the block votes once
 // per launch): 6.2 VALU operations per cell and generation of a window, 9.1
-// before.  8 rows per wave keep 59 VGPRs, eight waves per SIMD (16 rows: 104).
-// 8192^2 x 20: 653 -> 533 us (502 with every XCD on a contiguous range), of
-// which 4 passes over HBM take 420 at the rate of a copy and the VALU issue 381;
-// with the next window's cells loaded ahead by persistent blocks 685 (99 VGPRs).
+// before.  8 rows per wave keep 62 VGPRs, eight waves per SIMD (16 rows: 104).
+// 8192^2 x 20: 653 -> 533 us (500 with every XCD on a contiguous range; 527 with
+// cells of either sign, whose windows divide in four operations), of which 4
+// passes over HBM take 420 at the rate of a copy and the VALU issue 381; with the
+// next window's cells loaded ahead by persistent blocks 685 (99 VGPRs).  Windows
+// over the grid's edge keep the cells outside at nv by bits and leave out waves
+// without rows in it (20 iterations, with a select per cell, which became a
+// branch around each division / now: 4096^2 135 / 122 us, 20000 x 250 93 / 61).
 template <int K, int RPW, int NW, int NC>
 __global__ __launch_bounds__(64 * NW) void mean3_multi_kernel(float *__restrict__ out, const float *__restrict__ in,
                                                               int rows, int cols, float nv, int steps, int tiles_x,
@@ -54,15 +58,33 @@ __global__ __launch_bounds__(64 * NW) void mean3_multi_kernel(float *__restrict_
         for (int i = 0; i < RPW; i++) __builtin_memcpy(c[i], p + (size_t)i * cols, sizeof(c[i]));
     } else {
 #pragma unroll
-        for (int i = 0; i < RPW; i++) {
-            const int gy = gy0 + i;
-            const float *row = in + (size_t)min(max(gy, 0), rows - 1) * cols;
+        for (int i = 0; i < RPW; i++)
 #pragma unroll
-            for (int k = 0; k < NC; k++) {
-                const float v = row[min(max(gx + k, 0), cols - 1)];
-                c[i][k] = (unsigned)(gx + k) < (unsigned)cols && (unsigned)gy < (unsigned)rows ? v : nv;
-            }
+            for (int k = 0; k < NC; k++) c[i][k] = nv;
+        const float *p = in + (ptrdiff_t)gy0 * cols + gx;
+        if (gx >= 0 && gx + NC <= cols) {
+#pragma unroll
+            for (int i = 0; i < RPW; i++)
+                if ((unsigned)(gy0 + i) < (unsigned)rows)  // wave-uniform
+                    __builtin_memcpy(c[i], p + (ptrdiff_t)i * cols, sizeof(c[i]));
+        } else if (NC > 1 && gx + NC > 0 && gx < cols) {
+#pragma unroll
+            for (int i = 0; i < RPW; i++)
+#pragma unroll
+                for (int k = 0; k < NC; k++)
+                    if ((unsigned)(gy0 + i) < (unsigned)rows && (unsigned)(gx + k) < (unsigned)cols)
+                        c[i][k] = p[(ptrdiff_t)i * cols + k];
         }
+    }
+    // waves whose rows all lie outside the grid only hand on their edge rows
+    const bool live = gy0 < rows && gy0 + RPW > 0, rows_in = gy0 >= 0 && gy0 + RPW <= rows;
+    // columns outside the grid by bits: as selects they became a branch around
+    // each cell's division
+    uint32_t colmask[NC], nvcol[NC];
+#pragma unroll
+    for (int k = 0; k < NC; k++) {
+        colmask[k] = (unsigned)(gx + k) < (unsigned)cols ? ~0u : 0u;
+        nvcol[k] = ~colmask[k] & __float_as_uint(nv);
     }
     PairDomain domain;
     domain.push(nv);
@@ -101,6 +123,7 @@ __global__ __launch_bounds__(64 * NW) void mean3_multi_kernel(float *__restrict_
                 rs[0][k] = e[wave > 0 ? wave - 1 : 0][1][NC * lane + k];
                 rs[RPW + 1][k] = e[wave < NW - 1 ? wave + 1 : wave][0][NC * lane + k];
             }
+            if (!decltype(kInside)::value && !live) continue;
 #pragma unroll
             for (int i = 1; i < RPW - 1; i++) rowsum(i, rs[i + 1]);
 #pragma unroll
@@ -110,20 +133,26 @@ __global__ __launch_bounds__(64 * NW) void mean3_multi_kernel(float *__restrict_
                     // the column sum without its leading +0
                     const float t = __fadd_rn(__fadd_rn(rs[i][k], rs[i + 1][k]), rs[i + 2][k]);
                     const float q = decltype(kFast)::value ? div_pair(t, pair) : div_plus0(t, denom, rcp);
-                    c[i][k] = decltype(kInside)::value || ((unsigned)(gx + k) < (unsigned)cols &&
-                                                           (unsigned)(gy0 + i) < (unsigned)rows)
-                                  ? q
-                                  : nv;
+                    c[i][k] = decltype(kInside)::value ? q : __uint_as_float((__float_as_uint(q) & colmask[k]) | nvcol[k]);
                 }
+            if (!decltype(kInside)::value && !rows_in) {
+#pragma unroll
+                for (int i = 0; i < RPW; i++)
+                    if ((unsigned)(gy0 + i) >= (unsigned)rows)
+#pragma unroll
+                        for (int k = 0; k < NC; k++) c[i][k] = nv;
+            }
         }
     };
     const bool fast = __syncthreads_and(domain.ok());
-    if (!fast)
-        generations(std::false_type{}, std::false_type{});
-    else if (inside)
+    if (inside && fast)
         generations(std::true_type{}, std::true_type{});
-    else
+    else if (inside)
+        generations(std::true_type{}, std::false_type{});
+    else if (fast)
         generations(std::false_type{}, std::true_type{});
+    else
+        generations(std::false_type{}, std::false_type{});
 
     if (NC * lane >= K && NC * lane < W - K) {
 #pragma unroll
@@ -143,28 +172,32 @@ __global__ __launch_bounds__(64 * NW) void mean3_multi_kernel(float *__restrict_
 }
 
 constexpr int kMean3K = 6;     // generations per launch
-constexpr int kMean3Rows = 8;  // rows per wave, eight waves: windows of 64 rows
-
-template <int NC>
+template <int NC, int RPW, int NW>
 static int launch_mean3(float *out, const float *in, int rows, int cols, float nv, int steps) {
-    constexpr int TW = 64 * NC - 2 * kMean3K, TH = 8 * kMean3Rows - 2 * kMean3K;
+    constexpr int TW = 64 * NC - 2 * kMean3K, TH = NW * RPW - 2 * kMean3K;
     const int tiles_x = (cols + TW - 1) / TW;
     const long blocks = (long)tiles_x * ((rows + TH - 1) / TH);
     MSL_REQUIRE(blocks <= INT32_MAX, "msl_stencil2d_mean_iterate_f32: grid too large");
     const MeanPolicy<1> pol = MeanPolicy<1>::make();
-    mean3_multi_kernel<kMean3K, kMean3Rows, 8, NC><<<(int)blocks, 512, 0, ctx().stream>>>(
+    mean3_multi_kernel<kMean3K, RPW, NW, NC><<<(int)blocks, 64 * NW, 0, ctx().stream>>>(
         out, in, rows, cols, nv, steps, tiles_x, pol.denom, pol.rcp, rcp_pair(9.0));
     return check_launch("msl_stencil2d_mean_iterate_f32");
 }
 
-// 128-column windows once they give two blocks per CU.  20 iterations, 64 /
-// 128 columns: 300^2 28.2 / 39.4 us, 1024^2 35.5 / 44.9, 2048^2 67.4 / 67.9,
-// 3000^2 117 / 109, 4096^2 177 / 162.
+// 128-column windows once they give two blocks per CU, unless 64-column ones
+// cover the rows with fewer lanes.  20 iterations, 64 / 128 columns: 300^2 28.2 /
+// 39.4 us, 1024^2 35.5 / 44.9, 2048^2 67.4 / 67.9, 3000^2 117 / 109, 4096^2 177 /
+// 162.  64-column ones have eight waves of 8 rows while every block finds a CU of
+// its own, else four of 16, which exchange half the edge rows (300^2 24.1 /
+// 25.9 us, 1000^2 29.2 / 29.2, 125000 x 40 80 / 70, 156250 x 128 212 / 171).
 int mean3_multi_step(float *out, const float *in, int rows, int cols, float nv, int steps) {
     MSL_REQUIRE(steps >= 1 && steps <= kMean3K, "msl_stencil2d_mean_iterate_f32: generations per launch out of range");
-    const long wide = (long)((cols + 115) / 116) * ((rows + 51) / 52);
-    return wide >= 2L * ctx().num_cus ? launch_mean3<2>(out, in, rows, cols, nv, steps)
-                                      : launch_mean3<1>(out, in, rows, cols, nv, steps);
+    const long tiles2 = (cols + 115) / 116, tiles1 = (cols + 51) / 52;
+    const long trows = (rows + 51) / 52;
+    if (tiles2 * trows >= 2L * ctx().num_cus && 2 * tiles2 <= tiles1)
+        return launch_mean3<2, 8, 8>(out, in, rows, cols, nv, steps);
+    return tiles1 * trows <= ctx().num_cus ? launch_mean3<1, 8, 8>(out, in, rows, cols, nv, steps)
+                                           : launch_mean3<1, 16, 4>(out, in, rows, cols, nv, steps);
 }
 
 }  // namespace mslhip
