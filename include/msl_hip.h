@@ -161,8 +161,9 @@ int msl_stencil2d_mean_iterate_kernels(const float *d_a, const float *d_b, int r
  * examples/gameoflife.cpp:18-43 through DM::mapStencilMM,
  * src/dm.cpp:615-1208).                                                 */
 int msl_gol_i32(int32_t *d_out, const int32_t *d_in, int rows, int cols);
-/* iters generations from d_a, result in d_b for odd iters, else in d_a.  The
- * buffer without the result is left with bit-packed scratch.             */
+/* iters generations from d_a, result in d_b for odd iters, else in d_a.  Odd
+ * counts up to 7 on grids of at most 2^20 cells, and 1 and 3 on larger ones,
+ * leave d_a as it was; otherwise the buffer without the result is scratch.  */
 int msl_gol_iterate_i32(int32_t *d_a, int32_t *d_b, int rows, int cols, int iters, int *h_result_in_b);
 
 /* ------------------------------------------------------------------ */

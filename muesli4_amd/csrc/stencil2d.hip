@@ -331,7 +331,7 @@ constexpr int kMean3Steps = 6;  // most generations per launch of the radius-1 k
 // launch per generation), so the number of launches must have the parity of
 // iters; when it does not, one launch of several generations is split in
 // two (there is one, since launches of one generation each number iters).
-static std::vector<int> generation_plan(int iters, int k) {
+std::vector<int> generation_plan(int iters, int k) {
     std::vector<int> plan;
     for (int done = 0; done < iters; done += plan.back()) plan.push_back(std::min(k, iters - done));
     if ((int)(plan.size() & 1) != (iters & 1)) {
