@@ -208,6 +208,10 @@ int msl_selftest_div_odd_square(int r, uint64_t *h_mismatches);
  * sequence plus the ties-to-even rule for quotients exactly halfway
  * between two subnormals).                                              */
 int msl_selftest_div_six(uint64_t *h_mismatches);
+/* How a kernel of `blocks` workgroups of `threads` is launched (no device
+ * work): in how many launches, and the most threads of one of them.  HIP
+ * takes fewer than 2^32 threads per launch.                               */
+int msl_selftest_launch_split(int64_t blocks, int threads, int *h_launches, int64_t *h_most_threads);
 
 /* ------------------------------------------------------------------ */
 /* Batched mean blur.  No single reference counterpart: it replaces a loop

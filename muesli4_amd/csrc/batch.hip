@@ -858,8 +858,10 @@ static int enqueue_rounds(Batch &b, const RoundPlan &rp, double *d_sums, const R
             batch_round_kernel<true><<<blocks, 256, 0, s>>>(b.d_grids, rg.d_items + rr.off[0], rr.n[0], rg.d_partials,
                                                             rg.d_ctr + 2 * j);
         }
-        if (rr.n[1])
-            batch_tile_kernel<<<rr.n[1], kTileThreads, kTileLds, s>>>(b.d_grids, rg.d_items + rr.off[1]);
+        const int trc = launch_split(rr.n[1], kTileThreads, "msl_batch_run", [&](int first, int count) {
+            batch_tile_kernel<<<count, kTileThreads, kTileLds, s>>>(b.d_grids, rg.d_items + rr.off[1] + first);
+        });
+        if (trc) return trc;
         if (rr.n[2]) {
             const int bpc = std::max(1, std::min(b.blocks_per_cu, b.max_blocks_per_cu));
             const int blocks = std::max(1, std::min((rr.n[2] + 3) / 4, cus * bpc));

@@ -16,9 +16,9 @@ namespace mslhip {
 template <int R, int W, int M>
 __global__ __launch_bounds__(16 * W / M) void blur_tile_kernel(float *__restrict__ out, const float *__restrict__ in,
                                                                int rows, int cols, float nv, int steps, int tile_w,
-                                                               int tile_h, int tiles_x) {
+                                                               int tile_h, int tiles_x, int tile0) {
     extern __shared__ __attribute__((aligned(16))) float lds[];
-    const int tile = (int)xcd_tile(blockIdx.x, gridDim.x);
+    const int tile = tile0 + (int)xcd_tile(blockIdx.x, gridDim.x);
     blur_tile<R, W, M>(out, in, rows, cols, nv, steps, tile_w, tile_h, tile % tiles_x, tile / tiles_x, lds);
 }
 
@@ -28,11 +28,11 @@ static int launch_tile_rw(float *out, const float *in, int rows, int cols, float
     MSL_REQUIRE(tile_w >= 4 && tile_h >= 1 && tile_h + 2 * R * (steps - 1) <= kTileRows,
                 "msl_stencil2d_mean_f32: tile out of range");
     const int tiles_x = (cols + tile_w - 1) / tile_w;
-    const long blocks = (long)tiles_x * ((rows + tile_h - 1) / tile_h);
-    MSL_REQUIRE(blocks <= INT32_MAX, "msl_stencil2d_mean_f32: grid too large");
-    blur_tile_kernel<R, W, M><<<(int)blocks, 16 * W / M, blur_tile_lds(R, W, tile_h, steps), ctx().stream>>>(
-        out, in, rows, cols, nv, steps, tile_w, tile_h, tiles_x);
-    return check_launch("msl_stencil2d_mean_f32");
+    const long blocks = (long)tiles_x * (((long)rows + tile_h - 1) / tile_h);
+    return launch_split(blocks, 16 * W / M, "msl_stencil2d_mean_f32", [&](int first, int count) {
+        blur_tile_kernel<R, W, M><<<count, 16 * W / M, blur_tile_lds(R, W, tile_h, steps), ctx().stream>>>(
+            out, in, rows, cols, nv, steps, tile_w, tile_h, tiles_x, first);
+    });
 }
 
 template <int R>
@@ -85,7 +85,7 @@ TileShape tile_shape(int rows, int cols, int r, int steps) {
                 lat += (hi + rpr - 1) / rpr * (2 * r + 8) + m * (2 * r + 6);
             }
             const double tiles =
-                (double)((cols + tile_w - 1) / tile_w) * (double)((rows + th - 1) / th) / cus;
+                (double)((cols + tile_w - 1) / tile_w) * (double)(((long)rows + th - 1) / th) / cus;
             const double b = tiles <= 1.0 ? 1.0 : 0.5 * (std::ceil(tiles) + tiles);
             const double us = 1.90 + 0.613 * steps + 0.00719 * lat +
                               b * (2.12e-6 * vw + 1.70e-4 * (th + 2 * r * steps) * w + 0.0145 * steps * (w / (4 * m)));

@@ -69,6 +69,29 @@ int tune_int(const char *name, int dflt);
 std::string graph_key(const char *kind, const void *a, const void *b, long p0, long p1, long p2, long p3, long p4);
 int run_cached_graph(const std::string &key, const std::function<int()> &body);
 
+// Most workgroups of one launch: HIP takes fewer than 2^32 threads per launch
+// (MSL_LAUNCH_THREADS in the environment lowers that bound).
+long launch_limit(int threads);
+// Launches workgroups [0, blocks) of a kernel whose grid grows with the data,
+// in as many launches of (first workgroup, count) as that bound asks for.
+template <typename Part>
+int launch_split_plan(long blocks, int threads, const char *name, Part part) {
+    MSL_REQUIRE(blocks <= INT32_MAX, std::string(name) + ": grid too large");
+    const long most = launch_limit(threads);
+    for (long first = 0; first < blocks; first += most) {
+        const int rc = part((int)first, (int)(blocks - first < most ? blocks - first : most));
+        if (rc) return rc;
+    }
+    return MSL_OK;
+}
+template <typename Launch>
+int launch_split(long blocks, int threads, const char *name, Launch launch) {
+    return launch_split_plan(blocks, threads, name, [&](int first, int count) {
+        launch(first, count);
+        return check_launch(name);
+    });
+}
+
 // Number of workgroups that fills the device for a streaming kernel.
 inline int streaming_blocks(size_t work_items, int threads, int per_cu) {
     size_t want = (work_items + threads - 1) / threads;

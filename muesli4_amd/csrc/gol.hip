@@ -44,11 +44,11 @@ __device__ __forceinline__ uint32_t lane_above(uint32_t v) {  // lane l gets lan
 // 4096^2 take 35 us, bit-packed 43; 5 of 1024^2 14.5, 20.
 template <int K, int RPW>
 __global__ __launch_bounds__(256) void gol_window_kernel(int32_t *__restrict__ out, const int32_t *__restrict__ in,
-                                                         int rows, int cols, int steps, int tiles_x) {
+                                                         int rows, int cols, int steps, int tiles_x, int tile0) {
     constexpr int H = 4 * RPW, TW = 64 - 2 * K, TH = H - 2 * K;
     __shared__ uint32_t edge[4][2][64];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int tile = (int)xcd_tile(blockIdx.x, gridDim.x);
+    const int tile = tile0 + (int)xcd_tile(blockIdx.x, gridDim.x);
     const int gx = tile % tiles_x * TW - K + lane;
     const int gy0 = tile / tiles_x * TH - K + wave * RPW;
     const bool colok = (unsigned)gx < (unsigned)cols;
@@ -90,10 +90,10 @@ static int gol_window_step(int32_t *out, const int32_t *in, int rows, int cols, 
     constexpr int TW = 64 - 2 * K, TH = 4 * RPW - 2 * K;
     const int tiles_x = (cols + TW - 1) / TW;
     const long blocks = (long)tiles_x * (((long)rows + TH - 1) / TH);
-    MSL_REQUIRE(blocks <= INT32_MAX, "msl_gol_iterate_i32: grid too large");
     MSL_REQUIRE(steps >= 1 && steps <= K, "msl_gol_iterate_i32: generations per launch out of range");
-    gol_window_kernel<K, RPW><<<(int)blocks, 256, 0, ctx().stream>>>(out, in, rows, cols, steps, tiles_x);
-    return check_launch("msl_gol_iterate_i32");
+    return launch_split(blocks, 256, "msl_gol_iterate_i32", [&](int first, int count) {
+        gol_window_kernel<K, RPW><<<count, 256, 0, ctx().stream>>>(out, in, rows, cols, steps, tiles_x, first);
+    });
 }
 
 // Up to 2^20 cells, where launches bound the run, 8 generations of 64 x 64
@@ -112,9 +112,9 @@ static int gol_windows(int32_t *out, const int32_t *in, int rows, int cols, int 
 constexpr int kFirstRows = 8;
 
 __global__ __launch_bounds__(64) void gol_first_kernel(uint32_t *__restrict__ out, const int32_t *__restrict__ in,
-                                                       int rows, int cols, int words, int tiles_x) {
+                                                       int rows, int cols, int words, int tiles_x, int tile0) {
     const int lane = threadIdx.x;
-    const int tile = (int)xcd_tile(blockIdx.x, gridDim.x);
+    const int tile = tile0 + (int)xcd_tile(blockIdx.x, gridDim.x);
     const int tx = tile % tiles_x, ty = tile / tiles_x;
     const int x = tx * 64 + lane, y0 = ty * kFirstRows;
     const int xl = max(min(x - 1, cols - 1), 0), xc = min(x, cols - 1), xr = min(x + 1, cols - 1);
@@ -168,9 +168,10 @@ static_assert(kBitInner == 2, "the unpacking store writes 64 columns per row");
 
 template <bool kUnpack>
 __global__ __launch_bounds__(64) void gol_bits_kernel(void *__restrict__ out, const uint32_t *__restrict__ in,
-                                                      int rows, int cols, int words, int steps, int tiles_x) {
+                                                      int rows, int cols, int words, int steps, int tiles_x,
+                                                      int tile0) {
     const int lane = threadIdx.x;
-    const int tile = (int)xcd_tile(blockIdx.x, gridDim.x);
+    const int tile = tile0 + (int)xcd_tile(blockIdx.x, gridDim.x);
     const int tx = tile % tiles_x, ty = tile / tiles_x;
     const int w0 = tx * kBitInner - 1;
     const int y = ty * kBitRows - kBitSteps + lane;
@@ -234,14 +235,14 @@ __global__ __launch_bounds__(64) void gol_bits_kernel(void *__restrict__ out, co
 
 static int gol_bits_step(void *out, const uint32_t *in, int rows, int cols, int words, int steps, bool unpack) {
     const int tiles_x = (words + kBitInner - 1) / kBitInner;
-    const long blocks = (long)tiles_x * ((rows + kBitRows - 1) / kBitRows);
-    MSL_REQUIRE(blocks <= INT32_MAX, "msl_gol_iterate_i32: grid too large");
+    const long blocks = (long)tiles_x * (((long)rows + kBitRows - 1) / kBitRows);
     MSL_REQUIRE(steps >= 1 && steps <= kBitSteps, "msl_gol_iterate_i32: generations per launch out of range");
-    if (unpack)
-        gol_bits_kernel<true><<<(int)blocks, 64, 0, ctx().stream>>>(out, in, rows, cols, words, steps, tiles_x);
-    else
-        gol_bits_kernel<false><<<(int)blocks, 64, 0, ctx().stream>>>(out, in, rows, cols, words, steps, tiles_x);
-    return check_launch("msl_gol_iterate_i32");
+    return launch_split(blocks, 64, "msl_gol_iterate_i32", [&](int first, int count) {
+        if (unpack)
+            gol_bits_kernel<true><<<count, 64, 0, ctx().stream>>>(out, in, rows, cols, words, steps, tiles_x, first);
+        else
+            gol_bits_kernel<false><<<count, 64, 0, ctx().stream>>>(out, in, rows, cols, words, steps, tiles_x, first);
+    });
 }
 
 // iters generations from d_a, the result in d_b when iters is odd, else in
@@ -265,11 +266,11 @@ static int gol_run(int32_t *d_a, int32_t *d_b, int rows, int cols, int iters) {
     const int words = (cols + 31) / 32;
     const size_t packed = (size_t)rows * words;
     const int tiles_x = (cols + 63) / 64;
-    const long blocks = (long)tiles_x * ((rows + kFirstRows - 1) / kFirstRows);
-    MSL_REQUIRE(blocks <= INT32_MAX, "msl_gol_iterate_i32: grid too large");
+    const long blocks = (long)tiles_x * (((long)rows + kFirstRows - 1) / kFirstRows);
     uint32_t *src = reinterpret_cast<uint32_t *>(d_b);
-    gol_first_kernel<<<(int)blocks, 64, 0, ctx().stream>>>(src, d_a, rows, cols, words, tiles_x);
-    int rc = check_launch("msl_gol_iterate_i32");
+    int rc = launch_split(blocks, 64, "msl_gol_iterate_i32", [&](int first, int count) {
+        gol_first_kernel<<<count, 64, 0, ctx().stream>>>(src, d_a, rows, cols, words, tiles_x, first);
+    });
     if (rc) return rc;
     uint32_t *home = reinterpret_cast<uint32_t *>(odd ? d_a : d_b);  // the packed grids' buffer
     int left = iters - 1;

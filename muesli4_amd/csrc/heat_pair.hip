@@ -204,7 +204,9 @@ template <int kPQ, int kPY>
 static int launch_heat_pair(float *out, const float *in, int nx, int ny, int nz, float nv, const PairShape &s,
                             float *maxdiff) {
     const long blocks = (long)s.tiles_x * s.tiles_y * ((nz + s.zseg - 1) / s.zseg);
-    MSL_REQUIRE(blocks <= INT32_MAX, "msl_heat7_iterate_f32: cube too large");
+    // (planes of fewer than 2^30 cells, 32 columns and 11 rows or more, which
+    // heat_way asks for here, have at most 1.3 million tiles, in one segment each)
+    MSL_REQUIRE(blocks <= launch_limit(kPairThreads), "msl_heat7_iterate_f32: cube too large");
     const bool nt = stream_stores((size_t)nx * ny * nz * sizeof(float));
     const dim3 grid((unsigned)blocks), threads(kPairThreads);
     hipStream_t st = ctx().stream;

@@ -41,12 +41,12 @@ __device__ __forceinline__ float lane_from_right(float v) {  // lane l gets lane
 template <int K, int RPW, int NW, int NC>
 __global__ __launch_bounds__(64 * NW) void mean3_multi_kernel(float *__restrict__ out, const float *__restrict__ in,
                                                               int rows, int cols, float nv, int steps, int tiles_x,
-                                                              float denom, float rcp, RcpPair pair) {
+                                                              int tile0, float denom, float rcp, RcpPair pair) {
     constexpr int W = 64 * NC, H = NW * RPW, TW = W - 2 * K, TH = H - 2 * K;
     static_assert(K % NC == 0, "a lane's columns are stored together");
     __shared__ float edge[2][NW][2][W];  // double-buffered: one barrier per generation
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const int tile = (int)xcd_tile(blockIdx.x, gridDim.x);
+    const int tile = tile0 + (int)xcd_tile(blockIdx.x, gridDim.x);
     const int tx = tile % tiles_x, ty = tile / tiles_x;
     const int wx = tx * TW - K, wy = ty * TH - K;  // window origin
     const int gx = wx + NC * lane, gy0 = wy + wave * RPW;
@@ -176,12 +176,12 @@ template <int NC, int RPW, int NW>
 static int launch_mean3(float *out, const float *in, int rows, int cols, float nv, int steps) {
     constexpr int TW = 64 * NC - 2 * kMean3K, TH = NW * RPW - 2 * kMean3K;
     const int tiles_x = (cols + TW - 1) / TW;
-    const long blocks = (long)tiles_x * ((rows + TH - 1) / TH);
-    MSL_REQUIRE(blocks <= INT32_MAX, "msl_stencil2d_mean_iterate_f32: grid too large");
+    const long blocks = (long)tiles_x * (((long)rows + TH - 1) / TH);
     const MeanPolicy<1> pol = MeanPolicy<1>::make();
-    mean3_multi_kernel<kMean3K, RPW, NW, NC><<<(int)blocks, 64 * NW, 0, ctx().stream>>>(
-        out, in, rows, cols, nv, steps, tiles_x, pol.denom, pol.rcp, rcp_pair(9.0));
-    return check_launch("msl_stencil2d_mean_iterate_f32");
+    return launch_split(blocks, 64 * NW, "msl_stencil2d_mean_iterate_f32", [&](int first, int count) {
+        mean3_multi_kernel<kMean3K, RPW, NW, NC><<<count, 64 * NW, 0, ctx().stream>>>(
+            out, in, rows, cols, nv, steps, tiles_x, first, pol.denom, pol.rcp, rcp_pair(9.0));
+    });
 }
 
 // 128-column windows once they give two blocks per CU, unless 64-column ones
@@ -193,7 +193,7 @@ static int launch_mean3(float *out, const float *in, int rows, int cols, float n
 int mean3_multi_step(float *out, const float *in, int rows, int cols, float nv, int steps) {
     MSL_REQUIRE(steps >= 1 && steps <= kMean3K, "msl_stencil2d_mean_iterate_f32: generations per launch out of range");
     const long tiles2 = (cols + 115) / 116, tiles1 = (cols + 51) / 52;
-    const long trows = (rows + 51) / 52;
+    const long trows = ((long)rows + 51) / 52;
     if (tiles2 * trows >= 2L * ctx().num_cus && 2 * tiles2 <= tiles1)
         return launch_mean3<2, 8, 8>(out, in, rows, cols, nv, steps);
     return tiles1 * trows <= ctx().num_cus ? launch_mean3<1, 8, 8>(out, in, rows, cols, nv, steps)

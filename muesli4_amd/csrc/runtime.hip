@@ -69,6 +69,14 @@ int tune_int(const char *name, int dflt) {
     return v;
 }
 
+long launch_limit(int threads) {
+    static const long most_threads = [] {
+        const int forced = tune_int("MSL_LAUNCH_THREADS", 0);
+        return forced > 0 ? (long)forced : (1L << 32) - 1;
+    }();
+    return most_threads / threads > 0 ? most_threads / threads : 1;
+}
+
 __global__ void small_copy_kernel(char *__restrict__ dst, const char *__restrict__ src, size_t bytes) {
     for (size_t i = threadIdx.x; i < bytes; i += blockDim.x) dst[i] = src[i];
 }
@@ -346,6 +354,24 @@ int msl_timer_stop(float *h_ms) {
     MSL_HIP_TRY(hipEventSynchronize(g_ctx.t1));
     MSL_HIP_TRY(hipEventElapsedTime(h_ms, g_ctx.t0, g_ctx.t1));
     return MSL_OK;
+}
+
+int msl_selftest_launch_split(int64_t blocks, int threads, int *h_launches, int64_t *h_most_threads) {
+    MSL_REQUIRE(blocks >= 0 && threads >= 1 && threads <= 1024, "msl_selftest_launch_split: bad launch");
+    MSL_REQUIRE(h_launches != nullptr && h_most_threads != nullptr, "msl_selftest_launch_split: null out-pointer");
+    *h_launches = 0;
+    *h_most_threads = 0;
+    int64_t next = 0;
+    bool gapless = true;
+    const int rc = launch_split_plan((long)blocks, threads, "msl_selftest_launch_split", [&](int first, int count) {
+        gapless = gapless && first == next;
+        next = (int64_t)first + count;
+        ++*h_launches;
+        if ((int64_t)count * threads > *h_most_threads) *h_most_threads = (int64_t)count * threads;
+        return MSL_OK;
+    });
+    if (rc) return rc;
+    return gapless && next == blocks ? MSL_OK : fail(MSL_E_STATE, "msl_selftest_launch_split: workgroups left out");
 }
 
 int msl_graph_begin(void) {

@@ -144,9 +144,10 @@ constexpr size_t serve_tile_lds(int w) { return blur_tile_lds(kBatchMaxR, w, kTi
 // the run 31.8 -> 27.0 ms with one workgroup per tile or heat item.
 template <int W, int M>
 __global__ __launch_bounds__(16 * W / M) void serve_blur_kernel(const SBlur *__restrict__ descs,
-                                                                const int *__restrict__ item_desc, int k_launch) {
+                                                                const int *__restrict__ item_desc, int k_launch,
+                                                                int item0) {
     extern __shared__ __attribute__((aligned(16))) float lds[];
-    const int i = (int)xcd_mixed_tile(blockIdx.x, gridDim.x);
+    const int i = item0 + (int)xcd_mixed_tile(blockIdx.x, gridDim.x);
     const SBlur g = descs[__builtin_amdgcn_readfirstlane(item_desc[i])];
     const int gens = min(g.gens, g.steps - k_launch * g.gens);
     if (gens <= 0) return;
@@ -159,8 +160,9 @@ __global__ __launch_bounds__(16 * W / M) void serve_blur_kernel(const SBlur *__r
 // generations, or the last one of an odd count.
 __global__ __launch_bounds__(256) void serve_heat_kernel(const SHeat *__restrict__ descs,
                                                          const int *__restrict__ item_desc, int nitems,
-                                                         int k_launch) {
-    const int i = __builtin_amdgcn_readfirstlane((int)(xcd_mixed_tile(blockIdx.x, gridDim.x) * 4 + (threadIdx.x >> 6)));
+                                                         int k_launch, int block0) {
+    const int i = __builtin_amdgcn_readfirstlane(
+        (int)((block0 + xcd_mixed_tile(blockIdx.x, gridDim.x)) * 4 + (threadIdx.x >> 6)));
     if (i >= nitems) return;
     const int j = __builtin_amdgcn_readfirstlane(item_desc[i]);
     const SHeat g = descs[j];
@@ -447,8 +449,8 @@ static void tile_blur(SJob &J, bool light) {
     J.tiles_x = (s.d1 + J.tile_w - 1) / J.tile_w;
     J.tile_h = std::min((kTileRows - 2 * s.r * (J.gens - 1)) / 8 * 8, 48);
     if (light)
-        while (J.tile_h > 8 && (long)J.tiles_x * ((s.d0 + J.tile_h - 1) / J.tile_h) < ctx().num_cus / 2) J.tile_h -= 8;
-    J.nitems = J.tiles_x * ((s.d0 + J.tile_h - 1) / J.tile_h);
+        while (J.tile_h > 8 && (long)J.tiles_x * ((s.d0 - 1) / J.tile_h + 1) < ctx().num_cus / 2) J.tile_h -= 8;
+    J.nitems = J.tiles_x * ((s.d0 - 1) / J.tile_h + 1);
 }
 
 // A heat job's items of a round: the march handles whole blocks of kP planes
@@ -771,15 +773,20 @@ static int run_round(Server &S, int *did_work) {
         serve_expand_kernel<<<(items[1] + 255) / 256, 256, 0, st>>>(gsh, (int)dh.size(), items[1], R.d_item_desc[1]);
     for (int k = 0; k < std::max(nsub_max[0], nsub_max[1]); k++) {
         if (k < nsub_max[0] && light)
-            serve_blur_kernel<kLightW, kLightM>
-                <<<items[0], 16 * kLightW / kLightM, serve_tile_lds(kLightW), st>>>(
-                    gb, R.d_item_desc[0], k);
+            rc = launch_split(items[0], 16 * kLightW / kLightM, "msl_server round", [&](int first, int count) {
+                serve_blur_kernel<kLightW, kLightM><<<count, 16 * kLightW / kLightM, serve_tile_lds(kLightW), st>>>(
+                    gb, R.d_item_desc[0], k, first);
+            });
         else if (k < nsub_max[0])
-            serve_blur_kernel<kHeavyW, kHeavyM>
-                <<<items[0], 16 * kHeavyW / kHeavyM, serve_tile_lds(kHeavyW), st>>>(
-                    gb, R.d_item_desc[0], k);
-        if (k < nsub_max[1])
-            serve_heat_kernel<<<(items[1] + 3) / 4, 256, 0, st>>>(gh, R.d_item_desc[1], items[1], k);
+            rc = launch_split(items[0], 16 * kHeavyW / kHeavyM, "msl_server round", [&](int first, int count) {
+                serve_blur_kernel<kHeavyW, kHeavyM><<<count, 16 * kHeavyW / kHeavyM, serve_tile_lds(kHeavyW), st>>>(
+                    gb, R.d_item_desc[0], k, first);
+            });
+        if (!rc && k < nsub_max[1])
+            rc = launch_split((items[1] + 3) / 4, 256, "msl_server round", [&](int first, int count) {
+                serve_heat_kernel<<<count, 256, 0, st>>>(gh, R.d_item_desc[1], items[1], k, first);
+            });
+        if (rc) return rc;
     }
     if (items[3]) {
         serve_expand_kernel<<<(items[3] + 255) / 256, 256, 0, st>>>(gss_start, (int)ds.size(), items[3],
