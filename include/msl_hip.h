@@ -296,8 +296,8 @@ int msl_batch_run_loop(void *batch, int iters, double *d_sums, int *h_result_in_
  * The engine admits queued jobs in arrival order while their HBM bytes fit
  * its budget (one device allocation made at creation) and a slot is free,
  * keeps each job's state resident, and every round advances all active
- * jobs by one step with one persistent launch per job kind (continuous
- * batching).  Final states and sums are bit-identical whether a job runs
+ * jobs by several steps, in launches over the items of all of them
+ * (continuous batching).  Final states and sums are bit-identical whether a job runs
  * alone or in a mix.  Threading: msl_server_submit may be called from any
  * thread; step / drain / poll / run_trace from one thread.              */
 #define MSL_JOB_BLUR2D 1
@@ -331,7 +331,7 @@ int msl_server_create(size_t hbm_budget_bytes, int max_active, void **h_server);
 int msl_server_destroy(void *server);
 /* t_arrival < 0: now.  MSL_E_NOMEM if the job can never fit the budget. */
 int msl_server_submit(void *server, const msl_job *job, double t_arrival, int64_t *h_id);
-/* One round (admit, advance every active job one step, retire finished
+/* One round (admit, advance every active job some steps, retire finished
  * rounds); *h_active / *h_pending after the round.                     */
 int msl_server_step(void *server, int *h_active, int *h_pending);
 /* Rounds until nothing is pending, active or in flight.                */
@@ -342,6 +342,9 @@ int msl_server_drain(void *server);
 int msl_server_poll(void *server, int64_t id, msl_job_result *h_result, void *h_final, size_t final_bytes);
 int msl_server_info(const void *server, int64_t *h_rounds, size_t *h_peak_bytes, double *h_mean_active,
                     int64_t *h_done_jobs);
+/* Rounds so far that ran blur jobs in the tiles for load and in those for
+ * light load (fewer tiles than two per CU).                             */
+int msl_server_blur_rounds(const void *server, int64_t *h_loaded, int64_t *h_light);
 /* Replays an arrival trace in real time (arrival_s ascending, seconds from
  * the call) on an idle server and returns every job's result.         */
 int msl_server_run_trace(void *server, const msl_job *jobs, const double *arrival_s, int njobs,

@@ -402,6 +402,7 @@ struct Server {
     int64_t round_no = 0;
     int64_t done_rounds = 0;
     size_t peak_bytes = 0;
+    int64_t blur_rounds[2] = {0, 0};  // rounds with blur jobs in W = 128 tiles (load), in W = 64 ones (light)
     double active_sum = 0.0;  // sum over rounds of active jobs (for the mean)
     int64_t done_jobs = 0;
 };
@@ -806,6 +807,7 @@ static int run_round(Server &S, int *did_work) {
     R.finishing = std::move(finishing);
 
     // ---- advance the jobs
+    if (!S.blur.empty()) S.blur_rounds[light ? 1 : 0]++;
     S.active_sum += (double)(S.blur.size() + S.heat.size() + maps.size());
     auto advance = [](std::vector<SJob *> &v) {
         size_t w = 0;
@@ -998,6 +1000,14 @@ int msl_server_info(const void *server, int64_t *h_rounds, size_t *h_peak_bytes,
     if (h_peak_bytes) *h_peak_bytes = S->peak_bytes;
     if (h_mean_active) *h_mean_active = S->round_no ? S->active_sum / (double)S->round_no : 0.0;
     if (h_done_jobs) *h_done_jobs = S->done_jobs;
+    return MSL_OK;
+}
+
+int msl_server_blur_rounds(const void *server, int64_t *h_loaded, int64_t *h_light) {
+    MSL_REQUIRE(server != nullptr, "msl_server_blur_rounds: null server");
+    const Server *S = static_cast<const Server *>(server);
+    if (h_loaded) *h_loaded = S->blur_rounds[0];
+    if (h_light) *h_light = S->blur_rounds[1];
     return MSL_OK;
 }
 

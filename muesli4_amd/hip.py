@@ -136,6 +136,7 @@ SIGNATURES = {
     "msl_server_drain": [p],
     "msl_server_poll": [p, C.c_int64, PRES, p, sz],
     "msl_server_info": [p, PI64, C.POINTER(C.c_size_t), PD, PI64],
+    "msl_server_blur_rounds": [p, PI64, PI64],
     "msl_server_run_trace": [p, PJOB, PD, i32, PRES],
     "msl_serve_plain_loop": [PJOB, PD, i32, sz, PRES],
     "msl_timer_start": [],

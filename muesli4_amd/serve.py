@@ -123,6 +123,12 @@ class Server:
         return {"rounds": rounds.value, "peak_bytes": peak.value, "mean_active_jobs": round(mean_active.value, 2),
                 "done_jobs": done.value}
 
+    def blur_rounds(self) -> dict:
+        """Rounds that ran blur jobs in the tiles for load and for light load."""
+        loaded, light = C.c_int64(), C.c_int64()
+        call("msl_server_blur_rounds", self.handle, C.byref(loaded), C.byref(light))
+        return {"loaded": loaded.value, "light": light.value}
+
     def run_trace(self, jobs: List[dict], arrivals) -> List[dict]:
         n = len(jobs)
         arr = (Job * max(n, 1))(*[make_job(d) for d in jobs])
