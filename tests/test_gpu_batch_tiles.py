@@ -104,3 +104,47 @@ def test_narrow_grids_run_in_tiles_whatever_their_strips(tmp_path):
     b.close()
     for x, got, r in zip(grids, states, radii):
         np.testing.assert_array_equal(got, _oracle(x, r, 0.5, iters), err_msg=f"r={r}")
+
+
+@pytest.mark.parametrize("iters", [8, 11, 12])
+def test_tiles_of_every_generation_count(iters):
+    """Rounds of six generations at r = 1 (12 steps), four at r = 2 and 3 (8),
+    three at r = 4 and 5, two above; widths at the edges of both tile widths."""
+    print(f"[case] batch tiles x{iters}", flush=True)
+    hip.init(0)
+    widths = [1, 3, 5, 28, 29, 52, 53, 96, 97, 116, 117, 191]
+    shapes = [(40 + 13 * (k % 5), w) for k, w in enumerate(widths)]
+    for r in range(1, 9):
+        grids = _uniform(shapes, seed=10 * r)
+        b = Grids(grids, [r] * len(shapes), 2.5)
+        states, sums = b.run(iters)
+        b.close()
+        for x, got, s in zip(grids, states, sums):
+            want = _oracle(x, r, 2.5, iters)
+            np.testing.assert_array_equal(got.view(np.uint32), want.view(np.uint32), err_msg=f"r={r} {x.shape}")
+            ref = want.astype(np.float64)
+            assert abs(s - np.sum(ref)) <= FOLD_TOL * np.sum(np.abs(ref)), (r, x.shape)
+
+
+@pytest.mark.parametrize("nv", [0.0, -0.0, np.inf, np.nan])
+def test_tiles_with_special_values(nv):
+    print(f"[case] batch tiles, special values, nv={nv}", flush=True)
+    hip.init(0)
+    rng = np.random.default_rng(3)
+    grids, radii = [], []
+    for r in range(1, 9):
+        for v in (np.inf, -np.inf, np.nan, np.finfo(np.float32).max, 2.0**-149):
+            x = rng.uniform(-1.0, 1.0, (60, 70)).astype(np.float32)
+            x[rng.integers(0, 60, 4), rng.integers(0, 70, 4)] = v
+            grids.append(x)
+            radii.append(r)
+        grids.append(np.full((60, 70), -0.0, np.float32))
+        radii.append(r)
+    b = Grids(grids, radii, nv)
+    states, _ = b.run(4)
+    b.close()
+    for x, got, r in zip(grids, states, radii):
+        want = _oracle(x, r, nv, 4)
+        np.testing.assert_array_equal(got, want, err_msg=f"r={r}")
+        keep = ~np.isnan(want)
+        np.testing.assert_array_equal(got.view(np.uint32)[keep], want.view(np.uint32)[keep], err_msg=f"r={r}")
