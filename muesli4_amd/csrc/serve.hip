@@ -682,7 +682,7 @@ static int run_round(Server &S, int *did_work) {
         heat_us += (double)J->spec.d0 * J->spec.d1 * J->spec.d2 * 8.0 / 3.5e6;
     // at least 8 us per launch of either kind
     const double sub_us = (S.blur.empty() ? 0.0 : std::max(8.0, blur_us)) + (S.heat.empty() ? 0.0 : std::max(8.0, heat_us));
-    const int nsub = std::max(1, std::min(kMaxSub, (int)(kRoundUs / sub_us)));
+    const int nsub = sub_us > 0.0 ? std::max(1, std::min(kMaxSub, (int)(kRoundUs / sub_us))) : 1;
     // the fold of a finishing stencil job: its final state in kSumChunk chunks
     auto add_sum = [&](SJob *J, const float *data, long long n, int slot) {
         const int nchunks = (int)((n + kSumChunk - 1) / kSumChunk);
