@@ -41,8 +41,9 @@ constexpr int strip_max_waves_per_eu() { return (C == 4 && R >= 9 && R <= 10) ? 
 // checked period (8192^2: 4.39 -> 4.69 TB/s against whole periods of 64-row
 // segments); every other radius keeps whole periods (r = 9 at 128 rows
 // marches 146 of 147 rows anyway and lost 2 % to the checked copy).
+constexpr bool strip_checked_tail(int r, int c) { return c == 4 && r == 10; }
 template <int R, int C>
-constexpr int strip_tail_mode() { return (C == 4 && R == 10) ? 2 : 0; }
+constexpr int strip_tail_mode() { return strip_checked_tail(R, C) ? 2 : 0; }
 
 template <typename Pol, int MODE, bool NT = true, int C = 4>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, strip_max_waves_per_eu<Pol::R, C>())))
@@ -108,18 +109,20 @@ inline int row_mode(const T *in, const T *out, int cols) {
 // one per CU, else 8-wave tiles of 64 rows once those give two per CU and of 32
 // below; 128-column tiles, which read the fewest LDS cells per output, above
 // kTile1WideCells and at radii above 10 (whose 64-column tiles hold few
-// outputs) from four tiles per CU.  us per step, strip march / tile: 300 x
-// 1000 r = 2 4.1 / 3.6, 4 5.1 / 3.7; 1201 x 1999 r = 2 8.1 / 5.8, 4 9.2 / 6.4;
-// 2048^2 r = 2 7.5 / 7.8, 4 9.1 / 8.8, 10 17.7 / 11.7, 13 - / 14.6; 3000^2
-// r = 5 18.2 / 15.4, 7 22.0 / 16.7, 10 21.8 / 21.0, 13 30.7 / 24.0; 4096^2
-// r = 2 23.4 / 23.5, 5 27.8 / 25.4, 8 29.1 / 28.6, 10 30.7 / 30.9, 13 49.5 / 38.4;
-// 5000 x 5001 r = 5 42.9 / 33.3, 10 48.1 / 44.8, 16 81.0 / 68.6; 5792^2 r = 5
-// 47.0 / 42.4, 8 49.4 / 49.9, 10 52.3 / 58.8, 16 77.5 / 87.8.
-// Radius 10 on aligned rows marches above 10.5 million cells (one-call us from
-// memory, march / tile: 3000^2 21.3 / 18.6, 3400 x 3600 26.0 / 27.0; unaligned
-// rows 4095^2 42.5 / 35.8), and so do radii 5 and 6 at row strides of 4 KB
-// multiples, where the tiles' loads meet in few memory channels (r = 5,
-// 4096 x 4100 32.9 / 30.8, 4096^2 32.0 / 33.5).
+// outputs) from four tiles per CU.  us per step, march / tile, on the same
+// buffers: 300 x 1000 r = 2 4.1 / 3.6, 4 5.1 / 3.7; 1201 x 1999 r = 2 8.1 / 5.8, 4 9.2
+// / 6.4; 2048^2 r = 2 7.5 / 7.8, 4 9.1 / 8.8, 5 11.6 / 9.3, 10 17.4 / 11.3, 16 34.1 / 15.3;
+// 3000^2 r = 5 16.5 / 14.2, 9 19.6 / 17.8, 10 20.1 / 18.8, 11 24.4 / 20.0; 4000^2 r = 5
+// 24.6 / 21.8, 8 26.5 / 24.2, 9 30.1 / 27.5, 11 37.6 / 31.0; 4096^2 r = 2 23.4 / 23.5;
+// 5000^2 r = 5 33.5 / 31.8, 8 36.7 / 34.9, 9 41.4 / 40.4, 11 52.7 / 47.1; 5001^2 r = 5
+// 39.2 / 31.8, 10 44.2 / 42.7; 5792^2 r = 5 47.0 / 42.4, 8 49.4 / 49.9, 16 77.5 / 87.8.
+// On buffers that come from memory both take 4-8 us more.  Rows of 1024 to 6144
+// columns in steps of 1024 do not differ from others (25 million cells r = 5 33.8
+// / 31.7, at 4096 columns 34.1 / 34.4).  The radius whose march ends with a checked
+// period (strip_checked_tail: a quarter faster than its neighbour's at most
+// heights) marches on aligned rows from 13.6 million cells: r = 10 3400 x 3600 22.5 /
+// 23.1, 4000^2 26.9 / 29.1, 5000^2 37.4 / 42.5, from memory 29.0 / 27.4, 33.4 / 34.0,
+// 47.7 / 50.1 (r = 9 33.9 / 26.6, 37.1 / 32.9, 52.2 / 48.8).
 constexpr long kTile1WideCells = 9L << 19;
 
 // Whether the environment sets the shape of the march (strip_shape): the mean
@@ -156,8 +159,8 @@ static bool thin_iterate(int rows, int cols, int r) {
 
 static bool tile1_default(const float *in, const float *out, int r, int rows, int cols) {
     if (r < 2 || march_forced() || thin_step(rows, cols, r)) return false;
-    const bool march = (r == 10 && row_mode(in, out, cols) == kAligned) || (r <= 6 && cols % 1024 == 0);
-    return (long)rows * cols <= (r <= 4 ? 3L << 20 : march ? 10L << 20 : 25L << 20);
+    const bool tail = strip_checked_tail(r, 4) && row_mode(in, out, cols) == kAligned;
+    return (long)rows * cols <= (r <= 4 ? 3L << 20 : tail ? 13L << 20 : 25L << 20);
 }
 
 static TileShape tile1_shape(int rows, int cols, int r) {
