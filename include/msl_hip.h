@@ -15,8 +15,11 @@
  *  - Pointers named d_* are device pointers (from msl_malloc or any HIP
  *    allocation on the current device); h_* are host pointers.
  *  - All launches are stream-ordered on the library stream (msl_stream()).
- *    Entry points that return a value to the host wait until it is there
- *    (all earlier work of that stream is done by then).
+ *    Entry points that return a value to the host wait until it is there:
+ *    all earlier work of that stream has run by then.  Folds to the host do
+ *    not synchronise the stream, so what earlier kernels wrote to host memory
+ *    that is not coherent (hipHostMallocNonCoherent) is certain to be seen
+ *    only after msl_synchronize.
  *  - x = column, y = row, z = depth.  DM layout row*cols+col, DC layout
  *    (z*rows+y)*cols+x (reference include/nplmatrix.h:141-143,
  *    include/plcube.h:121-123).
@@ -136,8 +139,9 @@ int msl_stencil2d_mean_f32(float *d_out, const float *d_in, int rows, int cols, 
 /* iters ping-pong steps between d_a and d_b starting from d_a, captured
  * once into a HIP graph and replayed.  *h_result_in_b = 1 when the final
  * grid is in d_b (odd iters).  Launches may apply several generations
- * (r = 1: up to six; r = 2..7 on large grids with rows of 4 or more
- * cells: two; r >= 2 on smaller grids: up to six in LDS tiles) with results
+ * (r = 1: up to six; r >= 2 up to six in LDS tiles, at r >= 4 on smaller
+ * grids; r <= 7 on larger or thin grids with rows of 4 or more cells: two)
+ * with results
  * bit-identical to one launch per generation; d_b then holds intermediate
  * generations other than those of the one-per-launch schedule.            */
 int msl_stencil2d_mean_iterate_f32(float *d_a, float *d_b, int rows, int cols, int r, float nv, int iters,
@@ -228,8 +232,9 @@ int msl_selftest_launch_split(int64_t blocks, int threads, int *h_launches, int6
  * over an atomic work queue of (grid, strip, segment) items; grids of
  * radius <= 8 with 256-column strips advance two generations per item
  * (pairs of steps, one pair split when the number of rounds would not
- * have the parity of iters), narrow grids of those radii up to six per
- * round in LDS tiles, the others one.  The rounds and the per-grid
+ * have the parity of iters), narrow grids of those radii (fewer than 192
+ * columns, or in 64-column strips) up to six per round in LDS tiles, the
+ * others one.  The rounds and the per-grid
  * fold are captured once into a HIP graph (per iteration count and
  * d_sums) and replayed.  d_sums (nullable; ngrids doubles) receives the
  * compensated fold(sum) of each grid's final state (iters >= 1); the

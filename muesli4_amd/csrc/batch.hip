@@ -226,11 +226,10 @@ __global__ __launch_bounds__(256) void batch_round_kernel(const BGrid *__restric
 }
 
 // Tiles of narrow grids.  128-column tiles (64-column ones where they cover
-// the grid with fewer lanes), as many generations per round as leave about
-// half of a tile.  10 steps of the 2621 grids narrower than 192 columns in the
-// 4096-grid batch: 0.82 ms, 2.0 in one-generation strips.  (Wide grids in tiles
-// take 470 us per generation, in two-generation strips 435.)
-constexpr int kTileGens[kBatchPairMaxR + 1] = {0, 6, 4, 4, 3, 3, 2, 2, 2};
+// the grid with fewer lanes) of kTileGens generations per round.  10 steps of
+// the 2621 grids narrower than 192 columns in the 4096-grid batch: 0.82 ms, 2.0 in
+// one-generation strips.  (Wide grids in tiles take 470 us per generation, in
+// two-generation strips 435.)
 constexpr int kTileThreads = 512;    // W = 128, M = 4 or W = 64, M = 2
 constexpr size_t kTileLds = blur_tile_lds(kBatchPairMaxR, 128, kTileRows, 1);
 
@@ -693,10 +692,10 @@ static std::vector<int> pair_plan(int iters) {
 // parity of iters.
 static std::vector<int> tile_plan(int iters, int most) {
     std::vector<int> plan;
-    int rounds = (iters + most - 1) / most;
+    int rounds = iters > 0 ? (iters - 1) / most + 1 : 0;
     if ((rounds ^ iters) & 1) rounds++;
     for (; rounds > 0; rounds--) {
-        plan.push_back((iters + rounds - 1) / rounds);
+        plan.push_back((iters - 1) / rounds + 1);
         iters -= plan.back();
     }
     return plan;

@@ -17,12 +17,19 @@ namespace mslhip {
 
 constexpr int kTileRows = 64;  // most output rows of a tile's first generation
 
+// Generations per launch, by radius, of the batch's and the serving engine's
+// 128-column tiles.  Measured at r = 3, 5, 7 and 10 (us per generation of 2048^2 at
+// 1 / 2 / 3 / 4 generations, M = 4: 10.6 / 7.3 / 6.8 / 6.1, 11.1 / 9.1 / 8.4 / 8.5,
+// 12.0 / 10.4 / 11.0, 13.6 / 13.4 / 19.6); the radii between take the count of the
+// next larger one that was measured, r = 1 the most there are.
+constexpr int kTileGens[11] = {0, 6, 4, 4, 3, 3, 2, 2, 2, 2, 2};
+
 // Row pass: a row's quads sit in one wave (16 or 32 lanes), whose lanes all
 // read their windows before any of them stores, so the sums replace the row.
 // Reads past the valid columns feed only sums that no output uses.
-// Read: M rows per thread of the column pass, 64 / M rows per round of all
-// threads.  1 on grids of few tiles (16 waves per tile, the shortest chain),
-// 4 on many (fewest LDS reads per output).
+// M is the rows per thread of the column pass (all threads cover 64 / M rows at a
+// time): 1 on grids of few tiles (16 waves per tile, the shortest chain), 4 on
+// many (fewest LDS reads per output).
 template <int R, int W, int M>
 __device__ __forceinline__ void blur_tile(float *__restrict__ out, const float *__restrict__ in, int rows, int cols,
                                           float nv, int steps, int tile_w, int tile_h, int tx, int ty, float *lds) {

@@ -148,10 +148,11 @@ __device__ __forceinline__ void heat7_march(float *__restrict__ out, const float
 // full form (on thin cubes, which wait for memory, 5-10 % faster than the
 // short form and its check).
 constexpr int kT2X = kTX - 4;  // output columns of a two-generation wave tile
-// Output rows of a two-generation wave tile: 5 rows (90 VGPRs, five waves
+// Output rows of a two-generation wave tile: 5 rows (86-94 VGPRs, five waves
 // per SIMD) beat 8 (124, four) although the y halo grows from 4/8 to 4/5
-// (200 iterations of a 320^3 cube alone: 8 rows 7.13 ms, 5 6.90).  The serving
-// engine's items use it, and large thin cubes (heat_way); other cubes run
+// (200 iterations of a 320^3 cube alone: 8 rows 7.13 ms, 5 6.90).  Large thin
+// cubes (heat_way) and the serving engine's items use it; the latter's kernel
+// holds both forms of kSingle and takes 134 VGPRs, three waves.  Other cubes run
 // heat_tile.hip and heat_pair.hip.
 constexpr int kT2Y = 5;
 

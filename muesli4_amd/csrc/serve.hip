@@ -111,13 +111,9 @@ __global__ void serve_expand_kernel(const int *__restrict__ starts, int ndesc, i
     item_desc[i] = lo;
 }
 
-// Most generations of a blur job per launch: as many as the LDS tile still
-// leaves at least half of its columns and rows (W = 128: the fewest row
-// overlaps per output; W = 64, at light load, where launches count).
-// us per generation of 2048^2 at 1 / 2 / 3 / 4 generations and W = 128, M = 4:
-// r = 3 10.6 / 7.3 / 6.8 / 6.1, r = 5 11.1 / 9.1 / 8.4 / 8.5, r = 7 12.0 /
-// 10.4 / 11.0, r = 10 13.6 / 13.4 / 19.6.
-constexpr int kHeavyGens[kBatchMaxR + 1] = {0, 6, 4, 4, 3, 3, 2, 2, 2, 2, 2};
+// Most generations of a blur job per launch: under load kTileGens in W = 128
+// tiles (the fewest row overlaps per output), at light load, where launches
+// count, up to two more in W = 64 ones.
 constexpr int kLightGens[kBatchMaxR + 1] = {0, 6, 6, 6, 4, 4, 3, 3, 2, 2, 2};
 constexpr int kHeavyW = 128, kHeavyM = 4;
 constexpr int kLightW = 64, kLightM = 1;
@@ -445,7 +441,7 @@ static int validate_job(const msl_job &j, size_t budget) {
 static void tile_blur(SJob &J, bool light) {
     const msl_job &s = J.spec;
     const int w = light ? kLightW : kHeavyW;
-    J.gens = std::min(light ? kLightGens[s.r] : kHeavyGens[s.r], s.steps);
+    J.gens = std::min(light ? kLightGens[s.r] : kTileGens[s.r], s.steps);
     J.tile_w = (w - 2 * s.r * J.gens) / 4 * 4;
     J.tiles_x = (s.d1 + J.tile_w - 1) / J.tile_w;
     J.tile_h = std::min((kTileRows - 2 * s.r * (J.gens - 1)) / 8 * 8, 48);

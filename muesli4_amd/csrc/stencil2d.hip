@@ -352,10 +352,10 @@ std::vector<int> generation_plan(int iters, int k) {
 // most k each allow (LDS tiles: a launch's cost grows with its generations).
 static std::vector<int> even_plan(int iters, int k) {
     std::vector<int> plan;
-    int launches = (iters + k - 1) / k;
+    int launches = iters > 0 ? (iters - 1) / k + 1 : 0;
     if ((launches ^ iters) & 1) launches++;
     for (; launches > 0; launches--) {
-        plan.push_back((iters + launches - 1) / launches);
+        plan.push_back((iters - 1) / launches + 1);
         iters -= plan.back();
     }
     return plan;
