@@ -33,7 +33,7 @@ __device__ __forceinline__ float lane_from_right(float v) {  // lane l gets lane
 // before.  8 rows per wave keep 62 VGPRs, eight waves per SIMD (16 rows: 104).
 // 8192^2 x 20: 653 -> 533 us (500 with every XCD on a contiguous range; 527 with
 // cells of either sign, whose windows divide in four operations), of which 4
-// passes over HBM take 420 at the rate of a copy and the VALU issue 381; with the
+// passes over HBM take 370 at the rate of the map and the VALU issue 373; with the
 // next window's cells loaded ahead by persistent blocks 685 (99 VGPRs).  Windows
 // over the grid's edge keep the cells outside at nv by bits and leave out waves
 // without rows in it (20 iterations, with a select per cell, which became a
